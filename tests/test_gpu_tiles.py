@@ -10,7 +10,7 @@ import aristos_amd as ka
 from aristos_amd import synth
 from helpers import pack_inputs, random_layer
 from oracle import moe_ref
-from test_gpu_parity import MODE_IDS, MODES, _keys, _one_hot_layer, _out_to_np, _to_device, check_against_oracle
+from test_gpu_parity import MODE_IDS, MODES, _apply, _keys, _one_hot_layer, _out_to_np, _to_device, check_against_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -191,3 +191,34 @@ def test_32_bit_tiles_of_few_rows(mode, dt, H, I, act):
 def test_down_projection_on_the_smaller_tile(mode, dt, H, I, rows, cf):
     """Wide up-projections whose long, few down-projection tiles leave CUs idle."""
     _forced_rows(dt, H, I, rows, cf=cf, mode=mode)
+
+
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("dt,S,H,I", [(2, 2304, 320, 448), (3, 1152, 1088, 192), (0, 640, 128, 320)])
+def test_dense_output_over_its_inputs(mode, dt, S, H, I):
+    """The dense packing with its output laid over other rows of x, over weights and biases, up to the last element of
+    the inputs: every input is read before the output overwrites it, so the bits are those of an output
+    of its own. (The output in place of x row for row: above.)"""
+    keys = _keys(S, H, I, 1, 1, act=1, dt=dt)
+    c = moe_ref.cfg_from_keys(keys)
+    x, wg, w_up, w_down, b_up, b_down = random_layer(c, seed=S + I, w_std=0.08, bias_std=0.1)
+    iP = pack_inputs(c, x, wg, w_up, w_down, b_up, b_down)
+    dense = np.concatenate([iP[:S * H], iP[S * H + c.PX * H:]])
+    per16 = 16 // dense.itemsize
+    last = dense.size - S * H
+    offsets = [per16, H, last // 2 // per16 * per16, last // per16 * per16]   # 16-byte aligned, as outputs have to be
+    ka.initialize(keys)
+    try:
+        _apply(mode)
+        own = torch.empty(S * H, dtype=_to_device(c, dense[:1]).dtype, device="cuda")
+        ka.moe.forward_host_dense(_to_device(c, dense), own)
+        ka.moe.stream_synchronize()
+        want = _out_to_np(c, own)
+        for at in offsets:
+            buf = _to_device(c, dense)
+            torch.cuda.synchronize()
+            ka.moe.forward_host_dense(buf, buf[at:at + S * H])
+            ka.moe.stream_synchronize()
+            np.testing.assert_array_equal(_out_to_np(c, buf)[at:at + S * H], want, err_msg=f"output at element {at}")
+    finally:
+        ka.finalize()
