@@ -20,7 +20,8 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wextra", "-Wno-unused-parameter", "-Wno-pass-failed",
 ]
-SOURCES = ["config.cpp", "capi.hip", "kernels.hip", "kernels_f32.hip", "kernels_tf32.hip", "kernels_bf16.hip", "kernels_f16.hip"]
+SOURCES = ["config.cpp", "capi.hip", "kernels.hip", "kernels_f32.hip", "kernels_tf32.hip", "kernels_bf16.hip", "kernels_bf16_64.hip", "kernels_bf16_512.hip",
+           "kernels_f16.hip", "kernels_f16_64.hip", "kernels_f16_512.hip"]
 
 
 def _hipcc() -> str:
@@ -40,7 +41,7 @@ def _run(cmd: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
-def build_library(driver: bool = True, jobs: int = 6) -> str:
+def build_library(driver: bool = True, jobs: int = 8) -> str:
     """Compiles every HIP source into libkleos_amd.so (and the C++ driver); returns the library path.
     The sources are compiled side by side (one hipcc process each, objects under aristos_amd/build/),
     then linked."""
