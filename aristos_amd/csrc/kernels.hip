@@ -22,6 +22,13 @@ __global__ __launch_bounds__(kPhaseThreads) void slot_kernel(const LayerParams p
     for (uint32_t i = blockIdx.x * kPhaseThreads + threadIdx.x; i < p.n_super * p.E; i += gridDim.x * kPhaseThreads)
         other[i] = 0u;
 }
+
+__global__ __launch_bounds__(kPhaseThreads) void dense_rows_kernel(const LayerParams p) {
+    const uint32_t first = blockIdx.x * kPhaseThreads + threadIdx.x, stride = gridDim.x * kPhaseThreads;
+    dense_rows(p, first, stride);
+    uint32_t* other = p.super_count + size_t((p.epoch & 1u) ^ 1u) * p.n_super;
+    for (uint32_t i = first; i < p.n_super; i += stride) other[i] = 0u;
+}
 }  // namespace
 
 const char* unsupported_reason(uint32_t E, uint32_t k) {
@@ -162,6 +169,11 @@ hipError_t launch_gate(const LayerParams& p, int dtype, int num_cus, hipStream_t
 hipError_t launch_slots(const LayerParams& p, hipStream_t s) {
     const uint32_t grid = ceil_div_u32(p.n_gate_tiles, 4);
     hipLaunchKernelGGL(slot_kernel, dim3(grid), dim3(kPhaseThreads), 4 * p.E * sizeof(uint32_t), s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_dense_rows(const LayerParams& p, hipStream_t s) {
+    hipLaunchKernelGGL(dense_rows_kernel, dim3(ceil_div_u32(p.S, kPhaseThreads)), dim3(kPhaseThreads), 0, s, p);
     return hipGetLastError();
 }
 

@@ -21,6 +21,8 @@ hipError_t launch_gate(const LayerParams& p, int dtype, int num_cus, hipStream_t
 // splits * S * PX floats.
 uint32_t gate_splits_for(uint32_t S, uint32_t H, uint32_t E, uint32_t PX, int dtype, int num_cus);
 hipError_t launch_slots(const LayerParams& p, hipStream_t s);
+// In place of gate and slots where LayerParams::dense is set.
+hipError_t launch_dense_rows(const LayerParams& p, hipStream_t s);
 hipError_t launch_expert_gemm(const LayerParams& p, int dtype, int kind /*0 up, 1 down*/, int num_cus, hipStream_t s);
 hipError_t launch_combine(const LayerParams& p, int dtype, hipStream_t s);
 

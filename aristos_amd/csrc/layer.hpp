@@ -9,7 +9,8 @@ constexpr int kGateTileTokens = 16;   // tokens per gate tile (one MFMA column b
 constexpr int kSuperTiles = 32;       // gate tiles per coarse count row (512 tokens)
 constexpr int kMaxGateGroups = 16;    // 16 experts per group: up to 256 experts keep their logits in registers
 
-// LayerParams::dense: routed as any layer | rows are tokens, results through y and the combine | results stored by the down-projection
+// LayerParams::dense: routed as any layer | rows are tokens, results through y and the combine | results stored by the
+// down-projection (persistent kernel only)
 constexpr uint32_t kDenseNo = 0, kDenseRows = 1, kDenseDirect = 2;
 
 struct LayerParams {
@@ -20,7 +21,7 @@ struct LayerParams {
     uint32_t n_super;         // ceil(n_gate_tiles / 32)
     uint32_t tile_variant;    // tile of the expert projections (choose_tiles)
     uint32_t down_small;      // 1: the down-projection on the smaller tile of the variant (NarrowCfg)
-    uint32_t dense;           // one expert that keeps every token, no gate output: rows are tokens (persistent kernel only); a kDense value
+    uint32_t dense;           // one expert that keeps every token, no gate output: rows are tokens; a kDense value
     // ---- caller buffers, sliced as moe.cuh:92-98
     const void* x;            // [S, H]
     const void* wg;           // [PX, H]

@@ -139,9 +139,13 @@ int kleos_moe_forward(const void* iP, void* oP);
  * iP: x[S,H] | Wup[I,H] | Wdown[H,I] | bup[I] | bdown[H]   (A | B1 | B2 | D1 | D2; no gate weights)
  * oP: moeOut[S,H]                                          (C; no gate output)
  * D2 follows the I entries of D1 (the reference steps over H entries there, fffn.cuh:49, which is the
- * same place whenever I == H). The gate still runs, on zero gate weights and into a gate output that
- * the library owns; moeOut has the bits kleos_moe_forward gives for the same operands. Asynchronous on
- * the library stream. KLEOS_ESTATE when the context holds more than one expert.
+ * same place whenever I == H). Every token is a row of the one expert, as in fffn: no gate, whatever
+ * the token holds. moeOut has the bits kleos_moe_forward gives for the same operands; they differ for
+ * a token with an infinity or a NaN, which kleos_moe_forward routes nowhere (a zero row) and which
+ * goes through both products here. (With is_training 1 the gate runs, on zero gate weights and into a
+ * gate output that the library owns, for the sake of its loss, and such a token gets a zero row here
+ * too.) oP may overlap iP. Asynchronous on the library stream. KLEOS_ESTATE when the context holds
+ * more than one expert.
  */
 int kleos_moe_forward_dense(const void* iP, void* oP);
 /*

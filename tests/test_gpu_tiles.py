@@ -222,3 +222,41 @@ def test_dense_output_over_its_inputs(mode, dt, S, H, I):
             np.testing.assert_array_equal(_out_to_np(c, buf)[at:at + S * H], want, err_msg=f"output at element {at}")
     finally:
         ka.finalize()
+
+
+@pytest.mark.parametrize("dt", [0, 2], ids=["fp32", "bf16"])
+def test_dense_tokens_with_infinities_and_nan(dt):
+    """Nothing is routed in the dense packing, in either mode: a token that holds an infinity or a NaN goes through both
+    products like any other, and the other tokens keep their bits."""
+    S, H, I = 640, 128, 192
+    keys = _keys(S, H, I, 1, 1, act=0, dt=dt)
+    tdt = {0: torch.float32, 2: torch.bfloat16}[dt]
+    rng = np.random.default_rng(11)
+    x, w_up, w_down = (torch.from_numpy(rng.standard_normal(n)).to(tdt) for n in ((S, H), (I, H), (H, I)))
+    finite = x.clone()
+    x[7, 3], x[300, 100], x[639, 0], x[64, 64] = float("inf"), -float("inf"), float("inf"), float("nan")
+    special = [7, 64, 300, 639]
+    h = x.double() @ w_up.double().T
+    h = torch.where(h > 0, h, torch.zeros((), dtype=h.dtype))   # NaN gives 0, as in the kernels
+    want = h @ w_down.double().T
+    got = {}
+    ka.initialize(keys)
+    try:
+        for name, values in (("finite", finite), ("special", x)):
+            for mode, label in zip(MODES, MODE_IDS):
+                _apply(mode)
+                iP = torch.cat([values.flatten(), w_up.flatten(), w_down.flatten(), torch.zeros(H + I, dtype=tdt)]).cuda()
+                oP = torch.empty(S * H, dtype=tdt, device="cuda")
+                torch.cuda.synchronize()
+                ka.moe.forward_host_dense(iP, oP)
+                ka.moe.stream_synchronize()
+                got[name, label] = oP.view(S, H).cpu()
+    finally:
+        ka.finalize()
+    others = torch.ones(S, dtype=torch.bool)
+    others[special] = False
+    for label in MODE_IDS:
+        out = got["special", label].double()
+        for places in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(places(out), places(want)), label
+        assert torch.equal(got["special", label][others], got["finite", label][others]), label
