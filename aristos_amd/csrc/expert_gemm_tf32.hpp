@@ -3,11 +3,13 @@
 // A tf32 operand has 11 significant bits. Its upper 8 are a bf16 value (the upper half of the word) and
 // the remainder, at most 3 bits, is exactly one too: v = hi + lo. A product of two operands is then the sum
 // of four bf16 products, each exact in fp32 as the tf32 product itself is, and all four are added: nothing
-// is dropped, the sums are fp32 sums of exact products as on the fp32 matrix instructions. (An operand
-// below 2^-118 may lose bits of its remainder to underflow. An infinite operand times a remainder of zero is
-// NaN where the fp32 instructions give infinity: a wavefront that finds a NaN among its sums computes its
-// part of the tile again on those.) The bf16
+// is dropped, the sums are fp32 sums of exact products as on the fp32 matrix instructions. The bf16
 // instructions have sixteen times the fp32 rate, so four products per pair of operands leave a factor of four.
+// Two kinds of operands do not split: an infinity, whose product with a remainder of zero is NaN, and a value below
+// 2^-123, whose remainder has bits below the last of a bf16 subnormal (2^-133). A wavefront that finds a NaN among its
+// sums, or sums so small that such lost bits could show in them, computes its part of the tile again on the fp32
+// matrix instructions. (Noticing the lost bits takes 18 of a slice's 373 vector instructions: 936 -> 944 us at the
+// layer below.)
 #pragma once
 #include "expert_gemm.hpp"
 
@@ -53,7 +55,8 @@ struct GemmSplit {
     static constexpr int kRowBytes = kSliceK * 4, kRowsPerLoad = 8, kChunks = 8;
     static constexpr int kABytes = BM * kRowBytes, kBBytes = BN * kRowBytes, kStage = kABytes + kBBytes;
     static constexpr int kBiasBytes = BN * 4, kBiasOffset = 2 * kStage;
-    static constexpr int kSmemBytes = 2 * kStage + 2 * kBiasBytes;
+    static constexpr int kLostOffset = kBiasOffset + 2 * kBiasBytes;   // a word per bias slot: whether an operand of the tile lost bits
+    static constexpr int kSmemBytes = kLostOffset + 16;
     static constexpr int LA = BM / (kRowsPerLoad * kWaves), LB = BN / (kRowsPerLoad * kWaves);
     static_assert(TM == 8 && TN == 4 && LA == 4 && LB == 4, "the groups below are counted for these");
     static_assert(kWaves * 4096 <= kStage && kBiasBytes <= 1024);
@@ -99,6 +102,8 @@ struct GemmSplit {
             const uint32_t n = uint32_t(lane) * 4 < g.n_valid ? uint32_t(lane) * 4 : 0u;
             direct_load16<false>(g.bias + n, lds_address(smem) + kBiasOffset + bias_slot * kBiasBytes);
         }
+        // (last read by the epilogue of the tile before the previous one, written again behind the main loop's barriers)
+        if (tid == 0) *lost_word(smem, bias_slot) = 0u;
         t.a_base = g.a_base; t.a_row_index = g.a_row_index; t.a_rows = g.a_rows; t.lda = g.lda;
         t.b_base = g.b_base; t.ldb = g.ldb;
         t.c_base = g.c_base; t.ldc = g.ldc;
@@ -145,7 +150,12 @@ struct GemmSplit {
         const int hi_chunk = (c & 4) + ((c & 3) >> 1);
         return uint32_t(r * kRowBytes + ((hi_chunk ^ sw) << 4) + (c & 1) * 8);
     }
-    static __device__ __forceinline__ void split_store(char* kilobyte, uint32_t split_hi, u32x4 raw) {
+    // `lost`: what the remainders split by this thread had in their lower halves, which bf16 does not hold.
+    static __device__ __forceinline__ uint32_t* lost_word(char* smem, int bias_slot) { return reinterpret_cast<uint32_t*>(smem + kLostOffset) + bias_slot; }
+    static __device__ __forceinline__ void report_lost(const Tile& t, char* smem, uint32_t lost) {
+        if (lost & 0xffffu) *lost_word(smem, t.bias_slot) = 1u;
+    }
+    static __device__ __forceinline__ void split_store(char* kilobyte, uint32_t split_hi, u32x4 raw, uint32_t& lost) {
         u32x2 hi, lo;
         uint32_t rest[4];
 #pragma unroll
@@ -154,6 +164,7 @@ struct GemmSplit {
             const float v = __builtin_bit_cast(float, word & 0xffffe000u), h = __builtin_bit_cast(float, word & 0xffff0000u);
             rest[j] = __builtin_bit_cast(uint32_t, v - h);
         }
+        lost |= rest[0] | rest[1] | rest[2] | rest[3];
         // the upper halves of two words, packed
         hi[0] = __builtin_amdgcn_perm(raw[1], raw[0], 0x07060302u);
         hi[1] = __builtin_amdgcn_perm(raw[3], raw[2], 0x07060302u);
@@ -174,6 +185,7 @@ struct GemmSplit {
         const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
         const int wm = wave / WAVES_N, wn = wave % WAVES_N;
         const uint32_t split_hi = split_offset();
+        uint32_t lost = 0u;
         // every wavefront has left the previous tile's epilogue, staged where slice 1 goes
         asm volatile("s_barrier" ::: "memory");
         if (t.k_tiles > 1) {
@@ -191,7 +203,7 @@ struct GemmSplit {
 #pragma unroll
             for (int i = 0; i < LA + LB; ++i) raw[i] = load16(kilobyte(st, i) + 16 * lane);
 #pragma unroll
-            for (int i = 0; i < LA + LB; ++i) split_store(kilobyte(st, i), split_hi, raw[i]);
+            for (int i = 0; i < LA + LB; ++i) split_store(kilobyte(st, i), split_hi, raw[i], lost);
         }
         // The workgroup meets in front of a slice once this wavefront's split rows are in LDS.
         auto top = [&](uint32_t kt) {
@@ -222,9 +234,10 @@ struct GemmSplit {
                 if (next) {
                     char* st = smem + stage_of(t, kt + 1) * kStage;
 #pragma unroll
-                    for (int i = 0; i < LA + LB; ++i) split_store(kilobyte(st, i), split_hi, load16(kilobyte(st, i) + 16 * lane));
+                    for (int i = 0; i < LA + LB; ++i) split_store(kilobyte(st, i), split_hi, load16(kilobyte(st, i) + 16 * lane), lost);
                 }
             }
+            report_lost(t, smem, lost);
             return;
         }
 #pragma unroll
@@ -291,7 +304,7 @@ struct GemmSplit {
                 if (NEXT && ks == 1) {
                     // kilobyte o of slice kt+1: its values asked for here, split a group later. In flight at o = 0: its
                     // weight rows, then its activation rows; from o = LB on: those, then the weight rows of slice kt+2.
-                    if (o > 0) split_store(kilobyte(st1, o - 1), split_hi, raw);
+                    if (o > 0) split_store(kilobyte(st1, o - 1), split_hi, raw, lost);
                     if (o == 0) wait_vmcnt<LA>();
                     if (o == LB) wait_vmcnt<NEXT2 ? LB : 0>();
                     asm volatile("" ::: "memory");
@@ -300,17 +313,21 @@ struct GemmSplit {
                 if (NEXT2 && ks == 1 && o == 0) asm volatile("s_barrier" ::: "memory");   // the weight rows of this stage are free
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (NEXT) split_store(kilobyte(st1, TM - 1), split_hi, raw);
+            if (NEXT) split_store(kilobyte(st1, TM - 1), split_hi, raw, lost);
         };
         const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;
         for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::true_type{}, std::true_type{});
         if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::true_type{}, std::false_type{});
         slice(t.k_tiles - 1, std::false_type{}, std::false_type{});
+        report_lost(t, smem, lost);
     }
 
     // Bias, activation, rounding to tf32, rows written through the L2 in whole lines: panels of 32 rows x 32
     // columns go through 4 KB of the wavefront's own in the stage of the last slice.
     static __device__ __forceinline__ void finish(const Tile& t, Acc& acc, char* smem) {
+        float largest = 0.f;
+        const bool lost = *lost_word(smem, t.bias_slot) != 0u;   // the same in every wavefront
+        if (lost) largest = largest_operand(t, smem);
         if (rows_absent(t, __builtin_amdgcn_readfirstlane(int(local_tid() >> 6)) / WAVES_N)) return;
         bool nan = false;
 #pragma unroll
@@ -319,14 +336,68 @@ struct GemmSplit {
             for (int mi = 0; mi < TM; ++mi)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) nan |= acc[ni][mi][j] != acc[ni][mi][j];
+        if (lost) nan |= small_sums(t, acc, largest);
         if (__builtin_amdgcn_ballot_w64(nan) != 0u) recompute(t, smem);
         else if (t.act == 0) finish_act<0>(t, acc, smem);
         else if (t.act == 1) finish_act<1>(t, acc, smem);
         else finish_act<2>(t, acc, smem);
     }
-    // This wavefront's part of the tile once more, block by block on the fp32 matrix instructions from the rows in memory:
-    // what infinities and NaN among the operands give is what the 64 x 64 tiles give. Rows and columns past the
-    // last one repeat it and are not written.
+    // The largest operand of the tile, from the rows in memory: every thread looks at what it loaded for the main loop, the
+    // stage that the last slice is not in takes the results. Called by all wavefronts or none.
+    static __device__ __forceinline__ float largest_operand(const Tile& t, char* smem) {
+        float largest = 0.f;
+#pragma unroll 1
+        for (uint32_t k = 0; k < t.k_tiles * kSliceK; k += kSliceK) {
+            // (four loads at a time: the sums of the tile occupy half of the registers)
+            u32x4 v[4];
+            auto look = [&] {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const uint32_t word = v[i][j] & 0x7fffffffu;
+                        largest = __builtin_fmaxf(largest, __builtin_bit_cast(float, word));
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+#pragma unroll
+            for (int i = 0; i < LA; ++i) v[i] = load16(t.pa[i] + k);
+            look();
+#pragma unroll
+            for (int i = 0; i < LB; ++i) v[i] = load16(t.pb[i] + k);
+            look();
+        }
+        float* words = reinterpret_cast<float*>(smem + (last_stage(t) ^ 1) * kStage);
+        words[threadIdx.x] = largest;
+        __syncthreads();
+#pragma unroll 1
+        for (int i = 0; i < kThreads; ++i) largest = __builtin_fmaxf(largest, words[i]);
+        __syncthreads();   // the next tile's first loads go to that stage
+        return largest;
+    }
+    // Whether a sum of this lane is so small that bits lost in the split could show in it. A product loses less than 2^-133
+    // times the largest operand, a sum K times that; what is below the 26th bit of a sum disappears in its fp32 rounding.
+    static __device__ __forceinline__ bool small_sums(const Tile& t, const Acc& acc, float largest) {
+        const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+        const float visible = largest * float(t.k_tiles * kSliceK) * 0x1p-107f;
+        float least = __builtin_huge_valf();   // of the sums of rows that exist
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) {
+            float v = __builtin_huge_valf();
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni) {
+                asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(v) : "v"(acc[ni][mi][0]), "v"(acc[ni][mi][1]));
+                asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(v) : "v"(acc[ni][mi][2]), "v"(acc[ni][mi][3]));
+            }
+            if (uint32_t((wave / WAVES_N) * WM + mi * 16 + (lane & 15)) < t.m_valid) least = __builtin_fminf(least, v);
+        }
+        return !(least > visible);
+    }
+    // This wavefront's part of the tile once more, on the fp32 matrix instructions from the rows in memory: what infinities,
+    // NaN and the smallest operands give is what the 64 x 64 tiles give. Rows and columns past the last one repeat it
+    // and are not written. A row block against all four column blocks, ten loads in flight: bound by their round trips,
+    // about 0.6 ms per projection where it happens (one expert of 2 048 x 2 048, 8 192 tokens, an infinity in one token:
+    // 592 -> 1 784 us per forward; 3 160 a column block at a time; 2 190 with the 64 x 64 tiles throughout).
     static __device__ __forceinline__ void recompute(const Tile& t, const char* smem) {
         const uint32_t tid = local_tid();
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -334,28 +405,48 @@ struct GemmSplit {
         const uint32_t fr_row = lane & 15, fr_part = lane >> 4, K = t.k_tiles * kSliceK;
         const char* bias = smem + kBiasOffset + t.bias_slot * kBiasBytes;
 #pragma unroll 1
-        for (uint32_t block = 0; block < uint32_t(TM * TN); ++block) {
-            const uint32_t m = m0 + (block / TN) * 16 + fr_row, nb = n0 + (block % TN) * 16;
+        for (uint32_t mi = 0; mi < uint32_t(TM); ++mi) {
+            const uint32_t m = m0 + mi * 16 + fr_row;
             uint32_t row = m < t.m_valid ? m : t.m_valid - 1;
             if (t.a_row_index) {
                 row = uint32_t(load_coherent(t.a_row_index + row));
                 row = row < t.a_rows ? row : t.a_rows - 1;
             }
-            const uint32_t w_row = nb + fr_row < t.n_valid ? nb + fr_row : t.n_valid - 1;
             const float* x = t.a_base + size_t(row) * t.lda + 4 * fr_part;
-            const float* w = t.b_base + size_t(w_row) * t.ldb + 4 * fr_part;
-            f32x4 sum{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-            for (uint32_t k = 0; k < K; k += 16) sum = mma16_step(load16(w + k), load16(x + k), sum, tf32_t{});
-            const uint32_t n = nb + 4 * fr_part;
-            const f32x4 b4 = *reinterpret_cast<const f32x4*>(bias + n * 4);
-            f32x4 v;
+            const float* w[TN];
+            f32x4 sum[TN];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float s = sum[j] + b4[j];
-                v[j] = tf32_round(t.act == 0 ? activate<0>(s) : (t.act == 1 ? activate<1>(s) : activate<2>(s)));
+            for (int ni = 0; ni < TN; ++ni) {
+                const uint32_t n = n0 + ni * 16 + fr_row;
+                w[ni] = t.b_base + size_t(n < t.n_valid ? n : t.n_valid - 1) * t.ldb + 4 * fr_part;
+                sum[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
-            if (m < t.m_valid && n < t.n_valid) store16_through(t.c_base + size_t(m) * t.ldc + n, __builtin_bit_cast(u32x4, v));
+#pragma unroll 1
+            for (uint32_t k = 0; k < K; k += kSliceK) {
+                u32x4 xv[2], wv[2][TN];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    xv[h] = load16(x + k + 16 * h);
+#pragma unroll
+                    for (int ni = 0; ni < TN; ++ni) wv[h][ni] = load16(w[ni] + k + 16 * h);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int ni = 0; ni < TN; ++ni) sum[ni] = mma16_step(wv[h][ni], xv[h], sum[ni], tf32_t{});
+            }
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni) {
+                const uint32_t n = n0 + ni * 16 + 4 * fr_part;
+                const f32x4 b4 = *reinterpret_cast<const f32x4*>(bias + n * 4);
+                f32x4 v;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float s = sum[ni][j] + b4[j];
+                    v[j] = tf32_round(t.act == 0 ? activate<0>(s) : (t.act == 1 ? activate<1>(s) : activate<2>(s)));
+                }
+                if (m < t.m_valid && n < t.n_valid) store16_through(t.c_base + size_t(m) * t.ldc + n, __builtin_bit_cast(u32x4, v));
+            }
         }
     }
     template <int ACT>

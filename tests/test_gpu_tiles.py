@@ -260,3 +260,42 @@ def test_dense_tokens_with_infinities_and_nan(dt):
         for places in (torch.isnan, torch.isposinf, torch.isneginf):
             assert torch.equal(places(out), places(want)), label
         assert torch.equal(got["special", label][others], got["finite", label][others]), label
+
+
+@pytest.mark.parametrize("where", ["x", "w_up", "one token"])
+@pytest.mark.parametrize("exponent", [-124, -130, -135])
+def test_tf32_operands_below_what_splits_exactly(where, exponent):
+    """Operands whose remainder has bits below the last of a bf16 subnormal, against partners large enough for those bits
+    to show: the products of the undivided operands, as on the fp32 matrix cores, with and without ordinary tokens beside."""
+    S, H, I = 16384, 512, 512
+    rng = np.random.default_rng(5)
+
+    def values(*n):   # 11 significant bits, 1 <= |v| < 2
+        return torch.from_numpy(rng.integers(1024, 2048, n) * rng.choice([-1.0, 1.0], n) / 1024)
+    x, w_up, w_down = values(S, H), values(I, H), values(H, I) / 16
+    small, large = 2.0 ** exponent, 2.0 ** 90
+    if where == "x":
+        x, w_up = x * small, w_up * large
+    elif where == "w_up":
+        x, w_up = x * large, w_up * small
+    else:
+        x[1000], w_up = x[1000] * small, w_up * large
+        x[1001:] = x[1001:] / large
+    x, w_up, w_down = x.float(), w_up.float(), w_down.float()
+    iP = torch.cat([x.flatten(), w_up.flatten(), w_down.flatten(), torch.zeros(H + I)]).cuda()
+    ka.initialize(_keys(S, H, I, 1, 1, act=0, dt=1))
+    try:
+        oP = torch.zeros(S * H, device="cuda")
+        ka.moe.forward_host_dense(iP, oP)
+        ka.moe.stream_synchronize()
+        got = oP.view(S, H).cpu().double()
+    finally:
+        ka.finalize()
+
+    def operand(v):
+        return (v.view(torch.int32) & ~0x1fff).view(torch.float32).double()
+    want = torch.relu(operand(x) @ operand(w_up).T) @ w_down.double().T
+    rows = slice(None) if where != "one token" else slice(1000, 1001)
+    # h is rounded to 11 bits on the way, 2^-11 of each of its values at most, and the output once more
+    for part in (rows, slice(0, 1000), slice(1001, None)):
+        assert float((got - want)[part].norm()) <= (2.0 ** -11 + 1e-5) * float(want[part].norm())
