@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "layer.hpp"
 
@@ -84,16 +85,45 @@ template <> struct Elem16<f16_t> {
 __device__ __forceinline__ u32x4 load16(const void* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ __forceinline__ void store16(void* p, u32x4 v) { *reinterpret_cast<u32x4*>(p) = v; }
 
-// Phi(v) v, the erf form of GELU, without erff: with a = |v|,
-//   Phi(-a) = 0.5 erfc(a / sqrt 2) = exp(-a^2 / 2) t P(t),  t = 1 / (1 + 0.3 a),
-// P the polynomial of degree 7 of least largest relative error on 0 <= a <= 14 (1.4e-7; fitted by a linear program
-// over 1 800 points of scipy's erfcx). The form of Hastings' approximations. An epilogue holds up to 128 values a
-// lane and the activation is vector work that no matrix instruction covers: erff takes both of its branches in
-// nearly every wavefront, this takes 18 instructions and none. Against 64 bits on [-8, 8] in 32-bit arithmetic: largest error
-// 3.8e-7 and mean square 6.1e-8 (0.5 v (1 + erff(v / sqrt 2)): 4.5e-7 and 6.8e-8), and no cancellation for v < 0:
-// relative error 1.7e-6 at most instead of 1. Expert phase: 24 experts of 1 472 x 3 904, 1 920 tokens top-3, fp16: 200 ->
-// 189 us; one expert of 1 024 x 4 096, 2 048 tokens, bf16: 94.3 -> 90.6 us. Infinities and NaN give what the formula with erff gives: v times 1 or 0.
+// v Phi(v), the erf form of GELU, without erff: max(v, 0) - |v| Phi(-|v|), the maximum as (v + |v|) / 2 so that infinities
+// and NaN give what 0.5 v (1 + erff(v / sqrt 2)) gives. An epilogue holds up to 128 values a lane and the activation
+// is vector work that no matrix instruction covers; erff takes one of its branches where all values of a wavefront lie on
+// the same side of sqrt 2, and both elsewhere.
+// Phi(-a) = 2^-R(a), R the polynomial of degree 12 with R(0) = 1 that fits -log2 Phi(-a) best on [0, 9] (linear program
+// over 2 500 points of scipy's log_ndtr; error times ln 2, relative to Phi(-a): 2e-8 at 0, 1.2e-6 at 6, 3e-5 at 9; past
+// 9 R grows faster than it should and the value, below 1e-18, goes to 0 early). 18 instructions, one of them an exponential,
+// and no branch. Relative error (rms, largest) against 64 bits, in brackets that of the formula with erff, both emulated in
+// 32-bit arithmetic:
+//   0.1 <= |v| <= 0.5   5e-8, 1.7e-7  (4e-8, 1.5e-7)        -1.5 <= v <= -1   9e-8, 3.0e-7  (1.1e-7, 4.5e-7)
+//   -1 <= v <= -0.5     6e-8, 2.1e-7  (6e-8, 2.2e-7)        -3 <= v <= -2.5   3e-7, 1.1e-6  (3.5e-6, 1.2e-5)
+// and less than that of the formula for v > 0.5. Largest error on [-9, 9]: 2.4e-7 (4.5e-7).
+// us per forward: arguments of 0.4 (13 312 tokens, 8 experts top-4, 384 x 5 696, fp16) 771 with erff, 775 (827 with the
+// form of gelu_erf_32 for all arguments); of 0.8 (1 920 tokens, 24 experts top-3, 1 472 x 3 904, fp16) 265.5 (267.3); one
+// expert of 1 024 x 4 096, 2 048 tokens, bf16: 59.8 (62.1).
 __device__ __forceinline__ float gelu_erf(float v) {
+    const float a = __builtin_fminf(__builtin_fabsf(v), 64.0f);
+    float r = 1.04397678e-10f;
+    r = __builtin_fmaf(r, a, -5.55931567e-09f);
+    r = __builtin_fmaf(r, a, 1.31197893e-07f);
+    r = __builtin_fmaf(r, a, -1.80536017e-06f);
+    r = __builtin_fmaf(r, a, 1.59402152e-05f);
+    r = __builtin_fmaf(r, a, -9.17925572e-05f);
+    r = __builtin_fmaf(r, a, 0.000306411705f);
+    r = __builtin_fmaf(r, a, -2.20346319e-05f);
+    r = __builtin_fmaf(r, a, -0.00694667688f);
+    r = __builtin_fmaf(r, a, 0.0524530597f);
+    r = __builtin_fmaf(r, a, 0.459214509f);
+    r = __builtin_fmaf(r, a, 1.15110505f);
+    r = __builtin_fmaf(r, a, 1.0f);
+    return __builtin_fmaf(0.5f, __builtin_fabsf(v), 0.5f * v) - a * __builtin_amdgcn_exp2f(-r);
+}
+
+// fp32 results: far below zero the polynomial's R, some tens, has too few bits left for 32. From -2 down
+//   Phi(-a) = 0.5 erfc(a / sqrt 2) = exp(-a^2 / 2) t P(t),  t = 1 / (1 + 0.3 a),
+// the form of Hastings' approximations, P the polynomial of degree 7 of least largest relative error on 0 <= a <= 14
+// (1.4e-7; 1 800 points of scipy's erfcx): relative error 1.7e-7 rms at -2.5, 2.7e-6 at most at -8, 8e-6 at -13. (Towards
+// 0 its terms cancel to 0.5 and cost three bits; it is not used there.)
+__device__ __forceinline__ float gelu_erf_32(float v) {
     const float a = __builtin_fabsf(v);
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3f, a, 1.0f));
     float s = 0.03556416556239128f;
@@ -104,15 +134,15 @@ __device__ __forceinline__ float gelu_erf(float v) {
     s = __builtin_fmaf(s, t, 0.0999893993139267f);
     s = __builtin_fmaf(s, t, 0.12074293196201324f);
     s = __builtin_fmaf(s, t, 0.11962994933128357f);
-    const float tail = s * t * __builtin_amdgcn_exp2f(a * a * -0.72134752044448170368f);   // 0.5 log2 e
-    return v * (v > 0.0f ? 1.0f - tail : tail);
+    const float far = v * (s * t * __builtin_amdgcn_exp2f(a * a * -0.72134752044448170368f));   // 0.5 log2 e
+    return v < -2.0f ? far : gelu_erf(v);
 }
 
-// Activations of the reference (types.cuh:151-159): 0 = ReLU<float>, 1 = erf GELU<float>.
-template <int ACT>
+// Activations of the reference (types.cuh:151-159): 0 = ReLU<float>, 1 = erf GELU<float>. T: the Element the result becomes.
+template <int ACT, typename T>
 __device__ __forceinline__ float activate(float v) {
     if constexpr (ACT == 0) return v > 0.0f ? v : 0.0f;
-    else if constexpr (ACT == 1) return gelu_erf(v);
+    else if constexpr (ACT == 1) return std::is_same<T, float>::value ? gelu_erf_32(v) : gelu_erf(v);
     else return v;
 }
 

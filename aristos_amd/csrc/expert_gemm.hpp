@@ -163,7 +163,7 @@ __device__ __forceinline__ void epilogue16_act(const TileOut& t, f32x16 (&acc)[W
                     vec4 o;
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        o[j] = static_cast<E>(activate<ACT>(acc[ni][mi][4 * q + j] + float(b4[j])));
+                        o[j] = static_cast<E>(activate<ACT, E>(acc[ni][mi][4 * q + j] + float(b4[j])));
                     *reinterpret_cast<vec4*>(stg + fr_row * 128 + (((nl * 4 + q) ^ ((fr_row >> 1) & 7)) << 4) + fr_half * 8) = o;
                 }
             }
@@ -221,7 +221,7 @@ __device__ __forceinline__ void epilogue16_act(const TileOut& t, f32x4 (&acc)[WN
                     vec4 o;
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        o[j] = static_cast<E>(activate<ACT>(acc[ni][pm * 2 + ml][j] + float(b4[j])));
+                        o[j] = static_cast<E>(activate<ACT, E>(acc[ni][pm * 2 + ml][j] + float(b4[j])));
                     // columns nl*16 + 4*fr_part .. + 3 of the panel: chunk 2*nl + fr_part/2, half fr_part%2
                     *reinterpret_cast<vec4*>(stg + r * 128 + (((2 * nl + (fr_part >> 1)) ^ ((r >> 1) & 7)) << 4) + (fr_part & 1) * 8) = o;
                 }
@@ -951,7 +951,7 @@ struct GemmKSplit {
                     const char* at = smem + r * (BN * 4) + (((2 * c + h) ^ (r & 15)) << 4);
                     const f32x4 a = *reinterpret_cast<const f32x4*>(at), b = *reinterpret_cast<const f32x4*>(at + G::kSmemBytes);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) o[4 * h + j] = static_cast<E>(activate<ACT>(a[j] + b[j] + float(bias[4 * h + j])));
+                    for (int j = 0; j < 4; ++j) o[4 * h + j] = static_cast<E>(activate<ACT, E>(a[j] + b[j] + float(bias[4 * h + j])));
                 }
                 constexpr int kAgentScope = 16;   // sc1: written through the L2, like every output row
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), coherent_rows(t.half.c_base),
@@ -1186,7 +1186,7 @@ struct Gemm32 {
                     f32x4 v;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        v[j] = activate<ACT>(acc[ni][mi][4 * q + j] + b4[j]);
+                        v[j] = activate<ACT, T>(acc[ni][mi][4 * q + j] + b4[j]);
                         if constexpr (kTf32) v[j] = tf32_round(v[j]);
                     }
                     *reinterpret_cast<f32x4*>(stg + fr_row * 128 + (((2 * q + fr_half) ^ ((fr_row >> 1) & 7)) << 4)) = v;
@@ -1337,7 +1337,7 @@ struct Gemm32Wave {
         v += *reinterpret_cast<const f32x4*>(smem + kBiasOffset + t.bias_slot * kBiasBytes + c * 16);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            v[j] = activate<ACT>(v[j]);
+            v[j] = activate<ACT, T>(v[j]);
             if constexpr (Base::kTf32) v[j] = tf32_round(v[j]);
         }
         constexpr int kAgentScope = 16;   // sc1

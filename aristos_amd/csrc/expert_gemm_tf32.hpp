@@ -443,7 +443,7 @@ struct GemmSplit {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const float s = sum[ni][j] + b4[j];
-                    v[j] = tf32_round(t.act == 0 ? activate<0>(s) : (t.act == 1 ? activate<1>(s) : activate<2>(s)));
+                    v[j] = tf32_round(t.act == 0 ? activate<0, tf32_t>(s) : (t.act == 1 ? activate<1, tf32_t>(s) : activate<2, tf32_t>(s)));
                 }
                 if (m < t.m_valid && n < t.n_valid) store16_through(t.c_base + size_t(m) * t.ldc + n, __builtin_bit_cast(u32x4, v));
             }
@@ -469,7 +469,7 @@ struct GemmSplit {
                         const f32x4 b4 = *reinterpret_cast<const f32x4*>(bias + ni * 16 * 4);
                         f32x4 v;
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) v[j] = tf32_round(activate<ACT>(acc[ni][2 * pm + ml][j] + b4[j]));
+                        for (int j = 0; j < 4; ++j) v[j] = tf32_round(activate<ACT, tf32_t>(acc[ni][2 * pm + ml][j] + b4[j]));
                         *reinterpret_cast<f32x4*>(stg + r * 128 + (((4 * nl + fr_part) ^ ((r >> 1) & 7)) << 4)) = v;
                     }
 #pragma unroll

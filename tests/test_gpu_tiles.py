@@ -299,3 +299,28 @@ def test_tf32_operands_below_what_splits_exactly(where, exponent):
     # h is rounded to 11 bits on the way, 2^-11 of each of its values at most, and the output once more
     for part in (rows, slice(0, 1000), slice(1001, None)):
         assert float((got - want)[part].norm()) <= (2.0 ** -11 + 1e-5) * float(want[part].norm())
+
+
+@pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
+@pytest.mark.parametrize("low,high", [(0.001, 0.1), (0.1, 0.5), (0.5, 1.0), (1.0, 2.0)])
+def test_gelu_keeps_the_bits_of_small_arguments(low, high, sign):
+    """fp32, both projections the identity: no more than the roundings of 32-bit arithmetic between v Phi(v) and the
+    result. Exponent (its last rounding only, of at most 2.7, times ln 2, below |v| = 1), exponential, product, difference
+    and the fit's 2e-8: six of 2^-24 / sqrt 3 together in the mean square. Below -1 the difference of two numbers up to
+    six times the result, and an exponent of up to 5.5, four times that; 0.5 v (1 + erff(v / sqrt 2)) has 2.7e-7 there."""
+    S, H = 1024, 64
+    v = torch.from_numpy(sign * np.random.default_rng(3).uniform(low, high, S * H)).float()
+    eye = torch.eye(H)
+    iP = torch.cat([v, eye.flatten(), eye.flatten(), torch.zeros(2 * H)]).cuda()
+    ka.initialize(_keys(S, H, H, 1, 1, act=1, dt=0))
+    try:
+        oP = torch.empty(S * H, device="cuda")
+        ka.moe.forward_host_dense(iP, oP)
+        ka.moe.stream_synchronize()
+        got = oP.cpu().double().numpy()
+    finally:
+        ka.finalize()
+    v = v.double().numpy()
+    want = v * 0.5 * erfc(-v / np.sqrt(2.0))
+    rms = float(np.sqrt(np.mean(((got - want) / want) ** 2)))
+    assert rms <= 6 ** 0.5 * 2.0 ** -24 / 3 ** 0.5 * (4 if low >= 1.0 and sign < 0 else 1), rms
