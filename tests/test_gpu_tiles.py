@@ -324,3 +324,17 @@ def test_gelu_keeps_the_bits_of_small_arguments(low, high, sign):
     want = v * 0.5 * erfc(-v / np.sqrt(2.0))
     rms = float(np.sqrt(np.mean(((got - want) / want) ** 2)))
     assert rms <= 6 ** 0.5 * 2.0 ** -24 / 3 ** 0.5 * (4 if low >= 1.0 and sign < 0 else 1), rms
+
+
+@pytest.mark.parametrize("dt,S,H,E", [
+    (2, 128, 64, 8), (2, 128, 448, 8), (3, 128, 832, 64),       # whole units whose shares are 0 to 4 steps
+    (2, 8192, 1472, 16), (2, 8192, 1856, 40),                   # 5 and 6, 7 and 8 steps beside whole batches of 8 and of 4
+    (3, 128, 3904, 16), (2, 128, 2944, 20), (3, 128, 1984, 8),  # spread tiles: 15 and 16, 11 and 12, 7 and 8 steps
+    (0, 256, 320, 30), (1, 128, 704, 100),                      # 32-bit types: 16 values a step
+], ids=lambda v: str(v))
+def test_gate_shares_of_every_length(dt, S, H, E):
+    """The steps of a share that do not fill a batch of loads, as runs of 8, 4, 2 and 1."""
+    keys = _keys(S, H, 64, E, 1, dt=dt)
+    c = moe_ref.cfg_from_keys(keys)
+    iP = pack_inputs(c, *random_layer(c, seed=H + E, w_std=0.05, bias_std=0.1))
+    check_against_oracle(c, keys, iP, ka.MODE_FUSED)
