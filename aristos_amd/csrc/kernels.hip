@@ -162,6 +162,19 @@ hipError_t dispatch_dtype(int dtype, F&& go) {
     }
 }
 
+void tile_sizes(const LayerParams& p, int dtype, uint32_t sizes[4]) {
+    (void)dispatch_dtype(dtype, [&](auto tag) {
+        using T = decltype(tag);
+        return dispatch_variant<T>(p, [&](auto variant) {
+            constexpr int V = decltype(variant)::value;
+            const bool small = small_down<T, V>(p);
+            sizes[0] = TileShape<T, V>::BM; sizes[1] = TileShape<T, V>::BN;
+            sizes[2] = small ? kNarrowTileRows<V> : sizes[0]; sizes[3] = small ? kNarrowTileCols<V> : sizes[1];
+            return hipSuccess;
+        });
+    });
+}
+
 hipError_t launch_gate(const LayerParams& p, int dtype, int num_cus, hipStream_t s) {
     return dispatch_dtype(dtype, [&](auto tag) { return launch_gate_t<decltype(tag)>(p, num_cus, s); });
 }

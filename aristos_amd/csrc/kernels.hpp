@@ -14,6 +14,8 @@ uint32_t sched_error_word();
 // The tile variant of the expert projections for a layer, for LayerParams::tile_variant (needs S, H, I, E,
 // k, EC and cap_rows of p). Whatever launches an expert projection must have it set.
 void choose_tiles(LayerParams& p, int dtype, int num_cus);
+// Rows and columns of the tiles of both projections (up, then down), for a layer whose tiles are chosen.
+void tile_sizes(const LayerParams& p, int dtype, uint32_t sizes[4]);
 // Phase launchers (KLEOS_MODE_PHASED). dtype: 0 fp32, 2 bf16.
 hipError_t launch_gate(const LayerParams& p, int dtype, int num_cus, hipStream_t s);
 // Ranges the gate splits the hidden dimension into when it computes its logits as a tiled product
@@ -35,7 +37,6 @@ struct FusedPlan {
     size_t smem = 0;
     uint32_t mt_max = 0;   // row blocks per expert at full capacity
     uint32_t lag = 0;      // experts between an up-projection segment and its down-projection segment
-    double tile_share = 1.0;   // what a tile of the K-halving variants counts for in the scheduler statistics: its share of 256 x 256
     bool cooperative = false;   // launch through hipLaunchCooperativeKernel (residency verified per launch)
 };
 hipError_t plan_fused(const LayerParams& p, int dtype, int num_cus, FusedPlan* plan);

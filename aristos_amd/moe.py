@@ -81,6 +81,15 @@ def debug_mfma_probe(tile: int, iterations: int = 20000, zero_operands: bool = F
     return {"ms": float(ms.value), "tflops": float(flop.value) / (float(ms.value) * 1e-3) / 1e12}
 
 
+def debug_tiles(config, compute_units: int = 256) -> dict:
+    """kleos_debug_tiles: the tile variant of the layer `config` (a KleosConfig) on a device of that many CUs
+    and the rows and columns of the tiles of its two projections. Needs no GPU."""
+    st = config.to_struct()
+    out = (C.c_uint32 * 6)()
+    _capi.check(_capi.lib().kleos_debug_tiles(C.byref(st), int(compute_units), out))
+    return {"variant": out[0], "down_small": out[1], "up": (out[2], out[3]), "down": (out[4], out[5])}
+
+
 def set_schedule(schedule: int) -> None:
     """SCHEDULE_AUTO (default), SCHEDULE_DYNAMIC or SCHEDULE_STATIC: how the persistent launch hands
     out expert tiles."""

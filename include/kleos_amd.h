@@ -272,9 +272,8 @@ int kleos_phase_times(float ms[5]);
  * KLEOS_MODE_FUSED (the persistent kernel keeps them per workgroup; the reference has no
  * counterpart): [0..2] mean milliseconds a workgroup spent fetching tasks, waiting for an
  * unfinished dependency, publishing finished tiles; [3] expert tiles executed; [4] tiles handed out
- * before their inputs were complete; [5] tiles taken from another XCD's queue. A 16-bit layer too small
- * for tiles of 256 columns runs on tiles of 128 x 128 or 64 x 128; these count as the part of a 256 x 256
- * tile that they are. */
+ * before their inputs were complete; [5] tiles taken from another XCD's queue. Tiles of whatever size
+ * the layer's projections run on (kleos_debug_tiles). */
 int kleos_scheduler_stats(double stats[6]);
 /* Replaces kleos::mT (csrc/include/kleos/throughput.cuh:104-170), the probe the reference runs at
  * start-up to rate a device: one expert at full padded capacity (pEC rows) through the up-projection,
@@ -323,6 +322,12 @@ int kleos_debug_skip_launch_number(void);
  * counters instead of 0, so that with a non-zero skip every barrier runs into the limit, every kernel
  * still exits, and the status call reports the expiry. (0, 0) restores normal operation. */
 int kleos_debug_static_scratch_expiry(unsigned long long ticks, uint32_t skip_launch_numbers);
+/* The tiles the expert projections of the layer `cfg` run on, on a device of `compute_units` CUs:
+ * tiles[0] the variant of the kernel, [1] 1 when the down-projection has a tile of its own, [2] and [3]
+ * rows and columns of an up-projection tile, [4] and [5] of a down-projection tile (variant 2 hands a
+ * row block of at most 128 rows to a tile of that height). Touches no device. For tests and for whoever
+ * reads kleos_scheduler_stats. */
+int kleos_debug_tiles(const kleos_config_t* cfg, uint32_t compute_units, uint32_t tiles[6]);
 /* The code and message a failed HIP runtime call turns into at this boundary: KLEOS_OK for
  * hipSuccess (0), else KLEOS_EHIP with the runtime's name and description of `hip_error` in
  * kleos_last_error(). Touches no device: lets a test pin, for instance, what a refused cooperative

@@ -529,8 +529,9 @@ def test_timing_interfaces_of_the_persistent_launch():
     assert stamps.shape[1] == 8 and stamps.shape[0] >= 1
     assert (np.diff(stamps.astype(np.int64), axis=1) >= 0).all()
     kept = np.minimum(v["expert_count"].astype(np.int64), d.kept_capacity)
-    row_blocks = -(-kept // 256)
-    assert int(st["tiles"]) == int(row_blocks.sum()) * (-(-d.I // 256) + -(-d.H // 256))
+    tiles = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
+    (um, un), (dm, dn) = tiles["up"], tiles["down"]
+    assert st["tiles"] == int((-(-kept // um)).sum()) * -(-d.I // un) + int((-(-kept // dm)).sum()) * -(-d.H // dn)
     assert st["foreign_tiles"] <= st["tiles"]
 
 

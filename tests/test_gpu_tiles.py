@@ -338,3 +338,24 @@ def test_gate_shares_of_every_length(dt, S, H, E):
     c = moe_ref.cfg_from_keys(keys)
     iP = pack_inputs(c, *random_layer(c, seed=H + E, w_std=0.05, bias_std=0.1))
     check_against_oracle(c, keys, iP, ka.MODE_FUSED)
+
+
+@pytest.mark.parametrize("schedule", [ka.SCHEDULE_DYNAMIC, ka.SCHEDULE_STATIC], ids=["dynamic", "static"])
+@pytest.mark.parametrize("dt,S,H,I,E,k", [(2, 128, 1024, 2048, 16, 2), (3, 640, 448, 2816, 64, 2), (2, 2048, 1024, 4096, 1, 1), (0, 128, 256, 512, 8, 2)],
+                         ids=lambda v: str(v))
+def test_scheduler_statistics_count_tiles(dt, S, H, I, E, k, schedule):
+    """kleos_scheduler_stats counts every tile once, whatever its size, also where the down-projection has one of its own."""
+    keys = _keys(S, H, I, E, k, dt=dt)
+    c = moe_ref.cfg_from_keys(keys)
+    iP = _to_device(c, pack_inputs(c, *random_layer(c, seed=S + I, w_std=0.05)))
+    d = ka.initialize(keys)
+    try:
+        ka.moe.set_schedule(schedule)
+        ka.moe.forward_host_bench(iP, synth.alloc_outputs(d), skip=1, trials=2)
+        st, v = ka.moe.scheduler_stats(), ka.moe.debug_views(d)
+    finally:
+        ka.finalize()
+    kept = np.minimum(v["expert_count"].astype(np.int64), d.kept_capacity)
+    tiles = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
+    (um, un), (dm, dn) = tiles["up"], tiles["down"]
+    assert st["tiles"] == int((-(-kept // um)).sum()) * -(-I // un) + int((-(-kept // dm)).sum()) * -(-H // dn)
