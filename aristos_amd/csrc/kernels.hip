@@ -2,6 +2,8 @@
 // sizing, the slot kernel, the launch of a planned persistent kernel, and the switch over the
 // Element type in front of the launchers that kernels_f32.hip, kernels_bf16.hip and kernels_f16.hip
 // instantiate (kernels_impl.hpp).
+#include <cmath>
+
 #include "kernels_impl.hpp"
 
 namespace kleos_amd {
@@ -64,7 +66,28 @@ uint32_t mean_rows(const LayerParams& p) {
     if (rows > cap) rows = cap;
     return rows < 1 ? 1u : rows;
 }
-// A 16-bit tile by what a CU loads and multiplies (the figures at choose_tiles).
+// Rows an expert may hold, and for which share of the experts.
+struct RowShare { double rows, share; };
+// Routing that favours nobody gives an expert its mean, give or take the root of it. Where the capacity leaves room for
+// more than that (two and a half times the mean) one expert in ten is taken to be hot and hold twice the mean (of the shares and factors tried the one that loses to
+// the capacity rule at the fewest of the layers below); a single expert holds what it holds.
+int row_shares(const LayerParams& p, RowShare out[4]) {
+    const double cap = p.EC < p.cap_rows ? p.EC : p.cap_rows;
+    double mean = double(p.S) * p.k / p.E;
+    if (mean > cap) mean = cap;
+    auto held = [&](double rows) { return rows < 1.0 ? 1.0 : (rows > cap ? cap : rows); };
+    if (p.E == 1) { out[0] = RowShare{held(mean), 1.0}; return 1; }
+    const bool hot = cap >= 2.5 * mean;
+    const double all = hot ? 1.1 : 1.0, sigma = std::sqrt(mean);
+    out[0] = RowShare{held(mean - sigma), 0.25 / all};
+    out[1] = RowShare{held(mean), 0.5 / all};
+    out[2] = RowShare{held(mean + sigma), 0.25 / all};
+    if (hot) out[3] = RowShare{held(2.0 * mean), 0.1 / all};
+    return hot ? 4 : 3;
+}
+// A 16-bit tile by what a CU loads and multiplies (the figures at choose_tiles). The rows a tile has beyond the expert's
+// read one row of zeros and are not charged: charged like the others, the rule does 0.2 % better in the mean of the layers
+// below and loses to the capacity rule at some more of them.
 TileCost tile16_cost(uint32_t bm, uint32_t bn, uint32_t rows) {
     const uint32_t r = rows < bm ? rows : bm;
     const double load = (r + bn) * 2.0 / 47e3, multiply = 2.0 * (ceil_div_u32(r, 16) * 16) * bn / 5.1e6;
@@ -73,18 +96,20 @@ TileCost tile16_cost(uint32_t bm, uint32_t bn, uint32_t rows) {
 }  // namespace
 
 // The variants differ in how many rows and columns a tile has, so in how many rounds the CUs need for all of a
-// layer's tiles, and in the bytes and operations of a round. The estimate below, of both projections of experts
-// that hold their mean rows, decides:
-//   - a CU takes in about 47 KB a microsecond whatever it loads (measured over all 16-bit variants), a tile
-//     rows + columns of 2 bytes per value of K; 256 x 256 tiles also come close to the matrix rate, 5.1 GFLOP a
-//     millisecond and CU;
+// layer's tiles, and in the bytes and operations of a round. The estimate below, of both projections, decides:
+//   - an expert holds the rows of row_shares, so many row blocks on average;
+//   - a CU takes in about 47 KB a microsecond whatever it loads, a tile rows + columns of 2 bytes per value of K; 256 x 256
+//     tiles also come close to the matrix rate, 5.1 GFLOP a millisecond and CU;
 //   - a tile costs 5 us besides (look-ups, first slices, epilogue);
 //   - the weights pass at no more than 6.2 TB/s (tiles that share weights read them with the default policy, whose
-//     rate for weights read once is an eighth lower), and of two variants bound by that the larger tile is taken.
-// Measured against every variant at nineteen layers between 128 and 8 192 tokens and 1 and 256 experts it picks the
-// best one or one within 10 % of it. Where it moves a layer from the 256- and 128-row tiles to the smaller ones: 640
-// tokens, 8 experts top-2, 704 x 512: 58 -> 37 us per forward; 2 176 tokens, 16 experts top-2, 2 048 x 512: 91 -> 75;
-// 2 048 tokens, one expert, 1 024 x 4 096: 148 -> 108.
+//     rate for weights read once is an eighth lower), and of two variants bound by that the one considered first is taken:
+//     the large tile, then as below.
+// Measured against every variant at 487 layers drawn between 128 and 15 616 tokens, 1 and 511 experts, with and without
+// dropping and skew: 3.2 % from the best of them in the mean, more than 10 % at 59 of them; 15 % faster in the mean than a
+// choice by capacity alone (variant 1 up to 128 rows, 2 from 1 024, else 0), more than 3 % slower at seven (13 with
+// every expert at its mean). Where it moves a layer from the
+// 256- and 128-row tiles to the smaller ones: 640 tokens, 8 experts top-2, 704 x 512: 58 -> 37 us per forward; 2 176
+// tokens, 16 experts top-2, 2 048 x 512: 91 -> 75; 2 048 tokens, one expert, 1 024 x 4 096: 148 -> 108.
 // tf32: 256 x 256 tiles on the bf16 matrix cores, 128 clocks per value of K, one on a CU, against 64 x 64 tiles on
 // the fp32 ones, 32 clocks, two on a CU in turn (8 192 tokens, 64 experts top-2, 2 048 x 2 048: 512 : 2 048 by this
 // rule, 975 : 2 729 us measured).
@@ -98,16 +123,25 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
         const double plain = projections_us(p, TileCost{64, 64, 32.0, 0.0}, rows, num_cus, false);
         if (dtype == 1 && split < plain) p.tile_variant = 3u;
         // The 32 x 32 tile takes 12 clocks per value of K on a busy CU (its loads); a tile costs some 3 us besides. Its row
-        // blocks need a readiness counter each, of which there is one per 64 rows that an expert's arrays hold.
+        // blocks need a readiness counter each, of which there is one per 64 rows that an expert's arrays hold: that, not
+        // a measurement, keeps it to experts of at most 64 rows.
         const double medium = projections_us(p, TileCost{64, 64, 32.0, 6500.0}, rows, num_cus, false);
         const double small = projections_us(p, TileCost{32, 32, 12.0, 6500.0}, rows, num_cus, false);
         if (p.tile_variant == 0u && small < medium && ceil_div_u32(cap, 32) <= ceil_div_u32(p.cap_rows, 64)) p.tile_variant = 7u;
         return;
     }
     // (bm x bn tiles, the down-projection on dm x dn tiles)
+    RowShare shares[4];
+    const int n_shares = row_shares(p, shares);
+    auto projection = [&](uint32_t bm, uint32_t bn, uint32_t N, uint32_t K) {
+        double blocks = 0.0;
+        for (int i = 0; i < n_shares; ++i) blocks += shares[i].share * std::ceil(shares[i].rows / bm - 1e-9);
+        const double rounds = p.E * blocks * ceil_div_u32(N, bn) / num_cus;
+        const TileCost t = tile16_cost(bm, bn, rows);
+        return double(uint64_t(rounds + 0.999999)) * (K * t.per_k + t.fixed);
+    };
     auto estimate = [&](uint32_t bm, uint32_t bn, uint32_t dm, uint32_t dn, bool streams) {
-        const double tiles = projection_us(p, tile16_cost(bm, bn, rows), p.I, p.H, rows, num_cus, true) +
-                             projection_us(p, tile16_cost(dm, dn, rows), p.H, p.I, rows, num_cus, true);
+        const double tiles = projection(bm, bn, p.I, p.H) + projection(dm, dn, p.H, p.I);
         double memory = 4.0 * p.E * p.H * double(p.I) / 6.2e6;
         if (!streams && rows <= bm) memory *= 1.12;
         return (tiles > memory ? tiles : memory) + 0.1 * tiles;
@@ -123,22 +157,30 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
         if (estimated < us) { us = estimated; p.tile_variant = variant; p.down_small = small; }
     };
     // Experts of several row blocks each, one and more to an XCD: the 256-row tiles, which share their weights through
-    // an L2 and mix heights, without asking (4 096 tokens, 8 experts top-2, 1 024 x 1 024: 75 us against 90 with 128 x
-    // 128 tiles; 8 192 tokens, 12 experts, 768 x 3 072: 211 against 292; only the smallest lose, 53 against 47 at 512 x 512).
+    // an L2 and mix heights, without asking; the estimate does not know of the sharing. (4 096 tokens, 8 experts top-2,
+    // 1 024 x 1 024: 75 us against 90 with 128 x 128 tiles; 8 192 tokens, 12 experts, 768 x 3 072: 211 against 292; the
+    // smallest lose, 53 against 47 at 512 x 512. Where exactly the line should lie, below 8 experts and 512 rows, is not measured.)
     const bool many = cap >= kSharedRows && rows >= kSharedRows / 2 && p.E >= 8;
     const bool narrow = rows <= kNarrowRows, shared = cap >= kSharedRows;
     if (narrow) {
         consider(1, 0, estimate(128, 256, 128, 256, true));
         consider(1, 1, two_tiles(128, 256, 128, 128, true));
-    } else {
-        consider(shared ? 2 : 0, 0, estimate(256, 256, 256, 256, !shared));
-        if (!many) consider(2, 1, two_tiles(256, 256, 128, 256, false));   // (variant 2 halves the last tiles of many rows anyway)
     }
+    if (!narrow || cap > kNarrowRows) consider(shared ? 2 : 0, 0, estimate(256, 256, 256, 256, !shared));
+    if (!narrow && !many) consider(2, 1, two_tiles(256, 256, 128, 256, false));   // (variant 2 halves the last tiles of many rows anyway)
     if (many) return;
+    // 64 rows: the weights non-temporally (6) where an expert reads them once and they bound the layer. Where no expert is
+    // likely to hold more, a tile of 128 takes in no more rows and gains nothing on one of 64, which then comes first (40 such
+    // layers: 4 to 7 % faster than on 128).
+    const bool single = rows <= 64, likely = rows <= 32 || cap <= 64;
+    auto low = [&] {
+        consider(5, 0, estimate(64, 128, 64, 128, false));
+        if (single) consider(6, 0, estimate(64, 128, 64, 128, true));
+    };
+    if (likely) low();
     consider(4, 0, estimate(128, 128, 128, 128, false));
     consider(4, 1, two_tiles(128, 128, 64, 128, false));
-    const bool single = rows <= 64;
-    consider(single ? 6 : 5, 0, estimate(64, 128, 64, 128, single));
+    if (!likely) low();
 }
 
 uint32_t gate_splits_for(uint32_t S, uint32_t H, uint32_t E, uint32_t PX, int dtype, int num_cus) {
