@@ -171,13 +171,13 @@ CASES = [
     (256, 128, 192, 8, 2, 1.0, 1, 0, 1, 0.1),      # tf32 (the dtype the reference ships): 32-bit Elements of 10 mantissa bits
     (512, 192, 128, 64, 2, 1.0, 1, 1, 1, 0.1),     # tf32, E = 64, gelu
     (256, 64, 64, 300, 4, 1.0, 1, 0, 1, 0.0),      # tf32, E = 300: the gate in passes
-    (1024, 192, 320, 4, 2, 1.0, 1, 0, 2, 0.1),     # 512 rows per expert: 256-row tiles, odd slice counts
-    (512, 64, 64, 2, 1, 1.0, 1, 1, 2, 0.1),        # 256-row tiles over a single K slice
-    (768, 128, 192, 2, 2, 1.0, 1, 0, 3, 0.0),      # fp16, 256-row tiles, a partial row block
+    (1024, 192, 320, 4, 2, 1.0, 1, 0, 2, 0.1),     # 512 rows per expert, odd slice counts
+    (512, 64, 64, 2, 1, 1.0, 1, 1, 2, 0.1),        # a single K slice
+    (768, 128, 192, 2, 2, 1.0, 1, 0, 3, 0.0),      # fp16, a partial row block
     (256, 128, 256, 8, 2, 1.0, 1, 0, 3, 0.0),      # fp16
     (256, 192, 320, 12, 3, 1.0, 1, 1, 3, 0.1),     # fp16, gelu + biases, ragged sizes
     (512, 256, 256, 64, 2, 1.0, 1, 0, 3, 0.0),     # fp16, E = 64, several K slices
-    (2048, 192, 320, 2, 2, 1.0, 1, 1, 2, 0.1),     # 2048 rows per expert: the tile variant of large experts
+    (2048, 192, 320, 2, 2, 1.0, 1, 1, 2, 0.1),     # 2048 rows per expert
     (512, 128, 64, 320, 8, 1.0, 1, 0, 2, 0.0),     # E > 256: the gate in passes of 256 experts
     (256, 192, 64, 512, 6, 2.0, 1, 1, 2, 0.1),     # E = 512, cf = 2, gelu + biases
     (256, 64, 64, 384, 4, 1.0, 1, 0, 0, 0.0),      # fp32, E = 384
@@ -274,8 +274,8 @@ def test_identity_experts_return_input(mode):
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("k", [1, 2])
 def test_tile_heights_mixed_inside_one_layer(mode, k):
-    """A layer whose experts may hold 1024 rows and more walks 256-row blocks, and gives an expert's last
-    block to a 128-row tile when it holds at most 128 rows: experts of 40, 100, 129, 300, 2100 and 403
+    """A layer of large experts walks 256-row blocks, and gives an expert's last block to a 128-row tile when
+    it holds at most 128 rows (k = 2; with k = 1 the experts' mean is low enough for smaller tiles): experts of 40, 100, 129, 300, 2100 and 403
     rows (and two without any) in one launch, i.e. blocks of 40 and 100 rows (128-row tile), 129 rows
     (256-row tile), 256 + 44, 8 x 256 + 52 (full tiles followed by a 128-row tile) and 256 + 147. With
     k = 2 every token also goes to the next expert, which gives blocks of 140, 229, 173, 96 and 199
@@ -397,9 +397,9 @@ def test_dense_packing_of_a_single_expert(dt):
 # ------------------------------------------------------------------ back-to-back launches
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 def test_experts_that_fill_a_tile_to_every_quarter(mode):
-    """256-row tiles (the variant for experts of 129 to 1023 rows) whose experts hold 12, 62, 81, 147, 220
-    and 256 + 64 rows: the wavefronts of a tile own 64 rows each, and those whose rows do not exist leave
-    the arithmetic of the tile out. A constant input feature times a per-expert gate weight skews the
+    """Experts that hold 12, 62, 81, 147, 220 and 256 + 64 rows: the wavefronts of a 256-row tile own 64 rows
+    each, and those whose rows do not exist leave the arithmetic of the tile out. (A layer this small runs on
+    smaller tiles; test_gpu_tiles.py holds layers to every pair of tiles at the edges of its rows.) A constant input feature times a per-expert gate weight skews the
     routing; the two hottest experts overflow their capacity of 512."""
     keys = _keys(1024, 128, 256, 8, 2, cf=2.0)
     c = moe_ref.cfg_from_keys(keys)
@@ -435,8 +435,9 @@ def _one_hot_layer(c, rows, seed):
 def test_experts_that_end_inside_and_at_the_edges_of_16_row_blocks(mode, variant):
     """A wavefront computes only the blocks of 16 rows that hold rows of its tile (four versions of the
     main loop, for 1 to 4 blocks of its 64 rows). Experts of 1, 15, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65,
-    ... rows put the last row at the start, inside and at the end of every such block, in the 256-row
-    tile (capacity 256) and in the 128-row tile (capacity 128)."""
+    ... rows put the last row at the start, inside and at the end of every such block, with a capacity of
+    256 and of 128. (Layers this small run on 128- and 64-row tiles of either capacity; test_gpu_tiles.py holds
+    layers to every pair of tiles at these edges.)"""
     if variant == "256-row tiles":
         rows = [1, 15, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65, 100, 129, 200, 255]
         S, E = 2048, 32

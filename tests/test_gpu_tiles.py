@@ -83,9 +83,9 @@ def test_tf32_infinities_on_the_bf16_matrix_cores(where):
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("H,I,rows,cf", [
-    (64, 64, [1, 15, 16, 17, 31, 32, 33, 47, 63, 64, 65, 40, 30, 40, 20, 30], 2.0),          # 64-row tiles, one K slice: the second group has none
-    (192, 320, [1, 15, 16, 17, 31, 32, 33, 47, 63, 64, 65, 40, 30, 40, 20, 30], 2.0),        # the same over three and five slices, a last column tile of 64
-    (320, 448, [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 100, 60, 90, 130], 3.0),   # two row blocks and more
+    (64, 64, [1, 15, 16, 17, 31, 32, 33, 47, 63, 64, 65, 40, 30, 40, 20, 30], 2.0),          # 128-row tiles, one K slice: the second group has none
+    (192, 320, [1, 15, 16, 17, 31, 32, 33, 47, 63, 64, 65, 40, 30, 40, 20, 30], 2.0),        # three and five slices, a last column tile of 64
+    (320, 448, [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 100, 60, 90, 130], 3.0),   # 64-row tiles, two row blocks and more
     (1152, 1216, [1, 63, 64, 65, 111, 112, 113, 127, 128, 129, 200, 256, 257, 150, 140, 130], 3.0),   # 128-row tiles
     (1152, 64, [128, 120, 130, 126, 129, 127, 128, 128, 64, 100, 255, 1, 128, 128, 160, 162], 3.0),    # 128-row tiles, one K slice down
 ], ids=["64x64", "192x320", "320x448", "1152x1216", "1152x64"])
@@ -182,14 +182,15 @@ def test_32_bit_tiles_of_few_rows(mode, dt, H, I, act):
 
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("dt,H,I,rows,cf", [
-    (2, 64, 4096, [96, 97, 127, 128, 64, 65, 100, 91], 1.5),                # 128 x 256 up, 128 x 128 down: one column tile of 64
-    (3, 320, 4160, [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 384], 2.0),   # row blocks of two smaller ones, the last of them cut short
-    (2, 320, 6144, [1, 127, 128, 129, 255, 256, 257, 385, 512, 640], 2.5),  # 256 x 256 up, 128 x 256 down
+    (2, 64, 4096, [96, 97, 127, 128, 64, 65, 100, 91], 1.5),                # 64 x 128 both ways: one column tile of 64 down
+    (3, 320, 4160, [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 384], 2.0),   # 64 x 128 both ways, experts of up to six row blocks
+    (2, 320, 6144, [1, 127, 128, 129, 255, 256, 257, 385, 512, 640], 2.5),  # 128 x 128 up, 64 x 128 down: row blocks of two smaller ones, the last of them cut short
     (2, 192, 4096, [2304], 1.0),                                           # one expert, its row blocks dealt to the queues, an odd last one
     (3, 192, 4096, [1792], 1.0),
 ], ids=lambda v: str(v) if not isinstance(v, list) else str(len(v)) + "e")
 def test_down_projection_on_the_smaller_tile(mode, dt, H, I, rows, cf):
-    """Wide up-projections whose long, few down-projection tiles leave CUs idle."""
+    """Wide up-projections whose long, few down-projection tiles leave CUs idle. (The other pairs with a smaller tile
+    down: test_every_pair_of_16_bit_tiles_at_the_edges_of_its_rows.)"""
     _forced_rows(dt, H, I, rows, cf=cf, mode=mode)
 
 
@@ -359,3 +360,86 @@ def test_scheduler_statistics_count_tiles(dt, S, H, I, E, k, schedule):
     tiles = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
     (um, un), (dm, dn) = tiles["up"], tiles["down"]
     assert st["tiles"] == int((-(-kept // um)).sum()) * -(-I // un) + int((-(-kept // dm)).sum()) * -(-H // dn)
+
+
+def _assert_tiles(keys, want):
+    t = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
+    assert (t["variant"], t["down_small"]) == want, f"the layer runs on {t}: another layer is needed for these tiles"
+
+
+_ROWS_256 = [1, 15, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65, 100, 127, 128, 129, 192, 193, 255, 256, 257]
+_ROWS_128 = [1, 15, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65, 79, 81, 100, 127, 128, 129]
+_ROWS_64 = [1, 15, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65]
+
+
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("want,S,H,I,E,cf,edges", [
+    ((0, 0), 5120, 192, 448, 32, 3.0, _ROWS_256),       # 256 x 256, a last column tile of 192; experts of two row blocks
+    ((0, 0), 5120, 448, 192, 32, 4.0, _ROWS_256),
+    ((1, 0), 2048, 192, 704, 48, 4.0, _ROWS_128),       # 128 x 256
+    ((1, 0), 1536, 704, 64, 64, 4.0, _ROWS_64),
+    ((1, 1), 2048, 192, 2112, 48, 4.0, _ROWS_128),      # 128 x 256 up, 128 x 128 down
+    ((2, 0), 5120, 192, 192, 8, 4.0, [1, 129, 257, 700, 1024, 1025]),
+    ((2, 1), 5120, 192, 2048, 24, 3.0, _ROWS_256[-12:]),   # 256 x 256 up, 128 x 256 down
+    ((4, 0), 1024, 192, 320, 16, 4.0, [1, 63, 64, 65, 111, 112, 113, 127, 128, 129]),   # 128 x 128
+    ((4, 1), 2048, 192, 4160, 16, 4.0, [1, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 257]),   # 128 x 128 up, 64 x 128 down
+    ((5, 0), 1024, 192, 320, 48, 4.0, _ROWS_64),        # 64 x 128
+    ((6, 0), 128, 1088, 2112, 24, 6.0, [1, 15, 16, 17, 31, 33]),   # 64 x 128, weights non-temporal
+    ((6, 0), 128, 1088, 2112, 24, 24.0, [63, 65]),
+], ids=lambda v: v if isinstance(v, str) else (f"{v[0]}/{v[1]}" if isinstance(v, tuple) else str(len(v)) + "e" if isinstance(v, list) else str(v)))
+def test_every_pair_of_16_bit_tiles_at_the_edges_of_its_rows(mode, dt, want, S, H, I, E, cf, edges):
+    """Experts that end at and around the 16 rows of a matrix instruction, the 64 of a wavefront and the rows of a
+    tile, on the tiles that each row names, which the choice of the library is held to."""
+    keys = _keys(S, H, I, E, 1, cf=cf, act=1, dt=dt)
+    _assert_tiles(keys, want)
+    c = moe_ref.cfg_from_keys(keys)
+    share, rest = divmod(S - sum(edges), E - len(edges))
+    rows = edges + [share + 1] * rest + [share] * (E - len(edges) - rest)
+    assert max(rows) <= c.EC
+    _, v, _, _ = check_against_oracle(c, keys, _one_hot_layer(c, rows, seed=S + H), mode)
+    np.testing.assert_array_equal(v["expert_count"], np.array(rows))
+
+
+@pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("want,S,H,I", [((2, 0), 6272, 704, 704), ((2, 1), 4224, 1088, 1216), ((4, 0), 3072, 64, 704), ((4, 1), 1152, 64, 8192),
+                                        ((4, 1), 2176, 192, 4160), ((5, 0), 640, 320, 192)],
+                         ids=lambda v: v if isinstance(v, str) else (f"{v[0]}/{v[1]}" if isinstance(v, tuple) else str(v)))
+def test_dense_output_on_every_pair_of_tiles(dt, want, S, H, I):
+    """The dense output is stored with a pitch of H where the routed forward stores pieces one tile wide: the bits of a
+    routed forward on every pair of tiles that a single expert gets, with last row blocks and column tiles cut short."""
+    keys = _keys(S, H, I, 1, 1, act=1, dt=dt)
+    _assert_tiles(keys, want)
+    c = moe_ref.cfg_from_keys(keys)
+    x, wg, w_up, w_down, b_up, b_down = random_layer(c, seed=S + H, w_std=0.05, bias_std=0.1)
+    iP = pack_inputs(c, x, wg * 0, w_up, w_down, b_up, b_down)
+    dense = np.concatenate([iP[:S * H], iP[S * H + c.PX * H:]])
+    d = ka.initialize(keys)
+    try:
+        for schedule in (ka.SCHEDULE_DYNAMIC, ka.SCHEDULE_STATIC):
+            ka.moe.set_schedule(schedule)
+            oP = synth.alloc_outputs(d)
+            ka.moe.forward_host(_to_device(c, iP), oP)
+            ka.moe.stream_synchronize()
+            out = torch.empty(S * H, dtype=oP.dtype, device="cuda").fill_(float("nan"))
+            torch.cuda.synchronize()
+            ka.moe.forward_host_dense(_to_device(c, dense), out)
+            ka.moe.stream_synchronize()
+            np.testing.assert_array_equal(_out_to_np(c, out), _out_to_np(c, oP)[S * c.PX:])
+    finally:
+        ka.finalize()
+
+
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("E", [96, 200, 320])
+def test_tf32_large_tiles_with_many_experts(mode, E):
+    """256 x 256 tiles on the bf16 matrix cores with more than 64 experts: their workgroups of eight wavefronts hold two
+    gate units of four at a time, in each of the three gates above 64 experts."""
+    S, H, I = 16384, 128, 320
+    keys = _keys(S, H, I, E, 4, cf=2.0, dt=1)
+    _assert_tiles(keys, (3, 0))
+    c = moe_ref.cfg_from_keys(keys)
+    iP = pack_inputs(c, *random_layer(c, seed=E, w_std=0.08, bias_std=0.1))
+    mask = np.zeros(c.S, np.uint8)
+    mask[np.random.default_rng(E).choice(c.S, 600, replace=False)] = 1
+    check_against_oracle(c, keys, iP, mode, token_mask=mask)
