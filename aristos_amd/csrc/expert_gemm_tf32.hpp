@@ -8,8 +8,8 @@
 // Two kinds of operands do not split: an infinity, whose product with a remainder of zero is NaN, and a value below
 // 2^-123, whose remainder has bits below the last of a bf16 subnormal (2^-133). A wavefront that finds a NaN among its
 // sums, or sums so small that such lost bits could show in them, computes its part of the tile again on the fp32
-// matrix instructions. (Noticing the lost bits takes 18 of a slice's 373 vector instructions: 936 -> 944 us at the
-// layer below.)
+// matrix instructions. (Noticing the lost bits takes 17 of a slice's 364 vector instructions: 953 -> 959 us at the
+// layer below, the mean of two runs.)
 #pragma once
 #include "expert_gemm.hpp"
 
@@ -108,7 +108,10 @@ struct GemmSplit {
         t.b_base = g.b_base; t.ldb = g.ldb;
         t.c_base = g.c_base; t.ldc = g.ldc;
         t.m_valid = g.m_valid; t.n_valid = g.n_valid; t.k_tiles = g.K / kSliceK;
-        t.k_first = g.k_first < t.k_tiles ? g.k_first : 0u;
+        // Known to be scalar, it takes the slices' offsets off the vector unit: 364 instead of 381 vector instructions a
+        // slice, 32 registers spilled instead of 48. Against the tree that did not look for lost bits, in turn on one box,
+        // 981 -> 997 us per forward at the layer above without this, 949 -> 958 and 957 -> 959 with it.
+        t.k_first = __builtin_amdgcn_readfirstlane(g.k_first < t.k_tiles ? g.k_first : 0u);
         t.act = g.act; t.stage0 = stage0; t.bias_slot = bias_slot;
         const uint32_t k0 = first_value(t, 0), dst = stage_lds(t, smem, 0);
 #pragma unroll
