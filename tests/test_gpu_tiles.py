@@ -443,3 +443,15 @@ def test_tf32_large_tiles_with_many_experts(mode, E):
     mask = np.zeros(c.S, np.uint8)
     mask[np.random.default_rng(E).choice(c.S, 600, replace=False)] = 1
     check_against_oracle(c, keys, iP, mode, token_mask=mask)
+
+
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("E,H,cf", [(64, 64, 24.0), (300, 320, 96.0)])
+def test_queues_with_experts_without_rows(mode, E, H, cf):
+    """A workgroup looks for the segment of its next ticket from that of its last: queues whose experts hold no row in front
+    of, between and behind those that do, and whole queues of them, whose workgroups take tiles of the others."""
+    rows = [0] * E
+    for e, n in ((0, 300), (8, 1), (24, 257), (40, 129), (E - 3, 128), (3, 64), (E - 1, 401)):
+        rows[e] = n
+    assert sum(rows) % 128 == 0
+    _forced_rows(2, H, 576, rows, cf=cf, mode=mode)
