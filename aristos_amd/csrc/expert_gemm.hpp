@@ -976,7 +976,7 @@ struct GemmKSplit {
 // workgroups of four wavefronts on a CU, each in its own phase, cover each other's barriers.
 // Measured against the tile before it (slices of 16 values through registers, one at a time, one
 // workgroup on a CU): 1 024 tokens, 8 experts top-2, 1 024 x 4 096, fp32: 567 -> 347 us per forward, the
-// matrix cores busy 77 % of the time at 2.14 GHz; 8 192 tokens, 64 experts top-2, 2 048 x 2 048, tf32:
+// matrix cores busy 65 % of the whole launch at 2.3 GHz; 8 192 tokens, 64 experts top-2, 2 048 x 2 048, tf32:
 // 4 177 -> 2 729 us; 128 tokens, 8 experts, 256 x 512: 57 -> 44 us.
 // T: float, or tf32_t - then the operands lose their lower 13 mantissa bits on the way into the matrix
 // cores and the results are rounded to tf32 Elements.

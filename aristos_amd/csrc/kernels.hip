@@ -98,14 +98,14 @@ TileCost tile16_cost(uint32_t bm, uint32_t bn, uint32_t rows) {
 // The variants differ in how many rows and columns a tile has, so in how many rounds the CUs need for all of a
 // layer's tiles, and in the bytes and operations of a round. The estimate below, of both projections, decides:
 //   - an expert holds the rows of row_shares, so many row blocks on average;
-//   - a CU takes in about 47 KB a microsecond whatever it loads, a tile rows + columns of 2 bytes per value of K; 256 x 256
-//     tiles also come close to the matrix rate, 5.1 GFLOP a millisecond and CU;
+//   - a CU takes in about 47 KB a microsecond whatever it loads (fitted to times of all 16-bit variants), a tile rows +
+//     columns of 2 bytes per value of K; 256 x 256 tiles also come close to the matrix rate, 5.1 GFLOP a millisecond and CU;
 //   - a tile costs 5 us besides (look-ups, first slices, epilogue);
 //   - the weights pass at no more than 6.2 TB/s (tiles that share weights read them with the default policy, whose
 //     rate for weights read once is an eighth lower), and of two variants bound by that the one considered first is taken:
 //     the large tile, then as below.
 // Measured against every variant at 487 layers drawn between 128 and 15 616 tokens, 1 and 511 experts, with and without
-// dropping and skew: 3.2 % from the best of them in the mean, more than 10 % at 59 of them; 15 % faster in the mean than a
+// dropping and skew (profiles/tile_choice_16bit_layers.txt): 3.2 % from the best of them in the mean, more than 10 % at 59 of them; 15 % faster in the mean than a
 // choice by capacity alone (variant 1 up to 128 rows, 2 from 1 024, else 0), more than 3 % slower at seven (13 with
 // every expert at its mean). Where it moves a layer from the
 // 256- and 128-row tiles to the smaller ones: 640 tokens, 8 experts top-2, 704 x 512: 58 -> 37 us per forward; 2 176
@@ -148,9 +148,9 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     };
     // The smaller tile in the down-projection: a workgroup that goes over to it empties its pipeline once, and layers
     // bound by their weights gain nothing (256 tokens, 17 experts of 1 088 x 2 048: 59 -> 66 us without this allowance).
-    // Measured over 48 layers against the variants without it. 2 048 tokens, one expert, 1 024 x 4 096, dense: 71 -> 65
-    // us; 7 040 tokens, 768 x 2 240, dense: 110 -> 94; 640 tokens, 64 experts top-2, 448 x 2 816: 109 -> 97; 1 536
-    // tokens, one expert, 448 x 3 648: 62 -> 49.
+    // The best tiles without it against those with it, of the layers named above: 2 048 tokens, one expert, 1 024 x 4 096, dense:
+    // 67 -> 63 us; 6 400 tokens, 896 x 2 496, dense: 112 -> 100; 2 432 tokens, 11 experts top-3, 640 x 12 544: 472 -> 422;
+    // 1 024 tokens, 64 experts top-2, 320 x 9 216: 229 -> 218; 3 200 tokens, 320 x 14 144, dense: 215 -> 178.
     auto two_tiles = [&](uint32_t bm, uint32_t bn, uint32_t dm, uint32_t dn, bool streams) { return 1.06 * estimate(bm, bn, dm, dn, streams) + 5.0; };
     double us = 1e30;
     auto consider = [&](uint32_t variant, uint32_t small, double estimated) {
