@@ -1,4 +1,5 @@
-// Expert projections of the tf32 Element on the bf16 matrix cores.
+// Expert projections of the tf32 Element on the 16-bit matrix cores: GemmHalf, one fp16 product per pair of operands, and
+// GemmSplit, four bf16 products, for the tiles whose operands do not fit fp16.
 //
 // A tf32 operand has 11 significant bits. Its upper 8 are a bf16 value (the upper half of the word) and
 // the remainder, at most 3 bits, is exactly one too: v = hi + lo. A product of two operands is then the sum
@@ -14,6 +15,12 @@
 #include "expert_gemm.hpp"
 
 namespace kleos_amd {
+
+// Where a tile's results go.
+struct TileOut32 {
+    float* c_base;
+    uint32_t ldc, m_valid, n_valid;
+};
 
 // ------------------------------------------------------------------------------------------------
 // BM x BN tile, WAVES_M x WAVES_N wavefronts, K in slices of 32 values (128-byte rows) through two LDS
@@ -181,7 +188,8 @@ struct GemmSplit {
         return stage + 1024 * (threadIdx.x >> 6) + (i < LB ? kABytes + 1024 * kWaves * i : 1024 * kWaves * (i - LB));
     }
 
-    static __device__ __forceinline__ bool rows_absent(const Tile& t, int wm) { return uint32_t(wm * WM) >= t.m_valid; }
+    static __device__ __forceinline__ bool rows_absent_of(uint32_t m_valid, int wm) { return uint32_t(wm * WM) >= m_valid; }
+    static __device__ __forceinline__ bool rows_absent(const Tile& t, int wm) { return rows_absent_of(t.m_valid, wm); }
 
     template <typename Hook>
     static __device__ __forceinline__ void mainloop(const Tile& t, Acc& acc, char* smem, Hook&& after_first_barrier) {
@@ -326,7 +334,7 @@ struct GemmSplit {
     }
 
     // Bias, activation, rounding to tf32, rows written through the L2 in whole lines: panels of 32 rows x 32
-    // columns go through 4 KB of the wavefront's own in the stage of the last slice.
+    // columns go through 4 KB of the wavefront's own of `stage`.
     static __device__ __forceinline__ void finish(const Tile& t, Acc& acc, char* smem) {
         float largest = 0.f;
         const bool lost = *lost_word(smem, t.bias_slot) != 0u;   // the same in every wavefront
@@ -340,10 +348,13 @@ struct GemmSplit {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) nan |= acc[ni][mi][j] != acc[ni][mi][j];
         if (lost) nan |= small_sums(t, acc, largest);
+        const TileOut32 out{t.c_base, t.ldc, t.m_valid, t.n_valid};
+        const char* bias = smem + kBiasOffset + t.bias_slot * kBiasBytes;
+        char* stage = smem + last_stage(t) * kStage;
         if (__builtin_amdgcn_ballot_w64(nan) != 0u) recompute(t, smem);
-        else if (t.act == 0) finish_act<0>(t, acc, smem);
-        else if (t.act == 1) finish_act<1>(t, acc, smem);
-        else finish_act<2>(t, acc, smem);
+        else if (t.act == 0) finish_act<0>(out, acc, bias, stage);
+        else if (t.act == 1) finish_act<1>(out, acc, bias, stage);
+        else finish_act<2>(out, acc, bias, stage);
     }
     // The largest operand of the tile, from the rows in memory: every thread looks at what it loaded for the main loop, the
     // stage that the last slice is not in takes the results. Called by all wavefronts or none.
@@ -453,13 +464,13 @@ struct GemmSplit {
         }
     }
     template <int ACT>
-    static __device__ __forceinline__ void finish_act(const Tile& t, Acc& acc, char* smem) {
+    static __device__ __forceinline__ void finish_act(const TileOut32& t, Acc& acc, const char* bias_mem, char* stage) {
         const uint32_t tid = local_tid();
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
         const int wm = wave / WAVES_N, wn = wave % WAVES_N;
         const int fr_row = lane & 15, fr_part = lane >> 4;
-        char* stg = smem + last_stage(t) * kStage + wave * 4096;
-        const char* bias = smem + kBiasOffset + t.bias_slot * kBiasBytes + (wn * WN + 4 * fr_part) * 4;
+        char* stg = stage + wave * 4096;
+        const char* bias = bias_mem + (wn * WN + 4 * fr_part) * 4;
 #pragma unroll
         for (int pm = 0; pm < TM / 2; ++pm)
 #pragma unroll
@@ -485,6 +496,426 @@ struct GemmSplit {
                         __builtin_amdgcn_raw_buffer_store_b128(v, coherent_rows(t.c_base), int((size_t(m) * t.ldc + n) * 4), 0, kAgentScope);
                 }
             }
+    }
+};
+
+// ------------------------------------------------------------------------------------------------
+// The same tile with one fp16 product instead of four bf16 ones. An fp16 value holds the 11 significant bits of a tf32
+// operand; what it lacks is range. Every row of the tile is therefore scaled by a power of two of its own, chosen from the
+// row's values in the tile's first slice (their largest goes to 2^9 .. 2^10, so that the row may hold values 64 times as
+// large and keeps all bits of those down to 2^-24 of it), and the epilogue scales the sums back: scaling is exact, a
+// truncating conversion to fp16 cuts a value to what the tf32 instructions read of it, a product of two such values is exact
+// in fp32. What does not fit is noticed, and the whole tile then computed by GemmSplit:
+//   - a value that overflows, an infinity, a row whose first slice lies outside 2^-40 .. 2^40;
+//   - a value below 2^-14 once scaled, which may lose bits below 2^-24. One in some ten million of a random operand does,
+//     and no sum shows it: the tile is kept if all K products of a row (column) together could not lose more than
+//     2^-22 of the largest sum of that row (column), a fraction of what rounding the sums in fp32 loses.
+// (A NaN needs no care: it makes the same sums NaN.)
+//
+// K in slices of 32 values (128-byte rows). Four wavefronts bring the weight rows of a slice, four the activation rows, as
+// direct loads into rings of LDS of their own: two slices for weights, which come from memory, one for activations, which the
+// column tiles of an expert share in the L2 (vmcnt counts loads in order: a wavefront that brought both would wait for the weights
+// in front of its activations). A wavefront converts what it brought, eight rows at a time, from its ring into the one
+// slice that is multiplied; a ring slot is requested anew as soon as it has been read, without a barrier. The twelve
+// fragments of a slice fit the registers beside the accumulators, so that the converted slice is free early. Per slice kt:
+//   top       the workgroup meets: slice kt is converted
+//   group 0   all fragments of slice kt are read; behind a second barrier the converted slice may change
+//   group i   four matrix instructions of slice kt, between the request for eight rows of slice kt+1 and their conversion
+//
+// What bounds it: the weights, which have 64 KB a CU in flight (with all weight tiles read from one place, 460 us of 553), then the
+// LDS, through which a slice passes four times, 256 KB (450 us with the activations resident in L2 as well, 360 without the matrix
+// instructions). Measured, expert phase at 8 192 tokens, 64 experts top-2, 2 048 x 2 048: GemmSplit 890 us, this 553 (970 -> 640 us per
+// forward). On the way: both operands in one ring of 12 kilobytes a wavefront, the kernel still spilling, 640; raw rows converted in place
+// in two stages 737; loads to registers one slice ahead 761.
+// ------------------------------------------------------------------------------------------------
+template <int BM, int BN, int WAVES_M, int WAVES_N>
+struct GemmHalf {
+    static __device__ __forceinline__ uint32_t scalar(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); }
+    template <typename P>
+    static __device__ __forceinline__ P* scalar(P* p) {
+        const uint64_t a = reinterpret_cast<uint64_t>(p);
+        return reinterpret_cast<P*>((uint64_t(scalar(uint32_t(a >> 32))) << 32) | scalar(uint32_t(a)));
+    }
+    // A tile's arguments in scalar registers: they live through the main loop.
+    static __device__ __forceinline__ GemmTileArgs<float> scalar(const GemmTileArgs<float>& g) {
+        GemmTileArgs<float> s;
+        s.a_base = scalar(g.a_base); s.a_row_index = scalar(g.a_row_index); s.a_rows = scalar(g.a_rows); s.a_pad = scalar(g.a_pad);
+        s.b_base = scalar(g.b_base); s.bias = scalar(g.bias); s.c_base = scalar(g.c_base);
+        s.lda = scalar(g.lda); s.ldb = scalar(g.ldb); s.ldc = scalar(g.ldc); s.K = scalar(g.K); s.k_first = scalar(g.k_first);
+        s.m_valid = scalar(g.m_valid); s.n_valid = scalar(g.n_valid); s.act = scalar(g.act);
+        return s;
+    }
+    typedef GemmSplit<BM, BN, WAVES_M, WAVES_N> Split;
+    static constexpr int kWaves = Split::kWaves, kThreads = Split::kThreads, kSliceK = Split::kSliceK;
+    static constexpr int WM = Split::WM, WN = Split::WN, TM = Split::TM, TN = Split::TN, kRowsPerLoad = Split::kRowsPerLoad;
+    static constexpr int kLoaders = kWaves / 2;                          // wavefronts that bring the rows of one operand
+    static constexpr int L = BM / (kRowsPerLoad * kLoaders);             // kilobytes of a slice a wavefront brings
+    static_assert(BM == BN && L == TM, "the groups below are counted for these");
+    // LDS: the converted slice [BM rows | BN rows] of 64 bytes, then the rings that the loads land in: kRingX kilobytes for every wavefront
+    // that brings activations, kRingW for the others
+    static constexpr int kRowBytes = kSliceK * 2, kABytes = BM * kRowBytes, kConverted = (BM + BN) * kRowBytes;
+    static constexpr int kRingX = L, kRingW = 2 * L;
+    static constexpr int kRings = kLoaders * (kRingX + kRingW) * 1024;
+    static constexpr int kExponents = Split::kSmemBytes;                 // powers of two that scale a sum back: int32 [BM rows | BN columns]
+    static constexpr int kRangeOffset = kExponents + (BM + BN) * 4;      // per bias slot: the Range words
+    static constexpr int kRangeWords = 4;
+    static constexpr int kSmemBytes = kRangeOffset + 2 * kRangeWords * 4;
+    static_assert(kConverted + kRings <= 2 * Split::kStage && kWaves * 4096 <= kConverted);
+    typedef typename Split::Acc Acc;
+    struct Tile {
+        GemmTileArgs<float> g;
+        const float* rows[L];      // this lane's rows of the operand its wavefront brings, at its chunk of a slice
+        uint32_t k_tiles;
+        int bias_slot;
+    };
+
+    // words of a tile's range: largest scaled activation and weight (bits of a float), what the tile holds that calls for a second look
+    enum : uint32_t { kLargestX = 0, kLargestW = 1, kSeen = 2 };
+    enum : uint32_t { kOutOfRange = 1, kSmallX = 2, kSmallW = 4 };
+    static __device__ __forceinline__ uint32_t* range_words(char* smem, int bias_slot) {
+        return reinterpret_cast<uint32_t*>(smem + kRangeOffset) + bias_slot * kRangeWords;
+    }
+
+    static __device__ __forceinline__ int next_stage0(const Tile&) { return 0; }
+    static __device__ __forceinline__ uint32_t first_value(const Tile& t, uint32_t kt) {
+        const uint32_t slice = kt + t.g.k_first;
+        return (slice >= t.k_tiles ? slice - t.k_tiles : slice) * kSliceK;
+    }
+    // Odd wavefronts bring weight rows, even ones activation rows.
+    static __device__ __forceinline__ uint32_t brings_w() { return wave_index() & 1u; }
+    static __device__ __forceinline__ uint32_t loader() { return wave_index() >> 1; }
+    static __device__ __forceinline__ uint32_t ring_offset() { return kConverted + 1024 * (brings_w() ? kLoaders * kRingX + loader() * kRingW : loader() * kRingX); }
+    // A direct load with the policy of the wavefront's operand (non-temporal for weights), and the wait for all but W or X of a
+    // wavefront's loads. One statement each, so that the compiler sees no branch between the matrix instructions.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    static __device__ __forceinline__ void load(const float* src, uint32_t lds, uint32_t w) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_cmp_lg_u32 %2, 0\n\ts_cbranch_scc1 1f\n\tglobal_load_lds_dwordx4 %1, off\n\ts_branch 2f\n"
+                     "1:\n\tglobal_load_lds_dwordx4 %1, off nt\n2:" ::"s"(lds), "v"(src), "s"(w) : "memory", "m0", "scc");
+    }
+#pragma clang diagnostic pop
+    template <int X, int W>
+    static __device__ __forceinline__ void wait(uint32_t w) {
+        if constexpr (X == W) {
+            wait_vmcnt<X>();
+            asm volatile("" ::: "memory");
+        } else {
+            asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 1f\n\ts_waitcnt vmcnt(%1)\n1:\n\ts_waitcnt vmcnt(%2)" ::"s"(w), "i"(X), "i"(W) : "memory", "scc");
+            static_assert(W > X);
+        }
+    }
+    // As Gemm16::begin; requests as many slices as the wavefront's ring holds.
+    static __device__ __forceinline__ void begin(Tile& t, const GemmTileArgs<float>& args, int, int bias_slot, char* smem) {
+        const GemmTileArgs<float> g = scalar(args);
+        const uint32_t tid = local_tid();
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+        const int ld_r = lane >> 3, ld_c = lane & 7;
+        if (wave == 0 && lane < Split::kBiasBytes / 16) {
+            const uint32_t n = uint32_t(lane) * 4 < g.n_valid ? uint32_t(lane) * 4 : 0u;
+            direct_load16<false>(g.bias + n, lds_address(smem) + Split::kBiasOffset + bias_slot * Split::kBiasBytes);
+        }
+        // (last read by the epilogue of the tile before the previous one, written again behind the main loop's barriers)
+        if (tid < uint32_t(kRangeWords)) range_words(smem, bias_slot)[tid] = 0u;
+        t.g = g;
+        t.k_tiles = g.K / kSliceK;
+        t.g.k_first = g.k_first < t.k_tiles ? g.k_first : 0u;
+        t.bias_slot = bias_slot;
+        const bool w = wave & 1;
+        const int valid = w ? g.n_valid : g.m_valid;
+        uint32_t src[L];
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int row = kRowsPerLoad * ((wave >> 1) + kLoaders * i) + ld_r;
+            src[i] = row < valid ? row : valid - 1;
+        }
+        if (!w && g.a_row_index) {
+#pragma unroll
+            for (int i = 0; i < L; ++i) src[i] = uint32_t(load_coherent(g.a_row_index + src[i]));
+#pragma unroll
+            for (int i = 0; i < L; ++i) src[i] = src[i] < g.a_rows ? src[i] : g.a_rows - 1;
+        }
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int row = kRowsPerLoad * ((wave >> 1) + kLoaders * i) + ld_r;
+            const float* from = w ? g.b_base + size_t(src[i]) * g.ldb : g.a_base + size_t(src[i]) * g.lda;
+            if (!w && g.a_pad && row >= valid) from = g.a_pad;
+            t.rows[i] = from + 4 * ld_c;
+        }
+        const uint32_t ring = lds_address(smem) + ring_offset();
+#pragma unroll
+        for (int i = 0; i < L; ++i) load(t.rows[i] + first_value(t, 0), ring + 1024 * i, brings_w());
+        if (w && t.k_tiles > 1) {
+#pragma unroll
+            for (int i = 0; i < L; ++i) load(t.rows[i] + first_value(t, 1), ring + 1024 * (L + i), brings_w());
+        }
+    }
+
+    // ---- the conversion of a kilobyte
+    static __device__ __forceinline__ int swizzle(int r) { return (r >> 2) & 3; }
+    // Where the lane's four values go inside the 512 bytes that a kilobyte becomes.
+    static __device__ __forceinline__ uint32_t half_offset() {
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        const int r = lane >> 3, c = lane & 7;      // (the kilobytes of a wavefront are kLoaders * kRowsPerLoad rows apart: one swizzle)
+        return uint32_t(r * kRowBytes + (((c >> 1) ^ swizzle(kRowsPerLoad * (wave >> 1) + r)) << 4) + (c & 1) * 8);
+    }
+    // What a thread has seen of the scaled values: the largest, and the least that is not zero (2 * bits - 1, zero wraps to the top).
+    struct Seen { float largest = 0.f; uint32_t least = ~0u; };
+    static constexpr uint32_t kLeast = (0x38800000u << 1) - 1u;          // 2^-14, the least normal fp16 value
+    static __device__ __forceinline__ void convert(char* to, u32x4 raw, float scale, Seen& seen) {
+        float v[4];
+        uint32_t u[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t word = raw[j];
+            v[j] = __builtin_bit_cast(float, word) * scale;
+            u[j] = (__builtin_bit_cast(uint32_t, v[j]) << 1) - 1u;
+        }
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(seen.largest) : "v"(v[0]), "v"(v[1]));
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(seen.largest) : "v"(v[2]), "v"(v[3]));
+        const uint32_t a = u[0] < u[1] ? u[0] : u[1], b = u[2] < u[3] ? u[2] : u[3], c = a < b ? a : b;
+        seen.least = c < seen.least ? c : seen.least;
+        const u32x2 half{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(v[0], v[1])), __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(v[2], v[3]))};
+        *reinterpret_cast<u32x2*>(to) = half;
+    }
+    // The scale of the row whose values of the first slice lie in this lane and the seven beside it.
+    static __device__ __forceinline__ int row_exponent(u32x4 raw, uint32_t& seen) {
+        uint32_t largest = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t word = raw[j] & 0x7fffffffu;
+            largest = word > largest ? word : largest;
+        }
+        auto with = [&](uint32_t peer) { largest = peer > largest ? peer : largest; };
+        with(row16_peer<0>(largest));
+        with(row16_peer<1>(largest));
+        with(row16_peer<2>(largest));   // (the three steps combine aligned groups of eight lanes)
+        const int e = int(largest >> 23) - 127;
+        if (largest == 0u) return 0;
+        if (e < -40 || e > 40) { seen = kOutOfRange; return 0; }
+        return 9 - e;
+    }
+
+    template <typename Hook>
+    static __device__ __forceinline__ void mainloop(const Tile& t, Acc& acc, char* smem, Hook&& after_first_barrier) {
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+        Seen seen;
+        float scale[L];
+        uint32_t flags = 0u;
+        const uint32_t w = brings_w(), ring = lds_address(smem) + ring_offset();
+        const char* const ring_lane = smem + ring_offset() + 16 * lane;
+        char* const to = smem + (w ? kABytes : 0) + 512 * loader() + half_offset();
+        // Slice kt of the ring's slots: an activation slice takes the one place there is, a weight slice the place kt % 2.
+        auto place = [&](uint32_t kt) { return (kt & w) * (L * 1024u); };
+        // How far the loads have got when slice s is converted. Kilobyte i of it makes way for that of the slice one (activations) or two
+        // (weights) later. kBoth: slice s+2 exists; kOne: s+1 does; kNone: s is the last.
+        enum { kBoth, kOne, kNone };
+        u32x4 raw[2];   // kilobyte i of the slice being converted, and the one behind it
+        auto request = [&](auto stage_tag, auto i_tag, uint32_t s) {
+            constexpr int S = decltype(stage_tag)::value, i = decltype(i_tag)::value;
+            if constexpr (S == kBoth) wait<kRingX - 1, kRingW - 1>(w);
+            else if constexpr (S == kOne) wait<kRingX - 1, (kRingW - 1 - i > kRingX - 1 ? kRingW - 1 - i : kRingX - 1)>(w);
+            else wait<L - 1 - i, L - 1 - i>(w);
+            raw[i & 1] = load16(ring_lane + place(s) + 1024 * i);
+        };
+        // The kilobyte's values are in registers: its slot takes the later one.
+        auto reload = [&](auto stage_tag, auto i_tag, uint32_t s) {
+            constexpr int S = decltype(stage_tag)::value, i = decltype(i_tag)::value;
+            asm volatile("" : "+v"(raw[i & 1]));
+            if constexpr (S == kBoth) load(t.rows[i] + first_value(t, s + 1 + w), ring + place(s) + 1024 * i, w);
+            else if constexpr (S == kOne) { if (!w) load(t.rows[i] + first_value(t, s + 1), ring + 1024 * i, 0u); }
+        };
+        // Kilobytes 0 .. L-1 of slice s, the first of them requested: `between(i)` runs while number i + 1 is on its way.
+        auto convert_slice = [&](auto stage_tag, uint32_t s, auto&& between, auto&& first) {
+            static_for<L>([&](auto i_tag) {
+                constexpr int i = decltype(i_tag)::value;
+                reload(stage_tag, i_tag, s);
+                if constexpr (i + 1 < L) request(stage_tag, std::integral_constant<int, (i + 1 < L ? i + 1 : 0)>{}, s);
+                between(i);
+                first(i_tag);
+                convert(to + 512 * kLoaders * i, raw[i & 1], scale[i], seen);
+            });
+        };
+        auto stages = [&](uint32_t s, auto&& f) {
+            if (s + 2 < t.k_tiles) f(std::integral_constant<int, kBoth>{});
+            else if (s + 1 < t.k_tiles) f(std::integral_constant<int, kOne>{});
+            else f(std::integral_constant<int, kNone>{});
+        };
+        using First = std::integral_constant<int, 0>;
+        // every wavefront has left the previous tile's epilogue, staged where the converted rows go
+        asm volatile("s_barrier" ::: "memory");
+        stages(0, [&](auto stage_tag) {
+            request(stage_tag, First{}, 0u);
+            convert_slice(stage_tag, 0u, [](int) {}, [&](auto i_tag) {
+                constexpr int i = decltype(i_tag)::value;
+                const int e = row_exponent(raw[i & 1], flags);
+                scale[i] = __builtin_bit_cast(float, uint32_t(e + 127) << 23);
+                const int row = kRowsPerLoad * (int(loader()) + kLoaders * i) + (lane >> 3);
+                if ((lane & 7) == 0) reinterpret_cast<int*>(smem + kExponents)[(w ? BM : 0) + row] = -e;
+            });
+        });
+        auto top = [&](uint32_t kt) {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (kt == 0) after_first_barrier();
+        };
+        auto report = [&] {
+            if (seen.least < kLeast) flags |= w ? kSmallW : kSmallX;
+            if (seen.largest >= 65536.f) flags |= kOutOfRange;
+            uint32_t* words = range_words(smem, t.bias_slot);
+            atomicMax(words + (w ? kLargestW : kLargestX), __builtin_bit_cast(uint32_t, seen.largest));
+            if (flags) atomicOr(words + kSeen, flags);
+        };
+        auto nothing = [](auto) {};
+        if (Split::rows_absent_of(t.g.m_valid, __builtin_amdgcn_readfirstlane(wave) / WAVES_N)) {
+            // None of this wavefront's rows exist: it brings and converts its share of every slice between
+            // the same barriers, and multiplies nothing.
+            for (uint32_t kt = 0; kt < t.k_tiles; ++kt) {
+                top(kt);
+                if (kt + 1 < t.k_tiles) {
+                    asm volatile("s_barrier" ::: "memory");
+                    stages(kt + 1, [&](auto stage_tag) {
+                        request(stage_tag, First{}, kt + 1);
+                        convert_slice(stage_tag, kt + 1, [](int) {}, nothing);
+                    });
+                }
+            }
+            report();
+            return;
+        }
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+            for (int mi = 0; mi < TM; ++mi) acc[ni][mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int fr_row = lane & 15, fr_part = lane >> 4;
+        const int rx = wm * WM + fr_row, rw = wn * WN + fr_row;
+        const char* const from_x = smem + rx * kRowBytes + ((fr_part ^ swizzle(rx)) << 4);
+        const char* const from_w = smem + kABytes + rw * kRowBytes + ((fr_part ^ swizzle(rw)) << 4);
+        auto slice = [&](uint32_t kt, auto next_tag, auto stage_tag) {
+            constexpr bool NEXT = decltype(next_tag)::value;
+            top(kt);
+            f16x8 fw[TN], fx[TM];
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni) fw[ni] = __builtin_bit_cast(f16x8, load16(from_w + ni * 16 * kRowBytes));
+#pragma unroll
+            for (int mi = 0; mi < TM; ++mi) fx[mi] = __builtin_bit_cast(f16x8, load16(from_x + mi * 16 * kRowBytes));
+            __builtin_amdgcn_sched_barrier(0);
+            auto group = [&](int o) {
+#pragma unroll
+                for (int ni = 0; ni < TN; ++ni) acc[ni][o] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[ni], fx[o], acc[ni][o], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            if constexpr (NEXT) {
+                // Behind a barrier in front of the first conversion every wavefront has its fragments of slice kt in registers.
+                request(stage_tag, First{}, kt + 1);
+                group(0);
+                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+                asm volatile("s_barrier" ::: "memory");
+                convert_slice(stage_tag, kt + 1, [&](int i) { if (i + 1 < TM) group(i + 1); }, nothing);
+            } else {
+#pragma unroll
+                for (int o = 0; o < TM; ++o) group(o);
+            }
+        };
+        using Both = std::integral_constant<int, kBoth>; using One = std::integral_constant<int, kOne>; using None = std::integral_constant<int, kNone>;
+        const uint32_t both = t.k_tiles >= 3 ? t.k_tiles - 3 : 0u;
+        for (uint32_t kt = 0; kt < both; ++kt) slice(kt, std::true_type{}, Both{});
+        if (t.k_tiles >= 3) slice(t.k_tiles - 3, std::true_type{}, One{});
+        if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::true_type{}, None{});
+        slice(t.k_tiles - 1, std::false_type{}, None{});
+        report();
+    }
+
+    // Whether the bits that values below 2^-14 may have lost stay under the rounding of this wavefront's sums.
+    static __device__ __forceinline__ bool losses_hidden(const Tile& t, const Acc& acc, const uint32_t* words, uint32_t flags) {
+        const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+        // a sum loses less than K 2^-24 times the largest partner; 2^-22 of the largest sum of its row or column
+        const float count = float(t.k_tiles * kSliceK) * 0.25f;
+        const float least_row = count * __builtin_bit_cast(float, words[kLargestW]), least_col = count * __builtin_bit_cast(float, words[kLargestX]);
+        bool hidden = true;
+        float col[TN][4];
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) col[ni][j] = 0.f;
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) {
+            const bool exists = uint32_t((wave / WAVES_N) * WM + mi * 16 + (lane & 15)) < t.g.m_valid;
+            float row = 0.f;
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float v = __builtin_fabsf(acc[ni][mi][j]);
+                    row = __builtin_fmaxf(row, v);
+                    col[ni][j] = exists ? __builtin_fmaxf(col[ni][j], v) : col[ni][j];
+                }
+            row = __builtin_fmaxf(row, __shfl_xor(row, 16));
+            row = __builtin_fmaxf(row, __shfl_xor(row, 32));
+            if ((flags & kSmallX) && exists && !(row >= least_row)) hidden = false;
+        }
+        if (flags & kSmallW) {
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (!(row16_allreduce(col[ni][j], [](float a, float b) { return __builtin_fmaxf(a, b); }) >= least_col)) hidden = false;
+        }
+        return hidden;
+    }
+
+    // The tile by GemmSplit. A function of its own: its registers are not those of the main loop's tile.
+    static __device__ __attribute__((noinline)) void again(GemmTileArgs<float> args, uint32_t slot, uint32_t lds) {
+        const GemmTileArgs<float> g = scalar(args);
+        const int bias_slot = int(scalar(slot));
+        char* smem = (char*)(__attribute__((address_space(3))) char*)uintptr_t(scalar(lds));
+        typename Split::Tile t;
+        Acc acc;
+        Split::begin(t, g, 0, bias_slot, smem);
+        Split::mainloop(t, acc, smem, [] {});
+        __syncthreads();
+        Split::finish(t, acc, smem);
+        __syncthreads();   // the next tile's loads land where the other wavefronts stage their rows
+    }
+    static __device__ __forceinline__ void finish(const Tile& t, Acc& acc, char* smem) {
+        uint32_t* words = range_words(smem, t.bias_slot);
+        uint32_t seen = __builtin_amdgcn_readfirstlane(words[kSeen]);   // the same in every wavefront
+        const bool absent = Split::rows_absent_of(t.g.m_valid, __builtin_amdgcn_readfirstlane(int(local_tid() >> 6)) / WAVES_N);
+        if (seen != 0u && !(seen & kOutOfRange)) {
+            __syncthreads();   // everybody has read the word
+            if (!absent && !losses_hidden(t, acc, words, seen)) atomicOr(words + kSeen, uint32_t(kOutOfRange));
+            __syncthreads();
+            seen = __builtin_amdgcn_readfirstlane(words[kSeen]);
+        }
+        if (seen & kOutOfRange) {
+            again(t.g, t.bias_slot, uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)));
+            return;
+        }
+        if (absent) return;
+        if (t.g.act == 0) finish_act<0>(t, acc, smem);
+        else if (t.g.act == 1) finish_act<1>(t, acc, smem);
+        else finish_act<2>(t, acc, smem);
+    }
+    template <int ACT>
+    static __device__ __forceinline__ void finish_act(const Tile& t, Acc& acc, char* smem) {
+        const uint32_t tid = local_tid();
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+        const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+        const int* exponents = reinterpret_cast<const int*>(smem + kExponents);
+        u32x4 col[TN];
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni) col[ni] = load16(exponents + BM + wn * WN + ni * 16 + 4 * (lane >> 4));
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) {
+            const int row = exponents[wm * WM + mi * 16 + (lane & 15)];
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t c = col[ni][j];
+                    acc[ni][mi][j] = __builtin_amdgcn_ldexpf(acc[ni][mi][j], row + int(c));
+                }
+        }
+        Split::template finish_act<ACT>(TileOut32{t.g.c_base, t.g.ldc, t.g.m_valid, t.g.n_valid}, acc, smem + Split::kBiasOffset + t.bias_slot * Split::kBiasBytes, smem);
     }
 };
 

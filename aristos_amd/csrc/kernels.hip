@@ -110,9 +110,9 @@ TileCost tile16_cost(uint32_t bm, uint32_t bn, uint32_t rows) {
 // every expert at its mean). Where it moves a layer from the
 // 256- and 128-row tiles to the smaller ones: 640 tokens, 8 experts top-2, 704 x 512: 58 -> 37 us per forward; 2 176
 // tokens, 16 experts top-2, 2 048 x 512: 91 -> 75; 2 048 tokens, one expert, 1 024 x 4 096: 148 -> 108.
-// tf32: 256 x 256 tiles on the bf16 matrix cores, 128 clocks per value of K, one on a CU, against 64 x 64 tiles on
+// tf32: 256 x 256 tiles on the 16-bit matrix cores, 128 clocks per value of K, one on a CU, against 64 x 64 tiles on
 // the fp32 ones, 32 clocks, two on a CU in turn (8 192 tokens, 64 experts top-2, 2 048 x 2 048: 512 : 2 048 by this
-// rule, 975 : 2 729 us measured).
+// rule, 640 : 2 729 us measured).
 void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     const uint32_t cap = p.EC < p.cap_rows ? p.EC : p.cap_rows;
     const uint32_t rows = mean_rows(p);

@@ -302,6 +302,57 @@ def test_tf32_operands_below_what_splits_exactly(where, exponent):
         assert float((got - want)[part].norm()) <= (2.0 ** -11 + 1e-5) * float(want[part].norm())
 
 
+@pytest.mark.parametrize("operand", ["x", "w_up"])
+@pytest.mark.parametrize("rows", ["of any scale", "growing", "starting with zeros", "shrinking", "of small values that show", "out of range"])
+def test_tf32_rows_that_fit_fp16_and_rows_that_do_not(rows, operand):
+    """The 256 x 256 tf32 tile scales every row by its first 32 values and multiplies in fp16. Rows of any scale fit; values far
+    larger than the first ones, or so small beside them that fp16 cuts them, on their own or where the partners of the large ones
+    are zero, and rows beyond 2^40 have to give what undivided products give, each row (column) to its own scale."""
+    S, H, I = 16384, 512, 512
+    rng = np.random.default_rng(13)
+
+    def values(*n):   # 11 significant bits, 1 <= |v| < 2
+        return torch.from_numpy(rng.integers(1024, 2048, n) * rng.choice([-1.0, 1.0], n) / 1024)
+    x, w_up, w_down = values(S, H), values(I, H), values(H, I) / 16
+    a, b = (x, w_up) if operand == "x" else (w_up, x)
+    n = a.shape[0]
+    some = torch.from_numpy(rng.choice(n, n // 3, replace=False))
+    if rows == "of any scale":
+        a *= 2.0 ** torch.from_numpy(rng.integers(-30, 31, (n, 1))).double()
+    elif rows == "growing":
+        a[some, 100:] *= 2.0 ** 12
+    elif rows == "starting with zeros":
+        a[some, :300] = 0.0
+        a[some[:100]] = 0.0
+    elif rows == "shrinking":
+        a[some, 40:] *= 2.0 ** -30
+    elif rows == "of small values that show":
+        a[some, 40:] *= 2.0 ** -30
+        b[:, :40] = 0.0
+    else:
+        a[some] *= 2.0 ** 50
+    h = torch.relu(x @ w_up.T)
+    scale = h.norm(dim=0)
+    if operand == "w_up":   # every column of h counts as much as the others, whatever its scale
+        w_down *= torch.where(scale > 0, 2.0 ** -torch.floor(torch.log2(scale.clamp_min(1e-300))), torch.ones(()).double())
+    want = h @ w_down.T
+    iP = torch.cat([x.flatten(), w_up.flatten(), w_down.flatten(), torch.zeros(H + I).double()]).float().cuda()
+    keys = _keys(S, H, I, 1, 1, act=0, dt=1)
+    _assert_tiles(keys, (3, 0))
+    ka.initialize(keys)
+    try:
+        oP = torch.zeros(S * H, device="cuda")
+        ka.moe.forward_host_dense(iP, oP)
+        ka.moe.stream_synchronize()
+        got = oP.view(S, H).cpu().double()
+    finally:
+        ka.finalize()
+    ok = want.norm(dim=1) > 0
+    assert torch.equal(got[~ok], want[~ok])
+    # h is rounded to 11 bits on the way, 2^-11 of each of its values at most, and the output once more
+    assert float(((got - want).norm(dim=1)[ok] / want.norm(dim=1)[ok]).max()) <= 2 * 2.0 ** -11
+
+
 @pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
 @pytest.mark.parametrize("low,high", [(0.001, 0.1), (0.1, 0.5), (0.5, 1.0), (1.0, 2.0)])
 def test_gelu_keeps_the_bits_of_small_arguments(low, high, sign):
