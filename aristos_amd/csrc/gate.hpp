@@ -45,156 +45,14 @@ constexpr bool gate_unit_grouped(int kw) { return NG >= 1 && NG <= 4 && kw % 4 =
 // writes, so that the reads, which walk the rows four at a time, spread over all banks.
 constexpr int kGateParkStride = kWave + 1;
 // LDS floats needed by gate_unit with KW wavefronts: the partial accumulators (4*NG registers of
-// 64 lanes) of the KW shares of the hidden dimension of the block being reduced; in the grouped
-// epilogue those of both blocks, in padded rows, and the scratch of the groups.
+// 64 lanes) of the KW shares of the hidden dimension of the block being reduced, in padded rows (its epilogue's scratch
+// takes their place, 33 words an expert at most); up to 64 experts those of both blocks, and the scratch of the groups.
 template <int NG>
 constexpr int gate_smem_floats(int kw) {
     if (gate_unit_grouped<NG>(kw)) return 2 * kw * NG * 4 * kGateParkStride + (kw / 4) * int(kGateTileTokens * 64 + 64 + kGateTileTokens * 64);
-    return kw * (NG == 0 ? 16 : NG) * 4 * kWave;
+    return kw * (NG == 0 ? 16 * kWave : NG * kGateParkStride) * 4;
 }
 constexpr uint32_t kWideGateMaxK = 32;   // the wide gate keeps a tile's 16 * k picks in LDS
-
-// Softmax, top-k, outputs and the tile histogram of one 16-token tile, run by one wavefront that
-// holds the complete logits of the tile: acc[g][v] of lane l is expert 16 g + 4 (l / 16) + v of
-// token l % 16.
-template <typename T, int NG>
-__device__ __forceinline__ void gate_epilogue(const LayerParams& p, uint32_t tile, f32x4 (&acc)[NG], int lane) {
-    const int col = lane & 15, chunk = lane >> 4;
-    const uint32_t E = p.E;
-    const uint32_t token = tile * kGateTileTokens + col;
-    // This lane holds, for its token, experts e = 16 g + 4 chunk + v. The logits stay in the
-    // accumulator registers (padded experts set to -inf); probabilities are recomputed where they
-    // are needed rather than kept, and the selection rounds are packed two to a register: with 16
-    // expert groups there is no room for three more arrays of the accumulator's size.
-    const float kNegInf = -__builtin_inff();
-    float m = kNegInf;
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const uint32_t e = 16 * g + 4 * chunk + v;
-            if (e < E) p.logits[size_t(token) * E + e] = acc[g][v];
-            // softmax domain = the E real experts only (gate.cuh:550)
-            else acc[g][v] = kNegInf;
-            m = fmaxf(m, acc[g][v]);
-        }
-    m = fmaxf(m, __shfl_xor(m, 16));
-    m = fmaxf(m, __shfl_xor(m, 32));
-    float d = 0.f;
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) d += __expf(acc[g][v] - m);   // exp(-inf) = 0 for padded experts
-    d += __shfl_xor(d, 16);
-    d += __shfl_xor(d, 32);
-    const float inv_d = 1.0f / d;
-    auto prob = [&](float logit) { return __expf(logit - m) * inv_d; };
-    T* grow = static_cast<T*>(p.gate_out) + size_t(token) * p.PX;
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const uint32_t e = 16 * g + 4 * chunk + v;
-            // gateOut[t, e] = Element(p) (gate.cuh:590-605); padded columns are zero
-            if (e < p.PX) grow[e] = float_to_elem<T>(e < E ? prob(acc[g][v]) : 0.f);
-        }
-    for (uint32_t e = 16 * NG + 4 * chunk; e < p.PX; e += 16) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (e + v < p.PX) grow[e + v] = float_to_elem<T>(0.f);
-    }
-
-    if (p.is_training) {
-        // Column sums of the tile's probabilities for the load-balancing loss (gate.cuh:608-635):
-        // the 16 tokens of an expert sit in 16 consecutive lanes, summed by a fixed xor tree.
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t e = 16 * g + 4 * chunk + v;
-                float col_sum = prob(acc[g][v]);
-                col_sum += __shfl_xor(col_sum, 1);
-                col_sum += __shfl_xor(col_sum, 2);
-                col_sum += __shfl_xor(col_sum, 4);
-                col_sum += __shfl_xor(col_sum, 8);
-                if (col == 0 && e < E) store_through(p.tile_prob + size_t(tile) * E + e, col_sum);
-            }
-    }
-
-    // top-k: k rounds of arg-max, equal values go to the lower expert index (gate.cuh:654-670).
-    // picked[g][v / 2] holds, in the 16-bit half v % 2, 1 + the round that selected the expert.
-    uint32_t picked[NG][2];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) picked[g][0] = picked[g][1] = 0u;
-    auto round_of = [&](int g, int v) { return (picked[g][v >> 1] >> (16 * (v & 1))) & 0xffffu; };
-    float den = 0.f;
-    constexpr uint32_t kNone = 0x7fffffffu;
-    for (uint32_t r = 0; r < p.k; ++r) {
-        float best = kNegInf;
-        uint32_t bi = kNone;
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t e = 16 * g + 4 * chunk + v;
-                // padded experts hold -inf and can never beat the initial best
-                if (round_of(g, v) == 0 && acc[g][v] > best) {
-                    best = acc[g][v];
-                    bi = e;
-                }
-            }
-#pragma unroll
-        for (int off = 16; off <= 32; off <<= 1) {
-            const float ob = __shfl_xor(best, off);
-            const uint32_t oi = __shfl_xor(bi, off);
-            if (oi != kNone && (bi == kNone || ob > best || (ob == best && oi < bi))) {
-                best = ob;
-                bi = oi;
-            }
-        }
-        float pv = 0.f;
-#pragma unroll
-        for (int g = 0; g < NG; ++g)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const uint32_t e = 16 * g + 4 * chunk + v;
-                if (e == bi) {
-                    picked[g][v >> 1] |= (r + 1u) << (16 * (v & 1));
-                    pv = prob(acc[g][v]);
-                }
-            }
-        // exactly one of the four lanes of this token holds the winner; the others add 0
-        pv += __shfl_xor(pv, 16);
-        pv += __shfl_xor(pv, 32);
-        den += pv;   // mCw, accumulated in selection order (gate.cuh:669)
-        if (chunk == 0) {
-            store_through(p.topk_expert + size_t(token) * p.k + r, int32_t(bi));
-            store_through(p.topk_prob + size_t(token) * p.k + r, pv);
-        }
-    }
-    if (chunk == 0) store_through(p.combine_den + token, den);
-
-    // Histogram of the tile and each token's rank inside it (gate.cuh:678-696).
-    uint32_t* super = p.super_count + size_t(p.epoch & 1u) * p.n_super * E +
-                      size_t(tile / kSuperTiles) * E;
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const uint32_t e = 16 * g + 4 * chunk + v;
-            const uint32_t rnd = round_of(g, v);
-            const bool sel = rnd != 0;
-            const unsigned long long mask = __ballot(sel);
-            const uint32_t sub = uint32_t(mask >> (16 * chunk)) & 0xffffu;
-            if (sel)
-                store_through(p.topk_slot + size_t(token) * p.k + (rnd - 1), int32_t(__popc(sub & ((1u << col) - 1u))));
-            if (col == 0 && e < E) {
-                const uint32_t cnt = __popc(sub);
-                store_through(p.tile_count + size_t(tile) * E + e, cnt);
-                if (cnt) atomic_add_agent(super + e, cnt);
-            }
-        }
-}
 
 // Sums of the K steps s0 .. s1-1 of TB token blocks against NG groups of 16 experts, from zero: logits^T, experts are
 // the matrix-core rows, tokens its columns (gate.cuh:526-534). `xrow`, `wrow`: the lane's own row at its chunk of a step.
@@ -366,37 +224,43 @@ __device__ __forceinline__ void gate_unit(const LayerParams& p, uint32_t unit, f
         }
         return;
     }
-    // Block b: every wavefront parks the partial sums of its share in LDS, wavefront b adds them
-    // in ascending order of the shares (a fixed order: the logits depend neither on timing nor on
-    // which wavefront worked on which share).
+    // More experts, block after block: every wavefront parks the partial sums of its share in LDS, one group of four adds
+    // them in ascending order, each lane four experts of every 64, and finishes the block. Softmax and top-k by a single
+    // wavefront, whose lanes each held a quarter of a token's experts, were a chain of some 3 000 instructions beside idle
+    // wavefronts, with 2 045 registers spilled at 128 experts. 32-bit Elements, us per forward (256 columns up): 1 024 tokens of
+    // 1 024 values, 128 experts top-2, fp32 180 -> 129, 256 experts top-8 307 -> 247; 15 616 tokens of 512 values, 128 experts
+    // top-2, fp32 406 -> 298, tf32 391 -> 198, 256 experts top-4, tf32 497 -> 300; 4 096 tokens of 2 048, 256 experts, fp32 542 -> 490.
+    constexpr int NL = (NG + 3) / 4;
+    const uint32_t group = uint32_t(wave) >> 2, gtid = threadIdx.x & 255u;
+    uint32_t* gsm = reinterpret_cast<uint32_t*>(smem) + group * gate_group_words(p.E, p.k, p.is_training != 0);
+    const int sub = lane & 15;                              // experts 64 j + 4 sub .. + 3
+    const int tl = 4 * (wave & 3) + (lane >> 4);            // token inside the block
 #pragma unroll
     for (int b = 0; b < TB; ++b) {
-        float* dst = smem + part * (NG * 4 * kWave);
+        constexpr int kShare = NG * 4 * kGateParkStride;
+        float* dst = smem + part * kShare;
 #pragma unroll
         for (int g = 0; g < NG; ++g)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) dst[(g * 4 + v) * kWave + lane] = acc[b][g][v];
+            for (int v = 0; v < 4; ++v) dst[(g * 4 + v) * kGateParkStride + lane] = acc[b][g][v];
         __syncthreads();
-        if (wave == b) {
+        const bool mine = live[b] && group == 0;
+        f32x4 sum[NL];
 #pragma unroll
-            for (int g = 0; g < NG; ++g)
+        for (int j = 0; j < NL; ++j) {
+            sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (!mine || 16 * j + sub >= 4 * NG) continue;
+            const float* src = smem + (16 * j + (sub & 12)) * kGateParkStride + 16 * (sub & 3) + tl;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[b][g][v] = smem[(g * 4 + v) * kWave + lane];
+            for (int v = 0; v < 4; ++v) sum[j][v] = src[v * kGateParkStride];
 #pragma unroll
-            for (int w = 1; w < KW; ++w) {
-                const float* src = smem + w * (NG * 4 * kWave);
+            for (int w = 1; w < KW; ++w)
 #pragma unroll
-                for (int g = 0; g < NG; ++g)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[b][g][v] += src[(g * 4 + v) * kWave + lane];
-            }
+                for (int v = 0; v < 4; ++v) sum[j][v] += src[w * kShare + v * kGateParkStride];
         }
-        __syncthreads();
+        __syncthreads();   // the sums are in registers: their LDS is the epilogue's
+        gate_group_finish<T, NL>(p, unit * TB + b, mine, sum, gsm, gtid);
     }
-#pragma unroll
-    for (int b = 0; b < TB; ++b)
-        if (wave == b && live[b]) gate_epilogue<T, NG>(p, unit * TB + b, acc[b], lane);
-    __syncthreads();
 }
 
 // Few tokens leave most CUs without a gate unit, and a unit's loop runs at what one CU gets of the memory system (128
@@ -467,38 +331,27 @@ __device__ __forceinline__ void gate_spread(const LayerParams& p, uint32_t ways,
         __syncthreads();
         const bool last = valid && *flag != 0u;
         asm volatile("" ::: "memory");   // the sums are read behind the arrival
-        if constexpr (NG <= 4) {
-            const uint32_t part = uint32_t(wave) >> 2, gtid = threadIdx.x & 255u;
-            uint32_t* gsm = reinterpret_cast<uint32_t*>(smem) + kWave + part * gate_group_words(p.E, p.k, p.is_training != 0);
-            const int sub16 = lane & 15;                            // experts 4 sub16 .. 4 sub16 + 3
-            const int tl = 4 * (wave & 3) + (lane >> 4);            // token inside the tile
-            f32x4 sum[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
-            const bool mine = last && part == 0;
-            if (mine && sub16 < 4 * NG) {
-                // expert 4 sub16 + v is word v of lane 16 (sub16 % 4) + token of the share's group sub16 / 4
-                u32x4 v[KW];
+        const uint32_t part = uint32_t(wave) >> 2, gtid = threadIdx.x & 255u;
+        uint32_t* gsm = reinterpret_cast<uint32_t*>(smem) + kWave + part * gate_group_words(p.E, p.k, p.is_training != 0);
+        constexpr int NL = (NG + 3) / 4;
+        const int sub16 = lane & 15;                            // experts 64 j + 4 sub16 .. + 3
+        const int tl = 4 * (wave & 3) + (lane >> 4);            // token inside the tile
+        const bool mine = last && part == 0;
+        f32x4 sum[NL];
 #pragma unroll
-                for (int w = 0; w < KW; ++w)
-                    v[w] = load16_coherent(sums, uint32_t(((w * NG + (sub16 >> 2)) * kWave + 16 * (sub16 & 3) + tl) * 16));
-                sum[0] = __builtin_bit_cast(f32x4, v[0]);
+        for (int j = 0; j < NL; ++j) {
+            sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (!mine || 16 * j + sub16 >= 4 * NG) continue;
+            // expert 64 j + 4 sub16 + v is word v of lane 16 (sub16 % 4) + token of the share's group 4 j + sub16 / 4
+            u32x4 v[KW];
 #pragma unroll
-                for (int w = 1; w < KW; ++w) sum[0] += __builtin_bit_cast(f32x4, v[w]);
-            }
-            gate_group_finish<T, 1>(p, tile, mine, sum, gsm, gtid);
-        } else {
-            if (last && wave == 0) {
-                f32x4 acc[NG];
+            for (int w = 0; w < KW; ++w)
+                v[w] = load16_coherent(sums, uint32_t(((w * NG + 4 * j + (sub16 >> 2)) * kWave + 16 * (sub16 & 3) + tl) * 16));
+            sum[j] = __builtin_bit_cast(f32x4, v[0]);
 #pragma unroll
-                for (int g = 0; g < NG; ++g) acc[g] = __builtin_bit_cast(f32x4, load16_coherent(sums, uint32_t((g * kWave + lane) * 16)));
-#pragma unroll
-                for (int w = 1; w < KW; ++w)
-#pragma unroll
-                    for (int g = 0; g < NG; ++g)
-                        acc[g] += __builtin_bit_cast(f32x4, load16_coherent(sums, uint32_t(((w * NG + g) * kWave + lane) * 16)));
-                gate_epilogue<T, NG>(p, tile, acc, lane);
-            }
-            __syncthreads();
+            for (int w = 1; w < KW; ++w) sum[j] += __builtin_bit_cast(f32x4, v[w]);
         }
+        gate_group_finish<T, NL>(p, tile, mine, sum, gsm, gtid);
     }
 }
 
@@ -735,7 +588,7 @@ __device__ __forceinline__ f32x4 gate_partial_sum(const LayerParams& p, coherent
 // in runs of 256 and 128 bytes per token. The tile's picks meet in LDS: every pick counts the picks
 // of its expert by earlier tokens for its in-tile rank and adds itself to the tile's histogram,
 // which the group then writes out. Same sums over the
-// ranges, same selection rule and same order of the denominator as gate_epilogue; the softmax
+// ranges, same selection rule and same order of the denominator as the gate of more than 256 experts; the softmax
 // denominator is summed in a different (fixed) order.
 // `gsm`: gate_group_words(p) words of LDS private to the group. Every thread of the workgroup must
 // call the function the same number of times (it contains workgroup barriers); a group without a

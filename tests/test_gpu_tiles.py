@@ -144,6 +144,40 @@ def test_gate_tiles_spread_over_workgroups_keep_their_bits(dt, S, H, I, E):
     np.testing.assert_array_equal(out0, out1)
 
 
+@pytest.mark.parametrize("dt,S,H,E,k", [
+    (0, 512, 64, 65, 3),          # whole units in both modes; one expert past the first run of 64
+    (1, 384, 64, 128, 128),       # every expert picked by every token
+    (0, 256, 64, 129, 8),         # a third run of 64 that holds one expert
+    (1, 256, 64, 256, 5),
+    (0, 256, 512, 127, 4),        # spread over workgroups in the persistent launch
+    (1, 128, 1024, 256, 256),
+], ids=lambda v: str(v))
+def test_gate_of_many_experts_in_32_bits(dt, S, H, E, k):
+    """65 to 256 experts of 32-bit Elements: a block of 16 tokens by a group of four wavefronts. Against the oracle, the same bits
+    in both modes, and the gate's loss of a training step: sums over S probabilities, rounded in fp32, S 2^-24 = 3e-5 at most."""
+    keys = _keys(S, H, 64, E, k, dt=dt)
+    keys.is_training = 1
+    c = moe_ref.cfg_from_keys(keys)
+    iP = pack_inputs(c, *random_layer(c, seed=S + E, w_std=0.05, bias_std=0.1))
+    got = []
+    for mode in MODES[:2]:
+        d, v, out, _ = check_against_oracle(c, keys, iP, mode)
+        got.append((v, out))
+    for name in ("logits", "topk_expert", "topk_prob", "topk_slot", "expert_count"):
+        np.testing.assert_array_equal(got[0][0][name], got[1][0][name])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    ref = moe_ref.gate_loss(c, moe_ref.route(c, got[0][0]["logits"])["probs"], got[0][0]["expert_count"])
+    ka.initialize(keys)
+    try:
+        ka.moe.forward_host(_to_device(c, iP), synth.alloc_outputs(d))
+        ka.moe.stream_synchronize()
+        g = ka.moe.gate_loss(d.E)
+    finally:
+        ka.finalize()
+    assert abs(g["loss"] - ref["loss"]) <= 3e-5 * ref["loss"]
+    np.testing.assert_allclose(g["mean_prob"], ref["mean_prob"], rtol=3e-5, atol=1e-8)
+
+
 @pytest.mark.parametrize("dt,S,H,I", [(2, 128, 64, 64), (2, 2048, 320, 448), (3, 1152, 192, 1216), (0, 640, 128, 320), (1, 2304, 1088, 1152)])
 def test_dense_forward_leaves_the_routing_out(dt, S, H, I):
     """One expert in the dense packing: rows are tokens, nothing is routed. The bits of a routed forward, also between
