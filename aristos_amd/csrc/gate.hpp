@@ -230,6 +230,7 @@ __device__ __forceinline__ void gate_unit(const LayerParams& p, uint32_t unit, f
     // wavefronts, with 2 045 registers spilled at 128 experts. 32-bit Elements, us per forward (256 columns up): 1 024 tokens of
     // 1 024 values, 128 experts top-2, fp32 180 -> 129, 256 experts top-8 307 -> 247; 15 616 tokens of 512 values, 128 experts
     // top-2, fp32 406 -> 298, tf32 391 -> 198, 256 experts top-4, tf32 497 -> 300; 4 096 tokens of 2 048, 256 experts, fp32 542 -> 490.
+    static_assert(NG < 4 || NG % 4 == 0);
     constexpr int NL = (NG + 3) / 4;
     const uint32_t group = uint32_t(wave) >> 2, gtid = threadIdx.x & 255u;
     uint32_t* gsm = reinterpret_cast<uint32_t*>(smem) + group * gate_group_words(p.E, p.k, p.is_training != 0);
@@ -249,7 +250,7 @@ __device__ __forceinline__ void gate_unit(const LayerParams& p, uint32_t unit, f
 #pragma unroll
         for (int j = 0; j < NL; ++j) {
             sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (!mine || 16 * j + sub >= 4 * NG) continue;
+            if (!mine) continue;
             const float* src = smem + (16 * j + (sub & 12)) * kGateParkStride + 16 * (sub & 3) + tl;
 #pragma unroll
             for (int v = 0; v < 4; ++v) sum[j][v] = src[v * kGateParkStride];
@@ -336,20 +337,22 @@ __device__ __forceinline__ void gate_spread(const LayerParams& p, uint32_t ways,
         constexpr int NL = (NG + 3) / 4;
         const int sub16 = lane & 15;                            // experts 64 j + 4 sub16 .. + 3
         const int tl = 4 * (wave & 3) + (lane >> 4);            // token inside the tile
-        const bool mine = last && part == 0;
         f32x4 sum[NL];
 #pragma unroll
-        for (int j = 0; j < NL; ++j) {
-            sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (!mine || 16 * j + sub16 >= 4 * NG) continue;
-            // expert 64 j + 4 sub16 + v is word v of lane 16 (sub16 % 4) + token of the share's group 4 j + sub16 / 4
-            u32x4 v[KW];
+        for (int j = 0; j < NL; ++j) sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const bool mine = last && part == 0;
+        if (mine && sub16 < 4 * NG) {
 #pragma unroll
-            for (int w = 0; w < KW; ++w)
-                v[w] = load16_coherent(sums, uint32_t(((w * NG + 4 * j + (sub16 >> 2)) * kWave + 16 * (sub16 & 3) + tl) * 16));
-            sum[j] = __builtin_bit_cast(f32x4, v[0]);
+            for (int j = 0; j < NL; ++j) {
+                // expert 64 j + 4 sub16 + v is word v of lane 16 (sub16 % 4) + token of the share's group 4 j + sub16 / 4
+                u32x4 v[KW];
 #pragma unroll
-            for (int w = 1; w < KW; ++w) sum[j] += __builtin_bit_cast(f32x4, v[w]);
+                for (int w = 0; w < KW; ++w)
+                    v[w] = load16_coherent(sums, uint32_t(((w * NG + 4 * j + (sub16 >> 2)) * kWave + 16 * (sub16 & 3) + tl) * 16));
+                sum[j] = __builtin_bit_cast(f32x4, v[0]);
+#pragma unroll
+                for (int w = 1; w < KW; ++w) sum[j] += __builtin_bit_cast(f32x4, v[w]);
+            }
         }
         gate_group_finish<T, NL>(p, tile, mine, sum, gsm, gtid);
     }
