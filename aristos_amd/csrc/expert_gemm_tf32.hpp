@@ -507,9 +507,9 @@ struct GemmSplit {
 // truncating conversion to fp16 cuts a value to what the tf32 instructions read of it, a product of two such values is exact
 // in fp32. What does not fit is noticed, and the whole tile then computed by GemmSplit:
 //   - a value that overflows, an infinity, a row whose first slice lies outside 2^-40 .. 2^40;
-//   - a value below 2^-14 once scaled, which may lose bits below 2^-24. One in some ten million of a random operand does,
-//     and no sum shows it: the tile is kept if all K products of a row (column) together could not lose more than
-//     2^-22 of the largest sum of that row (column), a fraction of what rounding the sums in fp32 loses.
+//   - a value below 2^-14 once scaled, which may lose bits below 2^-24. One in some ten million of a random operand does. What
+//     the values of a row lose at most is added up, and the tile is kept if for every single one of its sums this stays below 2^-24 of
+//     the magnitudes of that sum's own products: less than adding them up in fp32 may lose anyway (`hidden`).
 // (A NaN needs no care: it makes the same sums NaN.)
 //
 // K in slices of 32 values (128-byte rows). Four wavefronts bring the weight rows of a slice, four the activation rows, as
@@ -557,8 +557,10 @@ struct GemmHalf {
     static constexpr int kRingX = L, kRingW = 2 * L;
     static constexpr int kRings = kLoaders * (kRingX + kRingW) * 1024;
     static constexpr int kExponents = Split::kSmemBytes;                 // powers of two that scale a sum back: int32 [BM rows | BN columns]
-    static constexpr int kRangeOffset = kExponents + (BM + BN) * 4;      // per bias slot: the Range words
-    static constexpr int kRangeWords = 4;
+    static constexpr int kLargest = kExponents + (BM + BN) * 4;          // of every scaled row: its largest value (bits of a float)
+    static constexpr int kLoss = kLargest + (BM + BN) * 4;               // what its values lose at most, in units of 2^-34 (hidden)
+    static constexpr int kRangeOffset = kLoss + (BM + BN) * 4;           // per bias slot: the Range words
+    static constexpr int kRangeWords = 4 + 2 * kWaves;
     static constexpr int kSmemBytes = kRangeOffset + 2 * kRangeWords * 4;
     static_assert(kConverted + kRings <= 2 * Split::kStage && kWaves * 4096 <= kConverted);
     typedef typename Split::Acc Acc;
@@ -569,12 +571,15 @@ struct GemmHalf {
         int bias_slot;
     };
 
-    // words of a tile's range: largest scaled activation and weight (bits of a float), what the tile holds that calls for a second look
-    enum : uint32_t { kLargestX = 0, kLargestW = 1, kSeen = 2 };
-    enum : uint32_t { kOutOfRange = 1, kSmallX = 2, kSmallW = 4 };
+    // words of a tile's range: what it holds that calls for a second look, then for every wavefront in which slices (their number
+    // modulo 64, two words) the rows it brings have values that lose bits
+    enum : uint32_t { kSeen = 0, kSlices = 4 };
+    enum : uint32_t { kOutOfRange = 1, kLossy = 2, kInDoubt = 4 };
     static __device__ __forceinline__ uint32_t* range_words(char* smem, int bias_slot) {
         return reinterpret_cast<uint32_t*>(smem + kRangeOffset) + bias_slot * kRangeWords;
     }
+
+    static __device__ __forceinline__ uint32_t* lossy_slices(char* smem, int bias_slot) { return range_words(smem, bias_slot) + kSlices + 2 * wave_index(); }
 
     static __device__ __forceinline__ int next_stage0(const Tile&) { return 0; }
     static __device__ __forceinline__ uint32_t first_value(const Tile& t, uint32_t kt) {
@@ -604,22 +609,16 @@ struct GemmHalf {
             static_assert(W > X);
         }
     }
-    // As Gemm16::begin; requests as many slices as the wavefront's ring holds.
-    static __device__ __forceinline__ void begin(Tile& t, const GemmTileArgs<float>& args, int, int bias_slot, char* smem) {
-        const GemmTileArgs<float> g = scalar(args);
+    // The word of a per-row array that belongs to the row whose values of kilobyte i lie in this lane.
+    static __device__ __forceinline__ uint32_t* row_word(char* smem, int array, int i) {
+        const uint32_t row = kRowsPerLoad * (loader() + kLoaders * i) + ((threadIdx.x & 63) >> 3);
+        return reinterpret_cast<uint32_t*>(smem + array) + (brings_w() ? BM : 0) + row;
+    }
+    // This lane's rows of the operand that its wavefront brings, at its chunk of a slice.
+    static __device__ __forceinline__ void locate(const GemmTileArgs<float>& g, const float* (&rows)[L]) {
         const uint32_t tid = local_tid();
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
         const int ld_r = lane >> 3, ld_c = lane & 7;
-        if (wave == 0 && lane < Split::kBiasBytes / 16) {
-            const uint32_t n = uint32_t(lane) * 4 < g.n_valid ? uint32_t(lane) * 4 : 0u;
-            direct_load16<false>(g.bias + n, lds_address(smem) + Split::kBiasOffset + bias_slot * Split::kBiasBytes);
-        }
-        // (last read by the epilogue of the tile before the previous one, written again behind the main loop's barriers)
-        if (tid < uint32_t(kRangeWords)) range_words(smem, bias_slot)[tid] = 0u;
-        t.g = g;
-        t.k_tiles = g.K / kSliceK;
-        t.g.k_first = g.k_first < t.k_tiles ? g.k_first : 0u;
-        t.bias_slot = bias_slot;
         const bool w = wave & 1;
         const int valid = w ? g.n_valid : g.m_valid;
         uint32_t src[L];
@@ -639,12 +638,33 @@ struct GemmHalf {
             const int row = kRowsPerLoad * ((wave >> 1) + kLoaders * i) + ld_r;
             const float* from = w ? g.b_base + size_t(src[i]) * g.ldb : g.a_base + size_t(src[i]) * g.lda;
             if (!w && g.a_pad && row >= valid) from = g.a_pad;
-            t.rows[i] = from + 4 * ld_c;
+            rows[i] = from + 4 * ld_c;
+        }
+    }
+    // As Gemm16::begin; requests as many slices as the wavefront's ring holds.
+    static __device__ __forceinline__ void begin(Tile& t, const GemmTileArgs<float>& args, int, int bias_slot, char* smem) {
+        const GemmTileArgs<float> g = scalar(args);
+        const uint32_t tid = local_tid();
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+        if (wave == 0 && lane < Split::kBiasBytes / 16) {
+            const uint32_t n = uint32_t(lane) * 4 < g.n_valid ? uint32_t(lane) * 4 : 0u;
+            direct_load16<false>(g.bias + n, lds_address(smem) + Split::kBiasOffset + bias_slot * Split::kBiasBytes);
+        }
+        // (last read by the epilogue of the tile before the previous one, written again behind the main loop's barriers)
+        if (tid < uint32_t(kRangeWords)) range_words(smem, bias_slot)[tid] = 0u;
+        t.g = g;
+        t.k_tiles = g.K / kSliceK;
+        t.g.k_first = g.k_first < t.k_tiles ? g.k_first : 0u;
+        t.bias_slot = bias_slot;
+        locate(g, t.rows);
+        if ((lane & 7) == 0) {   // written by this wavefront alone, last read by the previous tile in front of a barrier
+#pragma unroll
+            for (int i = 0; i < L; ++i) *row_word(smem, kLargest, i) = 0u;
         }
         const uint32_t ring = lds_address(smem) + ring_offset();
 #pragma unroll
         for (int i = 0; i < L; ++i) load(t.rows[i] + first_value(t, 0), ring + 1024 * i, brings_w());
-        if (w && t.k_tiles > 1) {
+        if (brings_w() && t.k_tiles > 1) {
 #pragma unroll
             for (int i = 0; i < L; ++i) load(t.rows[i] + first_value(t, 1), ring + 1024 * (L + i), brings_w());
         }
@@ -658,10 +678,11 @@ struct GemmHalf {
         const int r = lane >> 3, c = lane & 7;      // (the kilobytes of a wavefront are kLoaders * kRowsPerLoad rows apart: one swizzle)
         return uint32_t(r * kRowBytes + (((c >> 1) ^ swizzle(kRowsPerLoad * (wave >> 1) + r)) << 4) + (c & 1) * 8);
     }
-    // What a thread has seen of the scaled values: the largest, and the least that is not zero (2 * bits - 1, zero wraps to the top).
-    struct Seen { float largest = 0.f; uint32_t least = ~0u; };
-    static constexpr uint32_t kLeast = (0x38800000u << 1) - 1u;          // 2^-14, the least normal fp16 value
-    static __device__ __forceinline__ void convert(char* to, u32x4 raw, float scale, Seen& seen) {
+    static __device__ __forceinline__ uint32_t halves(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b)); }
+    // A scaled value loses bits if it is not zero, and below 2^-14, the least normal fp16 value: if 2 * bits - 1 is less than this.
+    static constexpr uint32_t kSmall = (0x38800000u << 1) - 1u;
+    // `largest`: of the scaled values that this thread has seen of the row. `least`: 2 * bits - 1 of those of the slice.
+    static __device__ __forceinline__ void convert(char* to, u32x4 raw, float scale, float& largest, uint32_t& least) {
         float v[4];
         uint32_t u[4];
 #pragma unroll
@@ -670,15 +691,14 @@ struct GemmHalf {
             v[j] = __builtin_bit_cast(float, word) * scale;
             u[j] = (__builtin_bit_cast(uint32_t, v[j]) << 1) - 1u;
         }
-        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(seen.largest) : "v"(v[0]), "v"(v[1]));
-        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(seen.largest) : "v"(v[2]), "v"(v[3]));
-        const uint32_t a = u[0] < u[1] ? u[0] : u[1], b = u[2] < u[3] ? u[2] : u[3], c = a < b ? a : b;
-        seen.least = c < seen.least ? c : seen.least;
-        const u32x2 half{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(v[0], v[1])), __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(v[2], v[3]))};
-        *reinterpret_cast<u32x2*>(to) = half;
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(v[0]), "v"(v[1]));
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(v[2]), "v"(v[3]));
+        asm("v_min3_u32 %0, %0, %1, %2" : "+v"(least) : "v"(u[0]), "v"(u[1]));
+        asm("v_min3_u32 %0, %0, %1, %2" : "+v"(least) : "v"(u[2]), "v"(u[3]));
+        *reinterpret_cast<u32x2*>(to) = u32x2{halves(v[0], v[1]), halves(v[2], v[3])};
     }
     // The scale of the row whose values of the first slice lie in this lane and the seven beside it.
-    static __device__ __forceinline__ int row_exponent(u32x4 raw, uint32_t& seen) {
+    static __device__ __forceinline__ int row_exponent(u32x4 raw, uint32_t& flags) {
         uint32_t largest = 0u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -691,7 +711,7 @@ struct GemmHalf {
         with(row16_peer<2>(largest));   // (the three steps combine aligned groups of eight lanes)
         const int e = int(largest >> 23) - 127;
         if (largest == 0u) return 0;
-        if (e < -40 || e > 40) { seen = kOutOfRange; return 0; }
+        if (e < -40 || e > 40) { flags |= kOutOfRange; return 0; }
         return 9 - e;
     }
 
@@ -699,9 +719,11 @@ struct GemmHalf {
     static __device__ __forceinline__ void mainloop(const Tile& t, Acc& acc, char* smem, Hook&& after_first_barrier) {
         const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
         const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-        Seen seen;
-        float scale[L];
+        float scale[L], largest[L];
+#pragma unroll
+        for (int i = 0; i < L; ++i) largest[i] = 0.f;
         uint32_t flags = 0u;
+        uint64_t lossy = 0;   // slices (modulo 64) in which a value loses bits
         const uint32_t w = brings_w(), ring = lds_address(smem) + ring_offset();
         const char* const ring_lane = smem + ring_offset() + 16 * lane;
         char* const to = smem + (w ? kABytes : 0) + 512 * loader() + half_offset();
@@ -727,14 +749,16 @@ struct GemmHalf {
         };
         // Kilobytes 0 .. L-1 of slice s, the first of them requested: `between(i)` runs while number i + 1 is on its way.
         auto convert_slice = [&](auto stage_tag, uint32_t s, auto&& between, auto&& first) {
+            uint32_t least = ~0u;
             static_for<L>([&](auto i_tag) {
                 constexpr int i = decltype(i_tag)::value;
                 reload(stage_tag, i_tag, s);
                 if constexpr (i + 1 < L) request(stage_tag, std::integral_constant<int, (i + 1 < L ? i + 1 : 0)>{}, s);
                 between(i);
                 first(i_tag);
-                convert(to + 512 * kLoaders * i, raw[i & 1], scale[i], seen);
+                convert(to + 512 * kLoaders * i, raw[i & 1], scale[i], largest[i], least);
             });
+            lossy |= uint64_t(__builtin_amdgcn_ballot_w64(least < kSmall) != 0u) << (s & 63u);
         };
         auto stages = [&](uint32_t s, auto&& f) {
             if (s + 2 < t.k_tiles) f(std::integral_constant<int, kBoth>{});
@@ -750,20 +774,26 @@ struct GemmHalf {
                 constexpr int i = decltype(i_tag)::value;
                 const int e = row_exponent(raw[i & 1], flags);
                 scale[i] = __builtin_bit_cast(float, uint32_t(e + 127) << 23);
+                if (e < 0) flags |= kLossy;
                 const int row = kRowsPerLoad * (int(loader()) + kLoaders * i) + (lane >> 3);
                 if ((lane & 7) == 0) reinterpret_cast<int*>(smem + kExponents)[(w ? BM : 0) + row] = -e;
             });
         });
         auto top = [&](uint32_t kt) {
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            meet();
             if (kt == 0) after_first_barrier();
         };
         auto report = [&] {
-            if (seen.least < kLeast) flags |= w ? kSmallW : kSmallX;
-            if (seen.largest >= 65536.f) flags |= kOutOfRange;
-            uint32_t* words = range_words(smem, t.bias_slot);
-            atomicMax(words + (w ? kLargestW : kLargestX), __builtin_bit_cast(uint32_t, seen.largest));
-            if (flags) atomicOr(words + kSeen, flags);
+            if (lossy != 0u) {
+                flags |= kLossy;
+                if (lane < 2) lossy_slices(smem, t.bias_slot)[lane] = uint32_t(lossy >> (32 * lane));
+            }
+#pragma unroll
+            for (int i = 0; i < L; ++i) {
+                if (largest[i] >= 65536.f) flags |= kOutOfRange;
+                atomicMax(row_word(smem, kLargest, i), __builtin_bit_cast(uint32_t, largest[i]));
+            }
+            if (flags) atomicOr(range_words(smem, t.bias_slot) + kSeen, flags);
         };
         auto nothing = [](auto) {};
         if (Split::rows_absent_of(t.g.m_valid, __builtin_amdgcn_readfirstlane(wave) / WAVES_N)) {
@@ -825,42 +855,137 @@ struct GemmHalf {
         report();
     }
 
-    // Whether the bits that values below 2^-14 may have lost stay under the rounding of this wavefront's sums.
-    static __device__ __forceinline__ bool losses_hidden(const Tile& t, const Acc& acc, const uint32_t* words, uint32_t flags) {
-        const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-        // a sum loses less than K 2^-24 times the largest partner; 2^-22 of the largest sum of its row or column
-        const float count = float(t.k_tiles * kSliceK) * 0.25f;
-        const float least_row = count * __builtin_bit_cast(float, words[kLargestW]), least_col = count * __builtin_bit_cast(float, words[kLargestX]);
-        bool hidden = true;
-        float col[TN][4];
+    // Whether, in every sum of this wavefront, what small values lost (kLoss) stays below 2^-24 of the magnitudes of the products: whether
+    // the products of some of the slices alone, converted one beside the other in LDS, are 2^24 of it.
+    static __device__ __forceinline__ bool covered(const GemmTileArgs<float>& g, const char* smem, uint32_t samples) {
+        const int wave = int(wave_index()), lane = threadIdx.x & 63, wm = wave / WAVES_N, wn = wave % WAVES_N, part = lane >> 4;
+        if (Split::rows_absent_of(g.m_valid, wm)) return true;
+        const int rx = wm * WM + (lane & 15), rw = wn * WN + (lane & 15);
+        const char* const from_x = smem + rx * kRowBytes + ((part ^ swizzle(rx)) << 4);
+        const char* const from_w = smem + kABytes + rw * kRowBytes + ((part ^ swizzle(rw)) << 4);
+        auto magnitudes = [](const char* from) {
+            u32x4 v = load16(from);
 #pragma unroll
-        for (int ni = 0; ni < TN; ++ni)
+            for (int j = 0; j < 4; ++j) v[j] &= 0x7fff7fffu;
+            return __builtin_bit_cast(f16x8, v);
+        };
+        // Where the scale is below one, a value of less than 2^-149 once scaled is zero then, and nobody has seen it.
+        const float unseen = float(g.K) * 0x1p-126f;
+        // The largest value of a row, and 2^24 of what it lost. A row that is not there, or is all zeros, loses nothing.
+        auto row = [&](uint32_t r, bool exists, float& most, float& lost) {
+            const float a = __builtin_bit_cast(float, reinterpret_cast<const uint32_t*>(smem + kLargest)[r]);
+            const float b = 0x1p-10f * float(reinterpret_cast<const uint32_t*>(smem + kLoss)[r]) + (reinterpret_cast<const int*>(smem + kExponents)[r] > 0 ? unseen : 0.f);
+            most = exists ? a : 0.f;
+            lost = most > 0.f ? b : 0.f;
+        };
+        float margin = 0.f;
+#pragma unroll 1
+        for (int ni = 0; ni < TN; ++ni) {
+            float most_w[4], lost_w[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) col[ni][j] = 0.f;
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t n = wn * WN + ni * 16 + 4 * part + j;
+                row(BM + n, n < g.n_valid, most_w[j], lost_w[j]);
+            }
+#pragma unroll 2
+            for (int mi = 0; mi < TM; ++mi) {
+                const uint32_t m = wm * WM + mi * 16 + (lane & 15);
+                float most_x, lost_x;
+                row(m, m < g.m_valid, most_x, lost_x);
+                f32x4 sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (uint32_t q = 0; q < samples; ++q)
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(magnitudes(from_w + q * kConverted + ni * 16 * kRowBytes), magnitudes(from_x + q * kConverted + mi * 16 * kRowBytes), sum, 0, 0, 0);
 #pragma unroll
-        for (int mi = 0; mi < TM; ++mi) {
-            const bool exists = uint32_t((wave / WAVES_N) * WM + mi * 16 + (lane & 15)) < t.g.m_valid;
-            float row = 0.f;
+                for (int j = 0; j < 4; ++j) margin = __builtin_fminf(margin, sum[j] - (lost_x * most_w[j] + most_x * lost_w[j]));
+            }
+        }
+        return margin >= 0.f;
+    }
+    // The workgroup meets, what it wrote to LDS is there. (Does not wait for what is on its way from memory: the next tile's ticket.)
+    static __device__ __forceinline__ void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+    // Whether it holds for all wavefronts, each of which calls this; `verdict`: the bit that says it does not.
+    static __device__ __forceinline__ bool all(bool holds, uint32_t* words, uint32_t verdict) {
+        if (!holds) atomicOr(words + kSeen, verdict);
+        meet();
+        return !(scalar(words[kSeen]) & verdict);
+    }
+    static __device__ __forceinline__ uint64_t lossy_of(char* smem, int bias_slot) {
+        const uint32_t* mask = lossy_slices(smem, bias_slot);
+        return uint64_t(scalar(mask[1])) << 32 | scalar(mask[0]);
+    }
+    // Whether the losses are covered for sure, without another look at the operands: against the slice that is still in LDS, all values of
+    // a row taken to be small in the slices where one that its wavefront brought was. Every wavefront calls it behind the main loop. In
+    // loops, as `hidden`: both are rarely called, and take as long as their instructions take to fetch.
+    static __device__ __forceinline__ bool hidden_for_sure(const Tile& t, char* smem) {
+        const uint32_t most = uint32_t(__builtin_popcountll(lossy_of(smem, t.bias_slot))) * ((t.k_tiles + 63u) / 64u) * kSliceK << 10;
+#pragma unroll 1
+        for (int i = 0; i < L; ++i) *row_word(smem, kLoss, i) = most;
+        meet();
+        return all(covered(t.g, smem, 1), range_words(smem, t.bias_slot), kInDoubt);
+    }
+    // What the small values lost, against four slices spread over K. A function of its own, as `again`.
+    static __device__ __attribute__((noinline)) bool hidden(GemmTileArgs<float> args, uint32_t slot, uint32_t lds) {
+        const GemmTileArgs<float> g = scalar(args);
+        const int bias_slot = int(scalar(slot));
+        char* smem = (char*)(__attribute__((address_space(3))) char*)uintptr_t(scalar(lds));
+        const uint32_t k_tiles = g.K / kSliceK;
+        const uint64_t lossy = lossy_of(smem, bias_slot);
+        const float* rows[L];
+        locate(g, rows);
+        float scale[L];
+        uint32_t units[L];   // less than 2^-24 a value, and no more than itself
 #pragma unroll
-            for (int ni = 0; ni < TN; ++ni)
+        for (int i = 0; i < L; ++i) {
+            scale[i] = __builtin_amdgcn_ldexpf(1.f, -int(*row_word(smem, kExponents, i)));
+            units[i] = 0u;
+        }
+        const uint32_t k_first = g.k_first < k_tiles ? g.k_first : 0u;
+#pragma unroll 1
+        for (uint32_t s = 0; s < k_tiles; ++s) {
+            if (!((lossy >> (s & 63u)) & 1u)) continue;
+            const uint32_t slice = s + k_first >= k_tiles ? s + k_first - k_tiles : s + k_first;
+            u32x4 raw[L];
+#pragma unroll
+            for (int i = 0; i < L; ++i) raw[i] = load16(rows[i] + slice * kSliceK);
+#pragma unroll
+            for (int i = 0; i < L; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float v = __builtin_fabsf(acc[ni][mi][j]);
-                    row = __builtin_fmaxf(row, v);
-                    col[ni][j] = exists ? __builtin_fmaxf(col[ni][j], v) : col[ni][j];
+                    const uint32_t word = raw[i][j] & 0x7fffffffu;
+                    const float v = __builtin_bit_cast(float, word) * scale[i];
+                    units[i] += word != 0u && v < 0x1p-14f ? uint32_t(__builtin_fminf(v * 0x1p34f, 1023.f)) + 1u : 0u;
                 }
-            row = __builtin_fmaxf(row, __shfl_xor(row, 16));
-            row = __builtin_fmaxf(row, __shfl_xor(row, 32));
-            if ((flags & kSmallX) && exists && !(row >= least_row)) hidden = false;
         }
-        if (flags & kSmallW) {
+        constexpr uint32_t kSamples = 4;
+        static_assert(int(kSamples) * kConverted <= Split::kBiasOffset);
+        const uint32_t samples = k_tiles < kSamples ? k_tiles : kSamples;
+        char* const to = smem + (brings_w() ? kABytes : 0) + 512 * loader() + half_offset();
+#pragma unroll 1
+        for (uint32_t q = 0; q < samples; ++q) {
+            u32x4 raw[L];
 #pragma unroll
-            for (int ni = 0; ni < TN; ++ni)
+            for (int i = 0; i < L; ++i) raw[i] = load16(rows[i] + k_tiles * q / samples * kSliceK);
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (!(row16_allreduce(col[ni][j], [](float a, float b) { return __builtin_fmaxf(a, b); }) >= least_col)) hidden = false;
+            for (int i = 0; i < L; ++i) {
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t word = raw[i][j];
+                    v[j] = __builtin_bit_cast(float, word) * scale[i];
+                }
+                *reinterpret_cast<u32x2*>(to + q * kConverted + 512 * kLoaders * i) = u32x2{halves(v[0], v[1]), halves(v[2], v[3])};
+            }
         }
-        return hidden;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {   // the eight lanes of a row
+            units[i] += row16_peer<0>(units[i]);
+            units[i] += row16_peer<1>(units[i]);
+            units[i] += row16_peer<2>(units[i]);
+            if ((threadIdx.x & 7) == 0) *row_word(smem, kLoss, i) = units[i];
+        }
+        meet();
+        return all(covered(g, smem, samples), range_words(smem, bias_slot), kOutOfRange);
     }
 
     // The tile by GemmSplit. A function of its own: its registers are not those of the main loop's tile.
@@ -878,17 +1003,14 @@ struct GemmHalf {
     }
     static __device__ __forceinline__ void finish(const Tile& t, Acc& acc, char* smem) {
         uint32_t* words = range_words(smem, t.bias_slot);
-        uint32_t seen = __builtin_amdgcn_readfirstlane(words[kSeen]);   // the same in every wavefront
+        const uint32_t seen = __builtin_amdgcn_readfirstlane(words[kSeen]);   // the same in every wavefront
         const bool absent = Split::rows_absent_of(t.g.m_valid, __builtin_amdgcn_readfirstlane(int(local_tid() >> 6)) / WAVES_N);
-        if (seen != 0u && !(seen & kOutOfRange)) {
-            __syncthreads();   // everybody has read the word
-            if (!absent && !losses_hidden(t, acc, words, seen)) atomicOr(words + kSeen, uint32_t(kOutOfRange));
-            __syncthreads();
-            seen = __builtin_amdgcn_readfirstlane(words[kSeen]);
-        }
-        if (seen & kOutOfRange) {
-            again(t.g, t.bias_slot, uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)));
-            return;
+        if (__builtin_expect(seen != 0u, 0)) {
+            const uint32_t lds = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem));
+            if ((seen & kOutOfRange) || (!hidden_for_sure(t, smem) && !hidden(t.g, t.bias_slot, lds))) {
+                again(t.g, t.bias_slot, lds);
+                return;
+            }
         }
         if (absent) return;
         if (t.g.act == 0) finish_act<0>(t, acc, smem);

@@ -387,6 +387,43 @@ def test_tf32_rows_that_fit_fp16_and_rows_that_do_not(rows, operand):
     assert float(((got - want).norm(dim=1)[ok] / want.norm(dim=1)[ok]).max()) <= 2 * 2.0 ** -11
 
 
+@pytest.mark.parametrize("small,base,p", [
+    ("x", 0, 14), ("x", 0, 24), ("x", 0, 26), ("w_up", 0, 26), ("x", 0, 34), ("w_up", 0, 34),
+    ("x", 0, 50), ("w_up", 0, 70),        # below what a second fp16 value holds
+    ("x", 39, 150), ("w_up", 39, 158),    # nothing is left of them once their row is scaled
+    ("x and w_up", 0, 18), ("x and w_up", 0, 30), ("x and w_up", 10, 60),
+], ids=lambda v: str(v))
+def test_tf32_sums_of_small_values_beside_large_sums(small, base, p):
+    """Values from column 40 on 2^-p times the others, where every second row of the other operand is zero in front of column
+    40: sums of the small values alone beside ordinary ones, in the same rows (columns). Each sum against its own products: a
+    place of 11 bits for the rounding of h, 2^-19 of the products' magnitudes for 16 slices summed in fp32. w_down is the
+    identity, which has h itself read back."""
+    S, H, I = 16384, 512, 512
+    rng = np.random.default_rng(17)
+
+    def values(*n):   # 11 significant bits, 1 <= |v| < 2
+        return torch.from_numpy(rng.integers(1024, 2048, n) * rng.choice([-1.0, 1.0], n) / 1024)
+    x, w_up = values(S, H), values(I, H)
+    for name, a, b in (("x", x, w_up), ("w_up", w_up, x)):
+        if name in small.split(" and "):
+            a *= 2.0 ** base
+            a[:, 40:] *= 2.0 ** -p
+            b[1::2, :40] = 0.0
+    want, magnitude = torch.relu(x @ w_up.T), x.abs() @ w_up.T.abs()
+    iP = torch.cat([x.flatten(), w_up.flatten(), torch.eye(H, dtype=torch.double).flatten(), torch.zeros(H + I).double()]).float().cuda()
+    keys = _keys(S, H, I, 1, 1, act=0, dt=1)
+    _assert_tiles(keys, (3, 0))
+    ka.initialize(keys)
+    try:
+        oP = torch.zeros(S * H, device="cuda")
+        ka.moe.forward_host_dense(iP, oP)
+        ka.moe.stream_synchronize()
+        got = oP.view(S, H).cpu().double()
+    finally:
+        ka.finalize()
+    assert ((got - want).abs() <= 2.0 ** -11 * want + 2.0 ** -19 * magnitude).all()
+
+
 @pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
 @pytest.mark.parametrize("low,high", [(0.001, 0.1), (0.1, 0.5), (0.5, 1.0), (1.0, 2.0)])
 def test_gelu_keeps_the_bits_of_small_arguments(low, high, sign):
