@@ -503,10 +503,11 @@ struct GemmSplit {
 // The same tile with one fp16 product instead of four bf16 ones. An fp16 value holds the 11 significant bits of a tf32
 // operand; what it lacks is range. Every row of the tile is therefore scaled by a power of two of its own, chosen from the
 // row's values in the tile's first slice (their largest goes to 2^9 .. 2^10, so that the row may hold values 64 times as
-// large and keeps all bits of those down to 2^-24 of it), and the epilogue scales the sums back: scaling is exact, a
-// truncating conversion to fp16 cuts a value to what the tf32 instructions read of it, a product of two such values is exact
-// in fp32. What does not fit is noticed, and the whole tile then computed by GemmSplit:
-//   - a value that overflows, an infinity, a row whose first slice lies outside 2^-40 .. 2^40;
+// large and keeps all bits of those down to 2^-24 of it; a row of zeros there takes after the rows beside it), and the epilogue
+// scales the sums back: scaling is exact, a truncating conversion to fp16 cuts a value to what the tf32 instructions read of
+// it, a product of two such values is exact in fp32. A row that outgrows its scale gets a smaller one on the way, and its sums with
+// it (`refit`). What does not fit is noticed, and the whole tile then computed by GemmSplit:
+//   - an infinity, a row whose first slice goes beyond 2^40 or that outgrows it by more than 2^38;
 //   - a value below 2^-14 once scaled, which may lose bits below 2^-24. One in some ten million of a random operand does. What
 //     the values of a row lose at most is added up, and the tile is kept if for every single one of its sums this stays below 2^-24 of
 //     the magnitudes of that sum's own products: less than adding them up in fp32 may lose anyway (`hidden`).
@@ -527,6 +528,13 @@ struct GemmSplit {
 // instructions). Measured, expert phase at 8 192 tokens, 64 experts top-2, 2 048 x 2 048: GemmSplit 890 us, this 553 (970 -> 640 us per
 // forward). On the way: both operands in one ring of 12 kilobytes a wavefront, the kernel still spilling, 640; raw rows converted in place
 // in two stages 737; loads to registers one slice ahead 761.
+//
+// What other values cost, us per forward of the same layer, GemmSplit throughout / when one row that outgrew its scale had the whole tile
+// multiplied again / now: random ones 953 / 653 / 620; h with 70, 90, 95 and 99 % zeros 979 / 705 / 718, 934 / 1 022 / 717, 931 / 1 039 / 862,
+// 916 / 1 025 / 1 024; x with a channel 200 times the others 825 / 931 / 645, with six of 100 to 1 000 times 815 / 925 / 671, with 90 %
+// zeros 1 068 / 1 051 / 797, with rows between 2^-20 and 2^20 1 143 / 792 / 773; w_up with 90 % zeros 946 / 1 120 / 729. Behind GELU, whose
+// small values are many, the channel gives 833 before and 853 now. (At 99 % zeros most products of a sum are zero, and the few tiles in which a
+// weight loses bits are not seen to be covered: they are multiplied twice.)
 // ------------------------------------------------------------------------------------------------
 template <int BM, int BN, int WAVES_M, int WAVES_N>
 struct GemmHalf {
@@ -559,7 +567,8 @@ struct GemmHalf {
     static constexpr int kExponents = Split::kSmemBytes;                 // powers of two that scale a sum back: int32 [BM rows | BN columns]
     static constexpr int kLargest = kExponents + (BM + BN) * 4;          // of every scaled row: its largest value (bits of a float)
     static constexpr int kLoss = kLargest + (BM + BN) * 4;               // what its values lose at most, in units of 2^-34 (hidden)
-    static constexpr int kRangeOffset = kLoss + (BM + BN) * 4;           // per bias slot: the Range words
+    static constexpr int kDrops = kLoss + (BM + BN) * 4;                 // by how much its scale has come down since the first slice (exponents)
+    static constexpr int kRangeOffset = kDrops + (BM + BN) * 4;          // per bias slot: the Range words
     static constexpr int kRangeWords = 4 + 2 * kWaves;
     static constexpr int kSmemBytes = kRangeOffset + 2 * kRangeWords * 4;
     static_assert(kConverted + kRings <= 2 * Split::kStage && kWaves * 4096 <= kConverted);
@@ -571,9 +580,9 @@ struct GemmHalf {
         int bias_slot;
     };
 
-    // words of a tile's range: what it holds that calls for a second look, then for every wavefront in which slices (their number
-    // modulo 64, two words) the rows it brings have values that lose bits
-    enum : uint32_t { kSeen = 0, kSlices = 4 };
+    // words of a tile's range: what it holds that calls for a second look, whether a row has outgrown its scale in the slice converted last,
+    // then for every wavefront in which slices (their number modulo 64, two words) the rows it brings have values that lose bits
+    enum : uint32_t { kSeen = 0, kOutgrown = 1, kSlices = 4 };
     enum : uint32_t { kOutOfRange = 1, kLossy = 2, kInDoubt = 4 };
     static __device__ __forceinline__ uint32_t* range_words(char* smem, int bias_slot) {
         return reinterpret_cast<uint32_t*>(smem + kRangeOffset) + bias_slot * kRangeWords;
@@ -659,7 +668,7 @@ struct GemmHalf {
         locate(g, t.rows);
         if ((lane & 7) == 0) {   // written by this wavefront alone, last read by the previous tile in front of a barrier
 #pragma unroll
-            for (int i = 0; i < L; ++i) *row_word(smem, kLargest, i) = 0u;
+            for (int i = 0; i < L; ++i) *row_word(smem, kLargest, i) = *row_word(smem, kDrops, i) = 0u;
         }
         const uint32_t ring = lds_address(smem) + ring_offset();
 #pragma unroll
@@ -697,33 +706,45 @@ struct GemmHalf {
         asm("v_min3_u32 %0, %0, %1, %2" : "+v"(least) : "v"(u[2]), "v"(u[3]));
         *reinterpret_cast<u32x2*>(to) = u32x2{halves(v[0], v[1]), halves(v[2], v[3])};
     }
-    // The scale of the row whose values of the first slice lie in this lane and the seven beside it.
-    static __device__ __forceinline__ int row_exponent(u32x4 raw, uint32_t& flags) {
-        uint32_t largest = 0u;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t word = raw[j] & 0x7fffffffu;
-            largest = word > largest ? word : largest;
-        }
+    static constexpr float kTooLarge = 65536.f;   // (a value of 11 bits below it is one of fp16)
+    // The largest of what the eight lanes of a row hold (bits of a magnitude).
+    static __device__ __forceinline__ uint32_t row_max(uint32_t largest) {
         auto with = [&](uint32_t peer) { largest = peer > largest ? peer : largest; };
         with(row16_peer<0>(largest));
         with(row16_peer<1>(largest));
         with(row16_peer<2>(largest));   // (the three steps combine aligned groups of eight lanes)
-        const int e = int(largest >> 23) - 127;
-        if (largest == 0u) return 0;
-        if (e < -40 || e > 40) { flags |= kOutOfRange; return 0; }
-        return 9 - e;
+        return largest;
+    }
+    static __device__ __forceinline__ int exponent(uint32_t magnitude) { return int(magnitude >> 23) - 127; }
+    // Sums times 2^(row + column), as the array of exponents has them.
+    static __device__ __forceinline__ void scale_sums(Acc& acc, const int* exponents) {
+        const int wave = int(wave_index()), lane = threadIdx.x & 63, wm = wave / WAVES_N, wn = wave % WAVES_N;
+        u32x4 col[TN];
+#pragma unroll
+        for (int ni = 0; ni < TN; ++ni) col[ni] = load16(exponents + BM + wn * WN + ni * 16 + 4 * (lane >> 4));
+#pragma unroll
+        for (int mi = 0; mi < TM; ++mi) {
+            const int row = exponents[wm * WM + mi * 16 + (lane & 15)];
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t c = col[ni][j];
+                    acc[ni][mi][j] = __builtin_amdgcn_ldexpf(acc[ni][mi][j], row + int(c));
+                }
+        }
     }
 
     template <typename Hook>
     static __device__ __forceinline__ void mainloop(const Tile& t, Acc& acc, char* smem, Hook&& after_first_barrier) {
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        const int wave = int(wave_index()), lane = threadIdx.x & 63;
         const int wm = wave / WAVES_N, wn = wave % WAVES_N;
         float scale[L], largest[L];
 #pragma unroll
         for (int i = 0; i < L; ++i) largest[i] = 0.f;
-        uint32_t flags = 0u;
         uint64_t lossy = 0;   // slices (modulo 64) in which a value loses bits
+        auto note_lossy = [&](uint32_t least, uint32_t s) { lossy |= uint64_t(scalar(uint32_t(__builtin_amdgcn_ballot_w64(least < kSmall) != 0u))) << (s & 63u); };
+        uint32_t* const words = range_words(smem, t.bias_slot);
         const uint32_t w = brings_w(), ring = lds_address(smem) + ring_offset();
         const char* const ring_lane = smem + ring_offset() + 16 * lane;
         char* const to = smem + (w ? kABytes : 0) + 512 * loader() + half_offset();
@@ -748,17 +769,46 @@ struct GemmHalf {
             else if constexpr (S == kOne) { if (!w) load(t.rows[i] + first_value(t, s + 1), ring + 1024 * i, 0u); }
         };
         // Kilobytes 0 .. L-1 of slice s, the first of them requested: `between(i)` runs while number i + 1 is on its way.
-        auto convert_slice = [&](auto stage_tag, uint32_t s, auto&& between, auto&& first) {
+        auto convert_slice = [&](auto stage_tag, uint32_t s, auto&& between) {
             uint32_t least = ~0u;
             static_for<L>([&](auto i_tag) {
                 constexpr int i = decltype(i_tag)::value;
                 reload(stage_tag, i_tag, s);
                 if constexpr (i + 1 < L) request(stage_tag, std::integral_constant<int, (i + 1 < L ? i + 1 : 0)>{}, s);
                 between(i);
-                first(i_tag);
                 convert(to + 512 * kLoaders * i, raw[i & 1], scale[i], largest[i], least);
             });
-            lossy |= uint64_t(__builtin_amdgcn_ballot_w64(least < kSmall) != 0u) << (s & 63u);
+            note_lossy(least, s);
+            float most = largest[0];
+#pragma unroll
+            for (int i = 1; i < L; i += 2) asm("v_max3_f32 %0, %0, %1, %2" : "+v"(most) : "v"(largest[i]), "v"(largest[i + 1 < L ? i + 1 : i]));
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(most >= kTooLarge) != 0u, 0)) {
+                if (!(scalar(words[kSeen]) & kOutOfRange)) words[kOutgrown] = 1u;
+            }
+        };
+        // Slice s is converted, and a row has outgrown its scale in it: the row's largest value goes to 2^14 .. 2^15 (one that towers over
+        // the others leaves them the more bits), the slice is converted once more, and kLoss says how the sums follow. Their last place lies at 2^-48 or above, and a row and a column
+        // together come down by 2^76 at most: a sum stays a normal number and keeps its bits. Every wavefront calls it, and meets the others behind it.
+        auto refit = [&](uint32_t s) {
+            uint32_t least = ~0u, flags = 0u;
+            static_for<L>([&](auto i_tag) {
+                constexpr int i = decltype(i_tag)::value;
+                const uint32_t most = row_max(__builtin_bit_cast(uint32_t, largest[i]));
+                int down = __builtin_bit_cast(float, most) >= kTooLarge ? exponent(most) - 14 : 0;
+                uint32_t* const drops = row_word(smem, kDrops, i);
+                if (int(*drops) + down > 38) { flags |= kOutOfRange; down = 0; }   // (an infinity among them)
+                if ((lane & 7) == 0) {
+                    *drops += uint32_t(down);
+                    *row_word(smem, kExponents, i) += uint32_t(down);
+                    *row_word(smem, kLoss, i) = uint32_t(-down);
+                }
+                scale[i] = __builtin_amdgcn_ldexpf(scale[i], -down);
+                largest[i] = __builtin_amdgcn_ldexpf(largest[i], -down);
+                if (scale[i] < 1.f) flags |= kLossy;
+                if (__builtin_amdgcn_ballot_w64(down != 0) != 0u) convert(to + 512 * kLoaders * i, load16(t.rows[i] + first_value(t, s)), scale[i], largest[i], least);
+            });
+            note_lossy(least, s);
+            if (flags) atomicOr(words + kSeen, flags);
         };
         auto stages = [&](uint32_t s, auto&& f) {
             if (s + 2 < t.k_tiles) f(std::integral_constant<int, kBoth>{});
@@ -766,46 +816,82 @@ struct GemmHalf {
             else f(std::integral_constant<int, kNone>{});
         };
         using First = std::integral_constant<int, 0>;
-        // every wavefront has left the previous tile's epilogue, staged where the converted rows go
-        asm volatile("s_barrier" ::: "memory");
+        meet();   // every wavefront has left the previous tile's epilogue, staged where the converted rows go; the tile's words are clear
         stages(0, [&](auto stage_tag) {
+            u32x4 slice0[L];
             request(stage_tag, First{}, 0u);
-            convert_slice(stage_tag, 0u, [](int) {}, [&](auto i_tag) {
+            static_for<L>([&](auto i_tag) {
                 constexpr int i = decltype(i_tag)::value;
-                const int e = row_exponent(raw[i & 1], flags);
-                scale[i] = __builtin_bit_cast(float, uint32_t(e + 127) << 23);
-                if (e < 0) flags |= kLossy;
-                const int row = kRowsPerLoad * (int(loader()) + kLoaders * i) + (lane >> 3);
-                if ((lane & 7) == 0) reinterpret_cast<int*>(smem + kExponents)[(w ? BM : 0) + row] = -e;
+                reload(stage_tag, i_tag, 0u);
+                slice0[i] = raw[i & 1];
+                if constexpr (i + 1 < L) request(stage_tag, std::integral_constant<int, (i + 1 < L ? i + 1 : 0)>{}, 0u);
             });
+            uint32_t row[L], rows = 0u;   // the largest magnitude of the row, and of the wavefront's rows
+#pragma unroll
+            for (int i = 0; i < L; ++i) {
+                row[i] = 0u;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t word = slice0[i][j] & 0x7fffffffu;
+                    row[i] = word > row[i] ? word : row[i];
+                }
+                row[i] = row_max(row[i]);
+                rows = row[i] > rows ? row[i] : rows;
+            }
+#pragma unroll
+            for (int other = 8; other < kWave; other *= 2) {
+                const uint32_t peer = __shfl_xor(rows, other);
+                rows = peer > rows ? peer : rows;
+            }
+            // Zeros say nothing of what follows them: such a row may hold four times the largest value of the rows beside it, or is taken to be
+            // of ordinary size. (Small values in front are left to refit: taken for a sparse row's, they cost rows that are small throughout
+            // more, 772 -> 899 us where rows lie between 2^-20 and 2^20, than they save a layer with 90 % zeros, 717 -> 711.)
+            const int guess = rows != 0u ? exponent(rows) - 4 : 0;
+            uint32_t least = ~0u, flags = 0u;
+            static_for<L>([&](auto i_tag) {
+                constexpr int i = decltype(i_tag)::value;
+                int e = row[i] != 0u ? exponent(row[i]) : guess;
+                if (e > 40) { flags |= kOutOfRange; e = 40; }
+                e = e < -40 ? -40 : e;
+                scale[i] = __builtin_bit_cast(float, uint32_t(9 - e + 127) << 23);
+                if (e > 9) flags |= kLossy;
+                if ((lane & 7) == 0) *row_word(smem, kExponents, i) = uint32_t(e - 9);
+                convert(to + 512 * kLoaders * i, slice0[i], scale[i], largest[i], least);
+            });
+            note_lossy(least, 0u);
+            if (flags) atomicOr(words + kSeen, flags);
         });
         auto top = [&](uint32_t kt) {
             meet();
             if (kt == 0) after_first_barrier();
         };
         auto report = [&] {
+            uint32_t flags = 0u;
             if (lossy != 0u) {
-                flags |= kLossy;
+                flags = kLossy;
                 if (lane < 2) lossy_slices(smem, t.bias_slot)[lane] = uint32_t(lossy >> (32 * lane));
             }
 #pragma unroll
             for (int i = 0; i < L; ++i) {
-                if (largest[i] >= 65536.f) flags |= kOutOfRange;
+                if (largest[i] >= kTooLarge) flags |= kOutOfRange;
                 atomicMax(row_word(smem, kLargest, i), __builtin_bit_cast(uint32_t, largest[i]));
             }
-            if (flags) atomicOr(range_words(smem, t.bias_slot) + kSeen, flags);
+            if (flags) atomicOr(words + kSeen, flags);
         };
-        auto nothing = [](auto) {};
-        if (Split::rows_absent_of(t.g.m_valid, __builtin_amdgcn_readfirstlane(wave) / WAVES_N)) {
+        if (Split::rows_absent_of(t.g.m_valid, wm)) {
             // None of this wavefront's rows exist: it brings and converts its share of every slice between
             // the same barriers, and multiplies nothing.
             for (uint32_t kt = 0; kt < t.k_tiles; ++kt) {
                 top(kt);
+                if (scalar(words[kOutgrown]) != 0u) {
+                    refit(kt);
+                    meet();
+                }
                 if (kt + 1 < t.k_tiles) {
                     asm volatile("s_barrier" ::: "memory");
                     stages(kt + 1, [&](auto stage_tag) {
                         request(stage_tag, First{}, kt + 1);
-                        convert_slice(stage_tag, kt + 1, [](int) {}, nothing);
+                        convert_slice(stage_tag, kt + 1, [](int) {});
                     });
                 }
             }
@@ -816,19 +902,34 @@ struct GemmHalf {
         for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
             for (int mi = 0; mi < TM; ++mi) acc[ni][mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const int fr_row = lane & 15, fr_part = lane >> 4;
-        const int rx = wm * WM + fr_row, rw = wn * WN + fr_row;
-        const char* const from_x = smem + rx * kRowBytes + ((fr_part ^ swizzle(rx)) << 4);
-        const char* const from_w = smem + kABytes + rw * kRowBytes + ((fr_part ^ swizzle(rw)) << 4);
+        // The lane's place in a fragment of 16 rows, the same for all, and the wavefront's first fragments: one vector register through the
+        // main loop, and no more (a spilled one is loaded behind all that is on its way)
+        const uint32_t from = lds_address(smem) + (lane & 15) * kRowBytes + (((lane >> 4) ^ swizzle(lane & 15)) << 4);
         auto slice = [&](uint32_t kt, auto next_tag, auto stage_tag) {
             constexpr bool NEXT = decltype(next_tag)::value;
             top(kt);
             f16x8 fw[TN], fx[TM];
+            auto read = [&] {
+                uint32_t x = uint32_t(wm * WM * kRowBytes), y = uint32_t(kABytes + wn * WN * kRowBytes);
+                asm volatile("" : "+s"(x), "+s"(y));
+                const auto from_x = (const __attribute__((address_space(3))) char*)uintptr_t(from + x), from_w = (const __attribute__((address_space(3))) char*)uintptr_t(from + y);
+                auto load16 = [](const __attribute__((address_space(3))) char* at) { return *(const __attribute__((address_space(3))) u32x4*)at; };
 #pragma unroll
-            for (int ni = 0; ni < TN; ++ni) fw[ni] = __builtin_bit_cast(f16x8, load16(from_w + ni * 16 * kRowBytes));
+                for (int ni = 0; ni < TN; ++ni) fw[ni] = __builtin_bit_cast(f16x8, load16(from_w + ni * 16 * kRowBytes));
 #pragma unroll
-            for (int mi = 0; mi < TM; ++mi) fx[mi] = __builtin_bit_cast(f16x8, load16(from_x + mi * 16 * kRowBytes));
+                for (int mi = 0; mi < TM; ++mi) fx[mi] = __builtin_bit_cast(f16x8, load16(from_x + mi * 16 * kRowBytes));
+            };
+            const uint32_t larger = words[kOutgrown];   // (in front of the fragments, which are waited for anyway)
+            read();
             __builtin_amdgcn_sched_barrier(0);
+            if (__builtin_expect(scalar(larger) != 0u, 0)) {
+                refit(kt);
+                meet();
+                if (threadIdx.x == 0) words[kOutgrown] = 0u;   // everybody has read it; set again behind the next barrier
+                scale_sums(acc, reinterpret_cast<const int*>(smem + kLoss));
+                read();
+                __builtin_amdgcn_sched_barrier(0);
+            }
             auto group = [&](int o) {
 #pragma unroll
                 for (int ni = 0; ni < TN; ++ni) acc[ni][o] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[ni], fx[o], acc[ni][o], 0, 0, 0);
@@ -840,7 +941,7 @@ struct GemmHalf {
                 group(0);
                 __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
                 asm volatile("s_barrier" ::: "memory");
-                convert_slice(stage_tag, kt + 1, [&](int i) { if (i + 1 < TM) group(i + 1); }, nothing);
+                convert_slice(stage_tag, kt + 1, [&](int i) { if (i + 1 < TM) group(i + 1); });
             } else {
 #pragma unroll
                 for (int o = 0; o < TM; ++o) group(o);
@@ -917,46 +1018,22 @@ struct GemmHalf {
     // Whether the losses are covered for sure, without another look at the operands: against the slice that is still in LDS, all values of
     // a row taken to be small in the slices where one that its wavefront brought was. Every wavefront calls it behind the main loop. In
     // loops, as `hidden`: both are rarely called, and take as long as their instructions take to fetch.
-    static __device__ __forceinline__ bool hidden_for_sure(const Tile& t, char* smem) {
-        const uint32_t most = uint32_t(__builtin_popcountll(lossy_of(smem, t.bias_slot))) * ((t.k_tiles + 63u) / 64u) * kSliceK << 10;
+    static __device__ __forceinline__ bool hidden_for_sure(const GemmTileArgs<float>& g, int bias_slot, char* smem) {
+        const uint32_t most = uint32_t(__builtin_popcountll(lossy_of(smem, bias_slot))) * ((g.K / kSliceK + 63u) / 64u) * kSliceK << 10;
 #pragma unroll 1
         for (int i = 0; i < L; ++i) *row_word(smem, kLoss, i) = most;
         meet();
-        return all(covered(t.g, smem, 1), range_words(smem, t.bias_slot), kInDoubt);
+        return all(covered(g, smem, 1), range_words(smem, bias_slot), kInDoubt);
     }
-    // What the small values lost, against four slices spread over K. A function of its own, as `again`.
-    static __device__ __attribute__((noinline)) bool hidden(GemmTileArgs<float> args, uint32_t slot, uint32_t lds) {
-        const GemmTileArgs<float> g = scalar(args);
-        const int bias_slot = int(scalar(slot));
-        char* smem = (char*)(__attribute__((address_space(3))) char*)uintptr_t(scalar(lds));
+    // What the small values lost, against four slices spread over K.
+    static __device__ __forceinline__ bool hidden(const GemmTileArgs<float>& g, int bias_slot, char* smem) {
         const uint32_t k_tiles = g.K / kSliceK;
         const uint64_t lossy = lossy_of(smem, bias_slot);
         const float* rows[L];
         locate(g, rows);
         float scale[L];
-        uint32_t units[L];   // less than 2^-24 a value, and no more than itself
 #pragma unroll
-        for (int i = 0; i < L; ++i) {
-            scale[i] = __builtin_amdgcn_ldexpf(1.f, -int(*row_word(smem, kExponents, i)));
-            units[i] = 0u;
-        }
-        const uint32_t k_first = g.k_first < k_tiles ? g.k_first : 0u;
-#pragma unroll 1
-        for (uint32_t s = 0; s < k_tiles; ++s) {
-            if (!((lossy >> (s & 63u)) & 1u)) continue;
-            const uint32_t slice = s + k_first >= k_tiles ? s + k_first - k_tiles : s + k_first;
-            u32x4 raw[L];
-#pragma unroll
-            for (int i = 0; i < L; ++i) raw[i] = load16(rows[i] + slice * kSliceK);
-#pragma unroll
-            for (int i = 0; i < L; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t word = raw[i][j] & 0x7fffffffu;
-                    const float v = __builtin_bit_cast(float, word) * scale[i];
-                    units[i] += word != 0u && v < 0x1p-14f ? uint32_t(__builtin_fminf(v * 0x1p34f, 1023.f)) + 1u : 0u;
-                }
-        }
+        for (int i = 0; i < L; ++i) scale[i] = __builtin_amdgcn_ldexpf(1.f, -int(*row_word(smem, kExponents, i)));
         constexpr uint32_t kSamples = 4;
         static_assert(int(kSamples) * kConverted <= Split::kBiasOffset);
         const uint32_t samples = k_tiles < kSamples ? k_tiles : kSamples;
@@ -977,22 +1054,54 @@ struct GemmHalf {
                 *reinterpret_cast<u32x2*>(to + q * kConverted + 512 * kLoaders * i) = u32x2{halves(v[0], v[1]), halves(v[2], v[3])};
             }
         }
+        float lost[L];   // less than 2^-24 a value, and no more than itself
 #pragma unroll
-        for (int i = 0; i < L; ++i) {   // the eight lanes of a row
-            units[i] += row16_peer<0>(units[i]);
-            units[i] += row16_peer<1>(units[i]);
-            units[i] += row16_peer<2>(units[i]);
-            if ((threadIdx.x & 7) == 0) *row_word(smem, kLoss, i) = units[i];
+        for (int i = 0; i < L; ++i) lost[i] = 0.f;
+        const uint32_t k_first = g.k_first < k_tiles ? g.k_first : 0u;
+#pragma unroll 1
+        for (uint32_t s = 0; s < k_tiles; ++s) {
+            if (!((lossy >> (s & 63u)) & 1u)) continue;
+            const uint32_t slice = s + k_first >= k_tiles ? s + k_first - k_tiles : s + k_first;
+            u32x4 raw[L];
+#pragma unroll
+            for (int i = 0; i < L; ++i) raw[i] = load16(rows[i] + slice * kSliceK);
+#pragma unroll
+            for (int i = 0; i < L; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t word = raw[i][j];
+                    const float v = __builtin_fabsf(__builtin_bit_cast(float, word) * scale[i]);
+                    lost[i] += v < 0x1p-14f ? __builtin_fminf(v, 0x1p-24f) : 0.f;
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < L; ++i) {   // the eight lanes of a row; rounded up, which covers the rounding of K additions as well
+            lost[i] += row16_peer<0>(lost[i]);
+            lost[i] += row16_peer<1>(lost[i]);
+            lost[i] += row16_peer<2>(lost[i]);
+            if ((threadIdx.x & 7) == 0) *row_word(smem, kLoss, i) = lost[i] > 0.f ? uint32_t(lost[i] * 0x1.04p34f) + 1u : 0u;
         }
         meet();
         return all(covered(g, smem, samples), range_words(smem, bias_slot), kOutOfRange);
     }
 
-    // The tile by GemmSplit. A function of its own: its registers are not those of the main loop's tile.
-    static __device__ __attribute__((noinline)) void again(GemmTileArgs<float> args, uint32_t slot, uint32_t lds) {
+    // The end of a tile whose words call for a second look: its sums if they stand, the tile by GemmSplit if they do not. A function of its own:
+    // its registers are not those of the main loop's tile. The caller lays the sums in memory for it, because the compiler has sums
+    // that live across a call there from the main loop to the epilogue of every tile, called or not: 64 MB per round of
+    // tiles, 785 us per forward of the layer above where this takes 620.
+    static __device__ __attribute__((noinline)) void settle(GemmTileArgs<float> args, uint32_t slot, uint32_t lds, const Acc* sums) {
         const GemmTileArgs<float> g = scalar(args);
         const int bias_slot = int(scalar(slot));
         char* smem = (char*)(__attribute__((address_space(3))) char*)uintptr_t(scalar(lds));
+        if (!(scalar(range_words(smem, bias_slot)[kSeen]) & kOutOfRange) && hidden(g, bias_slot, smem)) {
+            Acc acc;
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int mi = 0; mi < TM; ++mi) acc[ni][mi] = (*sums)[ni][mi];
+            write(g, acc, bias_slot, smem);
+            return;
+        }
         typename Split::Tile t;
         Acc acc;
         Split::begin(t, g, 0, bias_slot, smem);
@@ -1002,42 +1111,26 @@ struct GemmHalf {
         __syncthreads();   // the next tile's loads land where the other wavefronts stage their rows
     }
     static __device__ __forceinline__ void finish(const Tile& t, Acc& acc, char* smem) {
-        uint32_t* words = range_words(smem, t.bias_slot);
-        const uint32_t seen = __builtin_amdgcn_readfirstlane(words[kSeen]);   // the same in every wavefront
-        const bool absent = Split::rows_absent_of(t.g.m_valid, __builtin_amdgcn_readfirstlane(int(local_tid() >> 6)) / WAVES_N);
-        if (__builtin_expect(seen != 0u, 0)) {
-            const uint32_t lds = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem));
-            if ((seen & kOutOfRange) || (!hidden_for_sure(t, smem) && !hidden(t.g, t.bias_slot, lds))) {
-                again(t.g, t.bias_slot, lds);
-                return;
-            }
-        }
-        if (absent) return;
-        if (t.g.act == 0) finish_act<0>(t, acc, smem);
-        else if (t.g.act == 1) finish_act<1>(t, acc, smem);
-        else finish_act<2>(t, acc, smem);
-    }
-    template <int ACT>
-    static __device__ __forceinline__ void finish_act(const Tile& t, Acc& acc, char* smem) {
-        const uint32_t tid = local_tid();
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-        const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-        const int* exponents = reinterpret_cast<const int*>(smem + kExponents);
-        u32x4 col[TN];
-#pragma unroll
-        for (int ni = 0; ni < TN; ++ni) col[ni] = load16(exponents + BM + wn * WN + ni * 16 + 4 * (lane >> 4));
-#pragma unroll
-        for (int mi = 0; mi < TM; ++mi) {
-            const int row = exponents[wm * WM + mi * 16 + (lane & 15)];
+        const uint32_t seen = scalar(range_words(smem, t.bias_slot)[kSeen]);   // the same in every wavefront
+        if (__builtin_expect(seen != 0u && ((seen & kOutOfRange) || !hidden_for_sure(t.g, t.bias_slot, smem)), 0)) {
+            Acc sums;
 #pragma unroll
             for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t c = col[ni][j];
-                    acc[ni][mi][j] = __builtin_amdgcn_ldexpf(acc[ni][mi][j], row + int(c));
-                }
+                for (int mi = 0; mi < TM; ++mi) sums[ni][mi] = acc[ni][mi];
+            settle(t.g, t.bias_slot, uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)), &sums);
+        } else {
+            write(t.g, acc, t.bias_slot, smem);
         }
-        Split::template finish_act<ACT>(TileOut32{t.g.c_base, t.g.ldc, t.g.m_valid, t.g.n_valid}, acc, smem + Split::kBiasOffset + t.bias_slot * Split::kBiasBytes, smem);
+    }
+    static __device__ __forceinline__ void write(const GemmTileArgs<float>& g, Acc& acc, int bias_slot, char* smem) {
+        if (Split::rows_absent_of(g.m_valid, int(wave_index()) / WAVES_N)) return;
+        scale_sums(acc, reinterpret_cast<const int*>(smem + kExponents));
+        const TileOut32 out{g.c_base, g.ldc, g.m_valid, g.n_valid};
+        const char* bias = smem + Split::kBiasOffset + bias_slot * Split::kBiasBytes;
+        if (g.act == 0) Split::template finish_act<0>(out, acc, bias, smem);
+        else if (g.act == 1) Split::template finish_act<1>(out, acc, bias, smem);
+        else Split::template finish_act<2>(out, acc, bias, smem);
     }
 };
 

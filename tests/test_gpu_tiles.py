@@ -424,6 +424,57 @@ def test_tf32_sums_of_small_values_beside_large_sums(small, base, p):
     assert ((got - want).abs() <= 2.0 ** -11 * want + 2.0 ** -19 * magnitude).all()
 
 
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("operand", ["x", "w_up"])
+@pytest.mark.parametrize("rows", ["with a large channel", "starting with zeros", "starting with small values", "growing again and again"])
+def test_tf32_rows_whose_first_values_do_not_stand_for_them(rows, operand, mode):
+    """Rows that outgrow the scale of their first 32 values are scaled anew on the way: the rows (columns) beside them keep
+    their bits, which another order of the sums would change, and every sum is within a place of 11 bits of h and 2^-19 of its
+    products' magnitudes for 16 slices summed in fp32. w_down is the identity, which has h itself read back."""
+    S, H, I = 16384, 512, 512
+    rng = np.random.default_rng(19)
+    x, w_up = torch.from_numpy(rng.standard_normal((S, H))), torch.from_numpy(rng.standard_normal((I, H)))
+
+    def operands(x, w_up):   # 11 significant bits
+        return [(v.float().view(torch.int32) & ~0x1fff).view(torch.float32).double() for v in (x, w_up)]
+    plain = operands(x, w_up)
+    a = x if operand == "x" else w_up
+    some = torch.from_numpy(rng.choice(a.shape[0], a.shape[0] // 5, replace=False))
+    if rows == "with a large channel":
+        a[some, 300] *= 2.0 ** 12
+    elif rows == "starting with zeros":
+        a[some, :200] = 0.0
+        a[some[::2], 200:] *= 8.0
+    elif rows == "starting with small values":
+        a[some, :32] *= 2.0 ** -12
+    else:
+        for at in (33, 100, 101, 479, 480):
+            a[some, at:] *= 2.0 ** 7
+    changed = operands(x, w_up)
+    others = torch.ones(a.shape[0], dtype=torch.bool)
+    others[some] = False
+    keys = _keys(S, H, I, 1, 1, act=0, dt=1)
+    _assert_tiles(keys, (3, 0))
+    got = []
+    ka.initialize(keys)
+    try:
+        _apply(mode)
+        for xs, ws in (plain, changed):
+            iP = torch.cat([xs.flatten(), ws.flatten(), torch.eye(H, dtype=torch.double).flatten(), torch.zeros(H + I).double()]).float().cuda()
+            oP = torch.zeros(S * H, device="cuda")
+            torch.cuda.synchronize()
+            ka.moe.forward_host_dense(iP, oP)
+            ka.moe.stream_synchronize()
+            got.append(oP.view(S, H).cpu())
+    finally:
+        ka.finalize()
+    same = (lambda h: h[others]) if operand == "x" else (lambda h: h[:, others])
+    assert torch.equal(same(got[0]), same(got[1]))
+    for (xs, ws), h in zip((plain, changed), got):
+        want = torch.relu(xs @ ws.T)
+        assert ((h.double() - want).abs() <= 2.0 ** -11 * want + 2.0 ** -19 * (xs.abs() @ ws.abs().T)).all()
+
+
 @pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
 @pytest.mark.parametrize("low,high", [(0.001, 0.1), (0.1, 0.5), (0.5, 1.0), (1.0, 2.0)])
 def test_gelu_keeps_the_bits_of_small_arguments(low, high, sign):
