@@ -475,6 +475,32 @@ def test_tf32_rows_whose_first_values_do_not_stand_for_them(rows, operand, mode)
         assert ((h.double() - want).abs() <= 2.0 ** -11 * want + 2.0 ** -19 * (xs.abs() @ ws.abs().T)).all()
 
 
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("p", [46, 14, -14])
+@pytest.mark.parametrize("S,H,I,E,act", [(16384, 320, 320, 64, 0), (4096, 1088, 1152, 16, 1)])
+def test_tf32_tiles_that_are_scaled_anew_or_computed_again(mode, p, S, H, I, E, act):
+    """Some hidden units 2^p as large, their weights down 2^-p: a layer whose output is of ordinary size, every second expert of which
+    has rows of h (p > 0) or of w_down that outgrow their scale, and for p = 46 weights, and a growth of h, that fp16
+    does not hold: both projections through the bf16 products. Routed tokens, slices that start at another K for
+    every expert, row blocks and wavefronts cut short, biases."""
+    edges = [1, 16, 17, 127, 128, 129, 130, 255, 256, 257, 300, 384, 385, 512]
+    share, rest = divmod(S - sum(edges), E - len(edges))
+    rows = edges + [share + 1] * rest + [share] * (E - len(edges) - rest)
+    keys = _keys(S, H, I, E, 1, cf=2.0, act=act, dt=1)
+    _assert_tiles(keys, (3, 0))
+    c = moe_ref.cfg_from_keys(keys)
+    iP = _one_hot_layer(c, rows, seed=37 + H)
+    at = S * H + c.PX * H
+    w_up, w_down = iP[at:at + E * I * H].reshape(E, I, H), iP[at + E * I * H:at + 2 * E * I * H].reshape(E, H, I)
+    b_up = iP[at + 2 * E * I * H:at + 2 * E * I * H + E * I].reshape(E, I)
+    units = [37, 100, 101, I - 3]
+    w_up[::2, units] *= np.float32(2.0 ** p)
+    b_up[::2, units] *= np.float32(2.0 ** p)
+    w_down[::2, :, units] *= np.float32(2.0 ** -p)
+    _, v, _, _ = check_against_oracle(c, keys, iP, mode)
+    np.testing.assert_array_equal(v["expert_count"], np.array(rows))
+
+
 @pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
 @pytest.mark.parametrize("low,high", [(0.001, 0.1), (0.1, 0.5), (0.5, 1.0), (1.0, 2.0)])
 def test_gelu_keeps_the_bits_of_small_arguments(low, high, sign):
