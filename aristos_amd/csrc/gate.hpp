@@ -227,10 +227,10 @@ __device__ __forceinline__ void gate_unit(const LayerParams& p, uint32_t unit, f
     // More experts, block after block: every wavefront parks the partial sums of its share in LDS, one group of four adds
     // them in ascending order, each lane four experts of every 64, and finishes the block. Softmax and top-k by a single
     // wavefront, whose lanes each held a quarter of a token's experts, were a chain of some 3 000 instructions beside idle
-    // wavefronts, with 2 045 registers spilled at 128 experts. 32-bit Elements, us per forward (256 columns up): 1 024 tokens of
+    // wavefronts, with 2 053 to 2 110 registers spilled at 128 experts. 32-bit Elements, us per forward (256 columns up): 1 024 tokens of
     // 1 024 values, 128 experts top-2, fp32 180 -> 129, 256 experts top-8 307 -> 247; 15 616 tokens of 512 values, 128 experts
     // top-2, fp32 406 -> 298, tf32 391 -> 198, 256 experts top-4, tf32 497 -> 300; 4 096 tokens of 2 048, 256 experts, fp32 542 -> 490.
-    static_assert(NG < 4 || NG % 4 == 0);
+    static_assert(gate_unit_grouped<NG>(KW) || NG % 4 == 0);   // the reads below take whole runs of four groups
     constexpr int NL = (NG + 3) / 4;
     const uint32_t group = uint32_t(wave) >> 2, gtid = threadIdx.x & 255u;
     uint32_t* gsm = reinterpret_cast<uint32_t*>(smem) + group * gate_group_words(p.E, p.k, p.is_training != 0);
