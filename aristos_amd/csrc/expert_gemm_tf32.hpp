@@ -10,7 +10,7 @@
 // 2^-123, whose remainder has bits below the last of a bf16 subnormal (2^-133). A wavefront that finds a NaN among its
 // sums, or sums so small that such lost bits could show in them, computes its part of the tile again on the fp32
 // matrix instructions. (Noticing the lost bits takes 17 of a slice's 364 vector instructions: 953 -> 959 us at the
-// layer below, the mean of two runs.)
+// layer below, the mean of two runs, when every tile was GemmSplit's.)
 #pragma once
 #include "expert_gemm.hpp"
 
@@ -47,10 +47,10 @@ struct TileOut32 {
 //             activation rows, shared by the column tiles of an expert, from the L2)
 //   group 8.. slice kt+1 is split, the weight rows first
 //
-// Measured (8 192 tokens, 64 experts top-2, 2 048 x 2 048): 2 729 us per forward with the 64 x 64 tiles on the
-// fp32 matrix cores, 975 with these; the expert phase takes 870 us, 1 240 TFLOP/s of bf16 products, the rate the
+// Measured with all tiles on it (8 192 tokens, 64 experts top-2, 2 048 x 2 048): 2 729 us per forward with the 64 x 64 tiles on the
+// fp32 matrix cores, 975 with these; the expert phase took 870 us, 1 240 TFLOP/s of bf16 products, the rate the
 // bf16 tiles reach at the compute-bound shapes. Same distance from the layer computed in 64 bits (4.6e-4, the
-// rounding of the rows to tf32).
+// rounding of the rows to tf32). It runs now where GemmHalf's tile does not fit fp16, behind that product.
 // ------------------------------------------------------------------------------------------------
 template <int BM, int BN, int WAVES_M, int WAVES_N>
 struct GemmSplit {
@@ -117,7 +117,7 @@ struct GemmSplit {
         t.m_valid = g.m_valid; t.n_valid = g.n_valid; t.k_tiles = g.K / kSliceK;
         // Known to be scalar, it takes the slices' offsets off the vector unit: 364 instead of 381 vector instructions a
         // slice, 32 registers spilled instead of 48. Against the tree that did not look for lost bits, in turn on one box,
-        // 981 -> 997 us per forward at the layer above without this, 949 -> 958 and 957 -> 959 with it.
+        // 981 -> 997 us per forward at the layer above, all tiles GemmSplit's, without this, 949 -> 958 and 957 -> 959 with it.
         t.k_first = __builtin_amdgcn_readfirstlane(g.k_first < t.k_tiles ? g.k_first : 0u);
         t.act = g.act; t.stage0 = stage0; t.bias_slot = bias_slot;
         const uint32_t k0 = first_value(t, 0), dst = stage_lds(t, smem, 0);

@@ -38,9 +38,10 @@ def test_32_bit_tiles_at_the_edges_of_their_rows(mode, dt, H, I):
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("S,H,I,E,act", [(16384, 320, 320, 64, 0), (4096, 1088, 1152, 16, 1)])
 def test_tf32_tiles_on_the_bf16_matrix_cores(mode, S, H, I, E, act):
-    """256 x 256 tiles whose operands are split in LDS: experts that end around the 128 rows of a wavefront
+    """256 x 256 tiles, whose operands are scaled to fp16 in LDS: experts that end around the 128 rows of a wavefront
     row and the 256 of a tile, a last column tile of 64 and of 128 columns, K of ten slices and more. The
-    products are exact and summed in fp32 as on the fp32 matrix cores: the bounds are those of the other tiles."""
+    products are exact and summed in fp32 as on the fp32 matrix cores: the bounds are those of the other tiles. (The same
+    layers with operands that do not fit fp16: test_tf32_tiles_that_are_scaled_anew_or_computed_again.)"""
     edges = [1, 16, 17, 127, 128, 129, 130, 255, 256, 257, 300, 384, 385, 512]
     share, rest = divmod(S - sum(edges), E - len(edges))
     rows = edges + [share + 1] * rest + [share] * (E - len(edges) - rest)
@@ -49,8 +50,8 @@ def test_tf32_tiles_on_the_bf16_matrix_cores(mode, S, H, I, E, act):
 
 @pytest.mark.parametrize("where", ["x", "w_up", "w_down"])
 def test_tf32_infinities_on_the_bf16_matrix_cores(where):
-    """An infinite operand against operands whose remainder is zero (all are bf16 values): infinities and NaN in the
-    places where sums of the undivided products have them, and everything else as it is."""
+    """An infinite operand, which sends its tiles through the bf16 products, against operands whose remainder is zero there (all
+    are bf16 values): infinities and NaN in the places where sums of the undivided products have them, and everything else as it is."""
     S, H, I = 16384, 512, 512
     rng = np.random.default_rng(7)
     x, w_up, w_down = (torch.from_numpy(rng.standard_normal(n)).to(torch.bfloat16).float() for n in ((S, H), (I, H), (H, I)))
@@ -632,7 +633,7 @@ def test_dense_output_on_every_pair_of_tiles(dt, want, S, H, I):
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("E", [96, 200, 320])
 def test_tf32_large_tiles_with_many_experts(mode, E):
-    """256 x 256 tiles on the bf16 matrix cores with more than 64 experts: their workgroups of eight wavefronts hold two
+    """256 x 256 tiles on the 16-bit matrix cores with more than 64 experts: their workgroups of eight wavefronts hold two
     gate units of four at a time, in each of the three gates above 64 experts."""
     S, H, I = 16384, 128, 320
     keys = _keys(S, H, I, E, 4, cf=2.0, dt=1)
