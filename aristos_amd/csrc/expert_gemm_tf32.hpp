@@ -523,9 +523,10 @@ struct GemmSplit {
 //   group 0   all fragments of slice kt are read; behind a second barrier the converted slice may change
 //   group i   four matrix instructions of slice kt, between the request for eight rows of slice kt+1 and their conversion
 //
-// What bounds it: the weights, which have 64 KB a CU in flight (with all weight tiles read from one place, 460 us of 553), then the
-// LDS, through which a slice passes four times, 256 KB (450 us with the activations resident in L2 as well, 360 without the matrix
-// instructions). Measured, expert phase at 8 192 tokens, 64 experts top-2, 2 048 x 2 048: GemmSplit 890 us, this 553 (970 -> 640 us per
+// What bounds it: the weights, which have 64 KB a CU in flight (with all weight tiles read from one place, 477 us of 549), then the
+// way of a slice through LDS and its conversion (454 us with the activations resident in L2 as well, 419 without the matrix instructions; LDS
+// busy 26 % of the launch, bank conflicts 30 % of that, matrix cores 21 %). Measured, expert phase at 8 192 tokens, 64 experts top-2,
+// 2 048 x 2 048: GemmSplit 890 us, this as first built, with sums spilled behind the main loop, 574, now 549 (970 -> 650 -> 620 us per
 // forward). On the way: both operands in one ring of 12 kilobytes a wavefront, the kernel still spilling, 640; raw rows converted in place
 // in two stages 737; loads to registers one slice ahead 761.
 //
