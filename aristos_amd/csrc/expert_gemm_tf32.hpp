@@ -502,8 +502,9 @@ struct GemmSplit {
 // ------------------------------------------------------------------------------------------------
 // The same tile with one fp16 product instead of four bf16 ones. An fp16 value holds the 11 significant bits of a tf32
 // operand; what it lacks is range. Every row of the tile is therefore scaled by a power of two of its own, chosen from the
-// row's values in the tile's first slice (their largest goes to 2^9 .. 2^10, so that the row may hold values 64 times as
-// large and keeps all bits of those down to 2^-24 of it; a row of zeros there takes after the rows beside it), and the epilogue
+// row's values in the tile's first slice (of an activation row their largest goes to 2^9 .. 2^10, so that the row may hold values 64 times
+// as large and keeps all bits of those down to 2^-24 of it, of a weight row, which is seldom sparse, to 2^12 .. 2^13, 8 times and 2^-27;
+// a row of zeros there takes after the rows beside it), and the epilogue
 // scales the sums back: scaling is exact, a truncating conversion to fp16 cuts a value to what the tf32 instructions read of
 // it, a product of two such values is exact in fp32. A row that outgrows its scale gets a smaller one on the way, and its sums with
 // it (`refit`). What does not fit is noticed, and the whole tile then computed by GemmSplit:
@@ -526,16 +527,17 @@ struct GemmSplit {
 // What bounds it: the weights, which have 64 KB a CU in flight (with all weight tiles read from one place, 477 us of 549), then the
 // way of a slice through LDS and its conversion (454 us with the activations resident in L2 as well, 419 without the matrix instructions; LDS
 // busy 26 % of the launch, bank conflicts 30 % of that, matrix cores 21 %). Measured, expert phase at 8 192 tokens, 64 experts top-2,
-// 2 048 x 2 048: GemmSplit 890 us, this as first built, with sums spilled behind the main loop, 574, now 549 (970 -> 650 -> 620 us per
+// 2 048 x 2 048: GemmSplit 890 us, this as first built, with sums spilled behind the main loop, 574, now 549 (970 -> 650 -> 607 us per
 // forward). On the way: both operands in one ring of 12 kilobytes a wavefront, the kernel still spilling, 640; raw rows converted in place
 // in two stages 737; loads to registers one slice ahead 761.
 //
 // What other values cost, us per forward of the same layer, GemmSplit throughout / when one row that outgrew its scale had the whole tile
-// multiplied again / now: random ones 953 / 653 / 620; h with 70, 90, 95 and 99 % zeros 979 / 705 / 718, 934 / 1 022 / 717, 931 / 1 039 / 862,
-// 916 / 1 025 / 1 024; x with a channel 200 times the others 825 / 931 / 645, with six of 100 to 1 000 times 815 / 925 / 671, with 90 %
-// zeros 1 068 / 1 051 / 797, with rows between 2^-20 and 2^20 1 143 / 792 / 773; w_up with 90 % zeros 946 / 1 120 / 729. Behind GELU, whose
-// small values are many, the channel gives 833 before and 853 now. (At 99 % zeros most products of a sum are zero, and the few tiles in which a
-// weight loses bits are not seen to be covered: they are multiplied twice.)
+// multiplied again / now: random ones 953 / 653 / 607; h with 70, 90, 95 and 99 % zeros 979 / 705 / 660, 934 / 1 022 / 654, 931 / 1 039 / 664,
+// 916 / 1 025 / 807; x with a channel 200 times the others 825 / 931 / 590, with six of 100 to 1 000 times 815 / 925 / 671, with 90 %
+// zeros 1 068 / 1 051 / 763, with rows between 2^-20 and 2^20 1 143 / 792 / 778; w_up with 90 % zeros 946 / 1 120 / 715. Behind GELU, whose
+// small values are many, the channel gives 833 before and 792 now, the six 854 and 877. With weight rows at 2^9 like the others, so that one
+// in twenty tiles holds a weight that loses bits instead of one in 160: 99 % zeros, where most products of a sum are zero and such a
+// loss is not seen to be covered, 1 024, 90 % 717, random values 620, the channel behind GELU 853.
 // ------------------------------------------------------------------------------------------------
 template <int BM, int BN, int WAVES_M, int WAVES_N>
 struct GemmHalf {
@@ -743,6 +745,7 @@ struct GemmHalf {
         float scale[L], largest[L];
 #pragma unroll
         for (int i = 0; i < L; ++i) largest[i] = 0.f;
+        const int target = brings_w() ? 12 : 9;   // the largest value of a row's first slice goes to 2^target
         uint64_t lossy = 0;   // slices (modulo 64) in which a value loses bits
         auto note_lossy = [&](uint32_t least, uint32_t s) { lossy |= uint64_t(scalar(uint32_t(__builtin_amdgcn_ballot_w64(least < kSmall) != 0u))) << (s & 63u); };
         uint32_t* const words = range_words(smem, t.bias_slot);
@@ -847,16 +850,16 @@ struct GemmHalf {
             // Zeros say nothing of what follows them: such a row may hold four times the largest value of the rows beside it, or is taken to be
             // of ordinary size. (Small values in front are left to refit: taken for a sparse row's, they cost rows that are small throughout
             // more, 772 -> 899 us where rows lie between 2^-20 and 2^20, than they save a layer with 90 % zeros, 717 -> 711.)
-            const int guess = rows != 0u ? exponent(rows) - 4 : 0;
+            const int guess = rows != 0u ? exponent(rows) - 13 + target : 0;
             uint32_t least = ~0u, flags = 0u;
             static_for<L>([&](auto i_tag) {
                 constexpr int i = decltype(i_tag)::value;
                 int e = row[i] != 0u ? exponent(row[i]) : guess;
                 if (e > 40) { flags |= kOutOfRange; e = 40; }
                 e = e < -40 ? -40 : e;
-                scale[i] = __builtin_bit_cast(float, uint32_t(9 - e + 127) << 23);
-                if (e > 9) flags |= kLossy;
-                if ((lane & 7) == 0) *row_word(smem, kExponents, i) = uint32_t(e - 9);
+                scale[i] = __builtin_bit_cast(float, uint32_t(target - e + 127) << 23);
+                if (e > target) flags |= kLossy;
+                if ((lane & 7) == 0) *row_word(smem, kExponents, i) = uint32_t(e - target);
                 convert(to + 512 * kLoaders * i, slice0[i], scale[i], largest[i], least);
             });
             note_lossy(least, 0u);
@@ -1089,7 +1092,7 @@ struct GemmHalf {
     // The end of a tile whose words call for a second look: its sums if they stand, the tile by GemmSplit if they do not. A function of its own:
     // its registers are not those of the main loop's tile. The caller lays the sums in memory for it, because the compiler has sums
     // that live across a call there from the main loop to the epilogue of every tile, called or not: 64 MB per round of
-    // tiles, 785 us per forward of the layer above where this takes 620.
+    // tiles, 785 us per forward of the layer above where this took 620.
     static __device__ __attribute__((noinline)) void settle(GemmTileArgs<float> args, uint32_t slot, uint32_t lds, const Acc* sums) {
         const GemmTileArgs<float> g = scalar(args);
         const int bias_slot = int(scalar(slot));

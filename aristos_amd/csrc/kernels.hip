@@ -111,8 +111,8 @@ TileCost tile16_cost(uint32_t bm, uint32_t bn, uint32_t rows) {
 // 256- and 128-row tiles to the smaller ones: 640 tokens, 8 experts top-2, 704 x 512: 58 -> 37 us per forward; 2 176
 // tokens, 16 experts top-2, 2 048 x 512: 91 -> 75; 2 048 tokens, one expert, 1 024 x 4 096: 148 -> 108.
 // tf32: 256 x 256 tiles on the 16-bit matrix cores, 128 clocks per value of K, one on a CU, against 64 x 64 tiles on the fp32 ones,
-// 32 clocks, two on a CU in turn. The large tile takes what it is charged (620 us per forward at 8 192 tokens, 64 experts top-2, 2 048 x
-// 2 048, four rounds: 136 clocks; 272 at 2 048 tokens, 8 experts, one round each way: 123), bound by its loads; the 32 are the small one's
+// 32 clocks, two on a CU in turn. The large tile takes what it is charged (607 us per forward at 8 192 tokens, 64 experts top-2, 2 048 x
+// 2 048, four rounds: 133 clocks; 272 at 2 048 tokens, 8 experts, one round each way: 123), bound by its loads; the 32 are the small one's
 // matrix time, of which it reaches two thirds to three quarters (2 729 and 722 us: 43 and 47 clocks), so the line lies too high. Of
 // 28 layers around it, timed on both, the rule takes the better tile at 17, with all that it gives to the large tile among them (4 096
 // tokens, 8 experts top-2, 1 024 x 1 024: 171 against 392 us; 16 384, 64 experts top-1, 320 x 320: 119 against 132); 11 just below
