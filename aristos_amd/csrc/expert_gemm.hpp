@@ -24,7 +24,7 @@ namespace kleos_amd {
 // instructions run in four equal quarters: one K step each with 32x32x16, half a K step with 16x16x32).
 // With two stages the loads can instead run two slices ahead (AHEAD2): slice kt+2 is requested
 // into the stage of slice kt as soon as every wavefront has read its last fragments of slice kt (a
-// second workgroup barrier per slice, placed before the last quarter, whose matrix instructions
+// second workgroup barrier per slice, inside the third quarter, whose matrix instructions
 // the loads then follow one by one), so the memory pipeline holds requests across the wait for
 // slice kt+1 instead of running empty at every slice boundary.
 //
@@ -119,9 +119,9 @@ __device__ __forceinline__ uint32_t local_tid() {
 }
 
 // Epilogue of a WAVES_M x WAVES_N wavefront grid whose wavefronts each hold a WM x WN block of the
-// C^T accumulators: acc[ni][mi][v] is output column n = wn*WN + ni*32 + 8*(v/4) + 4*(lane/32) + v%4
-// of output row m = wm*WM + mi*32 + lane%32, i.e. a lane owns 4 consecutive columns of 16 rows per
-// 32x32 block. Bias, activation and the rounding to Element happen in registers; the wavefront
+// C^T accumulators, in 16 x 16 matrix-core tiles: acc[ni][mi][v] is output column n = wn*WN + ni*16 + 4*(lane/16) + v
+// of output row m = wm*WM + mi*16 + lane%16, i.e. a lane owns 4 consecutive columns per tile.
+// Bias, activation and the rounding to Element happen in registers; the wavefront
 // then transposes 32-row x 64-column panels through a private LDS region of 4 KB at
 // stage_mem + wave * 4096 (rows of 128 bytes, 16-byte chunk c of row r at position
 // c ^ ((r >> 1) & 7)) so that the global stores are 16 bytes per lane and cover whole 128-byte
@@ -139,63 +139,6 @@ constexpr int kEpiloguePanelRows = 32;
 // both outputs streamed, 2 913 with the intermediate rows alone, 2 953 with the output rows alone);
 // where the rows are read back soon, from the L2 that took them, it costs (64-expert shape 293
 // against 287 us, 16-expert shape 154 against 146 us).
-template <typename E, int WM, int WN, int WAVES_N, int ACT, bool STREAM_OUT>
-__device__ __forceinline__ void epilogue16_act(const TileOut& t, f32x16 (&acc)[WN / 32][WM / 32], char* stage_mem,
-                                               const char* bias_mem) {
-    typedef typename Elem16<E>::vec4 vec4;
-    constexpr int TM = WM / 32, kPanelRows = kEpiloguePanelRows;
-    const uint32_t tid = local_tid();
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const int fr_row = lane & 31, fr_half = lane >> 5;
-    char* stg = stage_mem + wave * (kPanelRows * 128);
-    const char* bias_lane = bias_mem + (wn * WN + 4 * fr_half) * 2;
-#pragma unroll
-    for (int mi = 0; mi < TM; ++mi) {
-#pragma unroll
-        for (int pn = 0; pn < WN / 64; ++pn) {
-#pragma unroll
-            for (int nl = 0; nl < 2; ++nl) {
-                const int ni = pn * 2 + nl;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const vec4 b4 = *reinterpret_cast<const vec4*>(bias_lane + (ni * 32 + 8 * q) * 2);
-                    vec4 o;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        o[j] = static_cast<E>(activate<ACT, E>(acc[ni][mi][4 * q + j] + float(b4[j])));
-                    *reinterpret_cast<vec4*>(stg + fr_row * 128 + (((nl * 4 + q) ^ ((fr_row >> 1) & 7)) << 4) + fr_half * 8) = o;
-                }
-            }
-            // the same wavefront wrote and reads the region: LDS operations of one wavefront
-            // complete in order
-#pragma unroll
-            for (int it = 0; it < kPanelRows * 8 / kWave; ++it) {
-                const int id = it * kWave + lane;
-                const int r = id >> 3, c = id & 7;
-                const u32x4 v = load16(stg + r * 128 + ((c ^ ((r >> 1) & 7)) << 4));
-                const uint32_t m = wm * WM + mi * 32 + r, n = wn * WN + pn * 64 + c * 8;
-                if (m < t.m_valid && n < t.n_valid) {
-                    constexpr int kAgentScope = STREAM_OUT ? 16 + 2 : 16;   // sc1 (+ nt)
-                    // (a tile's rows lie within 2 GiB of its first element: 256 rows of at most 2^22 bytes)
-                    __builtin_amdgcn_raw_buffer_store_b128(v, coherent_rows(t.c_base), int((size_t(m) * t.ldc + n) * sizeof(E)), 0,
-                                                           kAgentScope);
-                }
-            }
-        }
-    }
-}
-template <typename E, int WM, int WN, int WAVES_N, bool STREAM_OUT>
-__device__ __forceinline__ void epilogue16(const TileOut& t, f32x16 (&acc)[WN / 32][WM / 32], char* stage_mem,
-                                           const char* bias_mem) {
-    if (t.act == 0) epilogue16_act<E, WM, WN, WAVES_N, 0, STREAM_OUT>(t, acc, stage_mem, bias_mem);
-    else if (t.act == 1) epilogue16_act<E, WM, WN, WAVES_N, 1, STREAM_OUT>(t, acc, stage_mem, bias_mem);
-    else epilogue16_act<E, WM, WN, WAVES_N, 2, STREAM_OUT>(t, acc, stage_mem, bias_mem);
-}
-
-// The same epilogue for accumulators of 16 x 16 matrix-core tiles: acc[ni][mi][v] is output column
-// n = wn*WN + ni*16 + 4*(lane/16) + v of output row m = wm*WM + mi*16 + lane%16 - again 4 consecutive
-// columns per lane and tile, so the panels, their LDS layout and the stores are the ones above.
 // The matrix cores are idle meanwhile. What bounds it is vector work (an addition, the activation, half a conversion a value,
 // 4 clocks an instruction, two wavefronts a SIMD) and trips to LDS, so the bias is read once and not in front of every panel
 // (behind whose writes the compiler will not move it), and the four reads of a panel are in flight together: 1 900 clocks
@@ -251,6 +194,7 @@ __device__ __forceinline__ void epilogue16_act(const TileOut& t, f32x4 (&acc)[WN
                 const int r = (it * kWave + lane) >> 3, c = lane & 7;
                 const uint32_t m = wm * WM + pm * 32 + r, n = wn * WN + pn * 64 + c * 8;
                 constexpr int kAgentScope = STREAM_OUT ? 16 + 2 : 16;   // sc1 (+ nt)
+                // (a tile's rows lie within 2 GiB of its first element: 256 rows of at most 2^22 bytes)
                 if (m < t.m_valid && n < t.n_valid)
                     __builtin_amdgcn_raw_buffer_store_b128(v[it], rows, int((size_t(m) * t.ldc + n) * sizeof(E)), 0, kAgentScope);
             }
@@ -278,45 +222,20 @@ __device__ __forceinline__ void static_for(F&& f) {
 // neighbour at the same moment), they pass through the L2 without displacing the activation rows
 // that are shared (7.0 against 6.4 TB/s on a read-only stream of this shape).
 // AHEAD2 (two stages only): the loads run two slices ahead, at the price of a second workgroup
-// barrier per slice. It pays where the weights stream from HBM and a slice's loads take longer than
-// its matrix work (headline shape: 301 against 315 us for the expert phase); where the matrix work
-// dominates it needs SPREAD to pay (8-expert shape with hidden size 4096, both projections: 4.18 ms
-// with all loads of a slice at once against 4.11 one slice ahead, 3.95 with them shared out 4 + 4).
-// SPREAD (with AHEAD2): when the loads of a slice are issued. 0: all of them behind the matrix
-// instructions of the last quarter of the slice two before it, which frees their stage. Otherwise
-// only the first of them go there and the rest behind the first quarters of the next slice
-// (spread_count: 1 = 4 + 4, 2 = 3 + 3 + 2 of the 8 loads of a wavefront). The CU's load path takes in
-// about one 1 KB load every 36 clocks while all CUs stream; the 64 loads of a slice issued by eight
-// wavefronts inside one K step queue up in front of it, and each wavefront's matrix instructions sit
-// behind its loads in program order. Shared out evenly over all four K steps the last loads leave too
-// late (4.07 ms at the shape above); one barrier per slice instead of two (the barrier in front of the
-// last K step also standing for "the next slice has landed", its first fragments read behind that K
-// step's matrix instructions) loses the lead time it needs: 3.98 ms.
-#ifndef KLEOS_GEMM_BLOCK_SKIP
-#define KLEOS_GEMM_BLOCK_SKIP 1
-#endif
-// MI: the matrix-core tile. 32: 32x32x16 instructions (16 values of K each, 16 accumulator registers);
+// barrier per slice. The fragments of a slice's second K step are read behind the matrix instructions of the
+// first, so a wavefront has finished with the stage half a slice before it finishes the slice: the barrier that frees the stage
+// sits kReleaseAt matrix instructions into the third quarter (the last reads have returned by then), and the loads of slice kt+2
+// follow it, half of them in the third and half in the last quarter. Every load has between one and one and a half slices to land.
+// MI: the matrix-core tile. 32: 32x32x16 instructions (16 values of K each, 16 accumulator registers), which the gate's product uses;
 // 16: 16x16x32 instructions (32 values of K, 4 accumulator registers). The smaller tile reads and
 // writes half as many accumulator registers per multiply-add and draws less power for the same work
 // (instruction loops on random bf16 operands held in registers, whole device: 2.08 against 1.84
 // PFLOP/s at the same 1.31 kW), which is what bounds these kernels.
-// RELEASE (with AHEAD2 and 16-row matrix tiles, whose slices have two K steps): where the barrier
-// that frees a slice's stage sits. The fragments of the second K step are read behind the matrix
-// instructions of the first, so a wavefront has finished with the stage half a slice before it
-// finishes the slice. 0: the barrier stays in front of the last quarter. 2: it moves into the third
-// quarter, kReleaseAt matrix instructions in (the last reads have returned by then), and the first
-// loads of the slice after the next follow it there: a quarter of a slice more for them to land
-// (8-expert shape with hidden size 4096: 3 088 against 3 115 us per forward; no difference at the
-// 64- and 16-expert shapes). 1: all loads of that slice go behind the early barrier, half in the third
-// and half in the last quarter, none into the next slice: every load has between one and one and a
-// half slices to land (16-expert shape 146 against 150 us, 64-expert shape 284 against 287 us; the
-// 8-expert shape loses, 3 177 against 3 115 us: its loads, bunched into half a slice, hold up the
-// matrix instructions behind them).
 // STREAM_OUT: the output rows are stored with the non-temporal hint (see the epilogue above).
 // GROUPS: more than one when several groups of WAVES_M x WAVES_N wavefronts of a workgroup each run this on
 // LDS of their own (GemmKSplit); the wavefront numbers below are then those within a group.
-template <typename E, int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool STREAM_B, bool AHEAD2, int SPREAD = 0, int MI = 32,
-          int RELEASE = 0, bool STREAM_OUT = false, int GROUPS = 1>
+template <typename E, int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, bool STREAM_B, bool AHEAD2, int MI = 16,
+          bool STREAM_OUT = false, int GROUPS = 1>
 struct Gemm16 {
     typedef E Element;
     static constexpr int kBM = BM, kBN = BN, kWavesN = WAVES_N, kStages = STAGES;
@@ -347,29 +266,12 @@ struct Gemm16 {
     // 16-row tiles, wavefront tiles of four of them in height: a wavefront leaves out the blocks of 16
     // rows that hold no rows of the tile (64-expert shape with skewed routing: the experts' 13 039 rows
     // take the matrix instructions of 13 424 rows that way, of 14 656 with whole wavefronts left out only)
-    static constexpr bool kBlockSkip = KLEOS_GEMM_BLOCK_SKIP != 0 && MI == 16 && TM == 4;
-    static constexpr bool kEarlyRelease = RELEASE == 1;   // every load of a slice behind the early barrier of the slice two before it
-    static constexpr int kReleaseAt = 4;                  // matrix instructions of the third quarter in front of the early barrier
-    static_assert(RELEASE >= 0 && RELEASE <= 2);
-    static_assert(RELEASE == 0 || (AHEAD2 && MI == 16 && kSteps == 2));
+    static constexpr bool kBlockSkip = MI == 16 && TM == 4;
+    static constexpr int kReleaseAt = 4;                  // matrix instructions of the third quarter in front of the barrier that frees the stage
+    static_assert(!AHEAD2 || (MI == 16 && kSteps == 2));
     static constexpr int kQuarters = 4;                            // a slice's matrix instructions in four equal runs
     static constexpr int kPerQuarter = TN * TM * kSteps / kQuarters;
     static constexpr int kPanelRows = kEpiloguePanelRows;          // epilogue staging: 32 rows x 64 columns per wavefront
-    // loads of a slice (per wavefront) issued at the last quarter of the slice two before it [0] and at
-    // quarters 0, 1, 2 of the slice before it [1..3]
-    static constexpr int spread_count(int i) {
-        constexpr int L = LA + LB;
-        switch (SPREAD) {
-            case 1: return i < 2 ? L / 2 : 0;                                                       // 4 4 0 0
-            case 2: return i == 0 || i == 1 ? (3 * L) / 8 : (i == 2 ? L - 2 * ((3 * L) / 8) : 0);   // 3 3 2 0
-            default: return i == 0 ? L : 0;                                                         // all at once
-        }
-    }
-    static constexpr bool kEarlyFirst = RELEASE == 2;     // only the first loads move with the barrier; the others stay in the next slice
-    static_assert(RELEASE != 2 || spread_count(3) == 0, "the third quarter carries no loads of the next slice");
-    static_assert(SPREAD >= 0 && SPREAD <= 2);
-    static_assert(SPREAD == 0 || (AHEAD2 && (LA + LB) % 8 == 0));
-    static_assert(spread_count(0) + spread_count(1) + spread_count(2) + spread_count(3) == LA + LB);
     static_assert(BK == 32 || BK == 64);
     static_assert(MI == 32 || MI == 16);
     static_assert(kQuarters % kSteps == 0 && (TN * TM * kSteps) % kQuarters == 0);
@@ -438,6 +340,48 @@ struct Gemm16 {
         for (int j = 0; j < COUNT; ++j) issue_one(t, sa, sb, k0, FIRST + j);
     }
 
+    // begin() in parts. The load of the bias, by the first wavefront:
+    static __device__ __forceinline__ void load_bias(const GemmTileArgs<elem16_t>& g, int bias_slot, char* smem, uint32_t wave, uint32_t lane) {
+        if (wave == 0 && lane < uint32_t(kBiasBytes / 16)) {
+            const uint32_t n = lane * 8 < g.n_valid ? lane * 8 : 0u;
+            direct_load16<false>(g.bias + n, lds_address(smem) + kBiasOffset + bias_slot * kBiasBytes);
+        }
+    }
+    // Where the lane's 16 bytes of the tile's activation rows `row` come from. The slot->token table was written earlier in the
+    // same launch, possibly on another XCD: device-coherent loads, all in flight together (an index is clamped
+    // to the table it points into, so that no value it could ever hold turns into an address
+    // outside the caller's buffer).
+    static __device__ __forceinline__ void source_rows(const elem16_t* (&pa)[LA], const GemmTileArgs<elem16_t>& g, const uint32_t (&row)[LA], uint32_t ld_p) {
+        uint32_t src[LA];
+#pragma unroll
+        for (int i = 0; i < LA; ++i) src[i] = row[i] < g.m_valid ? row[i] : g.m_valid - 1;
+        if (g.a_row_index) {
+#pragma unroll
+            for (int i = 0; i < LA; ++i) src[i] = uint32_t(load_coherent(g.a_row_index + src[i]));
+#pragma unroll
+            for (int i = 0; i < LA; ++i) src[i] = src[i] < g.a_rows ? src[i] : g.a_rows - 1;
+        }
+#pragma unroll
+        for (int i = 0; i < LA; ++i) {
+            const elem16_t* from = g.a_base + size_t(src[i]) * g.lda;
+            if (g.a_pad && row[i] >= g.m_valid) from = g.a_pad;
+            pa[i] = from + ((ld_p ^ swizzle(row[i])) << 3);
+        }
+    }
+    static __device__ __forceinline__ void weight_rows(const elem16_t* (&pb)[LB], const GemmTileArgs<elem16_t>& g, const uint32_t (&row)[LB], uint32_t ld_p) {
+#pragma unroll
+        for (int i = 0; i < LB; ++i) {
+            const uint32_t r = row[i] < g.n_valid ? row[i] : g.n_valid - 1;
+            pb[i] = g.b_base + size_t(r) * g.ldb + ((ld_p ^ swizzle(row[i])) << 3);
+        }
+    }
+    static __device__ __forceinline__ void describe(Tile& t, const GemmTileArgs<elem16_t>& g, int stage0, int bias_slot) {
+        t.c_base = g.c_base; t.ldc = g.ldc;
+        t.m_valid = g.m_valid; t.n_valid = g.n_valid; t.k_tiles = g.K / BK;
+        t.k_first = g.k_first < t.k_tiles ? g.k_first : 0u;
+        t.act = g.act; t.stage0 = stage0; t.bias_slot = bias_slot;
+    }
+
     // Per-lane source addresses, the load of the bias into LDS slot `bias_slot`, then the loads of
     // the first STAGES-1 slices. Activation rows past the valid range read zeros (a_pad; the last valid
     // row without it) and weight rows past it re-read the last valid row: their products land in
@@ -449,43 +393,15 @@ struct Gemm16 {
         const uint32_t tid = local_tid();
         const int wave = group_wave(__builtin_amdgcn_readfirstlane(tid >> 6)), lane = tid & 63;
         const int ld_r = lane / kChunks, ld_p = lane % kChunks;
-        if (wave == 0 && lane < kBiasBytes / 16) {
-            const uint32_t n = uint32_t(lane) * 8 < g.n_valid ? uint32_t(lane) * 8 : 0u;
-            direct_load16<false>(g.bias + n, lds_address(smem) + kBiasOffset + bias_slot * kBiasBytes);
-        }
-        // The lane's source rows. The slot->token table was written earlier in the same launch,
-        // possibly on another XCD: device-coherent loads, all in flight together (an index is clamped
-        // to the table it points into, so that no value it could ever hold turns into an address
-        // outside the caller's buffer).
-        uint32_t src[LA];
+        load_bias(g, bias_slot, smem, wave, lane);
+        uint32_t arow[LA], brow[LB];
 #pragma unroll
-        for (int i = 0; i < LA; ++i) {
-            const int row = kRowsPerLoad * (wave + kWaves * i) + ld_r;
-            src[i] = row < int(g.m_valid) ? row : g.m_valid - 1;
-        }
-        if (g.a_row_index) {
+        for (int i = 0; i < LA; ++i) arow[i] = kRowsPerLoad * (wave + kWaves * i) + ld_r;
 #pragma unroll
-            for (int i = 0; i < LA; ++i) src[i] = uint32_t(load_coherent(g.a_row_index + src[i]));
-#pragma unroll
-            for (int i = 0; i < LA; ++i) src[i] = src[i] < g.a_rows ? src[i] : g.a_rows - 1;
-        }
-#pragma unroll
-        for (int i = 0; i < LA; ++i) {
-            const int row = kRowsPerLoad * (wave + kWaves * i) + ld_r;
-            const elem16_t* from = g.a_base + size_t(src[i]) * g.lda;
-            if (g.a_pad && row >= int(g.m_valid)) from = g.a_pad;
-            t.pa[i] = from + ((ld_p ^ swizzle(row)) << 3);
-        }
-#pragma unroll
-        for (int i = 0; i < LB; ++i) {
-            const int row = kRowsPerLoad * (wave + kWaves * i) + ld_r;
-            const uint32_t r = row < int(g.n_valid) ? row : g.n_valid - 1;
-            t.pb[i] = g.b_base + size_t(r) * g.ldb + ((ld_p ^ swizzle(row)) << 3);
-        }
-        t.c_base = g.c_base; t.ldc = g.ldc;
-        t.m_valid = g.m_valid; t.n_valid = g.n_valid; t.k_tiles = g.K / BK;
-        t.k_first = g.k_first < t.k_tiles ? g.k_first : 0u;
-        t.act = g.act; t.stage0 = stage0; t.bias_slot = bias_slot;
+        for (int i = 0; i < LB; ++i) brow[i] = kRowsPerLoad * (wave + kWaves * i) + ld_r;
+        source_rows(t.pa, g, arow, ld_p);
+        weight_rows(t.pb, g, brow, ld_p);
+        describe(t, g, stage0, bias_slot);
 #pragma unroll
         for (int st = 0; st < STAGES - 1; ++st)
             if (uint32_t(st) < t.k_tiles) issue_slice(t, smem, st);
@@ -509,7 +425,7 @@ struct Gemm16 {
             // None of this wavefront's rows exist (an expert with few rows): it brings its share of
             // every slice into LDS at the same points of the same sequence of barriers as the others,
             // and leaves the fragment reads and the matrix instructions out.
-            if constexpr (kEarlyRelease) {
+            if constexpr (AHEAD2) {
                 constexpr int L = LA + LB;
                 asm volatile("s_barrier" ::: "memory");
                 if (t.k_tiles > 1) issue_range<0, L>(t, smem, 1);
@@ -521,21 +437,6 @@ struct Gemm16 {
                     if (kt + 2 < t.k_tiles) {
                         asm volatile("s_barrier" ::: "memory");
                         issue_range<0, L>(t, smem, kt + 2);
-                    }
-                }
-            } else if constexpr (AHEAD2) {
-                constexpr int N0 = spread_count(0);
-                asm volatile("s_barrier" ::: "memory");
-                if (t.k_tiles > 1) issue_range<0, N0>(t, smem, 1);
-                for (uint32_t kt = 0; kt < t.k_tiles; ++kt) {
-                    if (kt + 1 < t.k_tiles) wait_vmcnt<N0>();
-                    else wait_vmcnt<0>();
-                    asm volatile("s_barrier" ::: "memory");
-                    if (kt == 0) after_first_barrier();
-                    if (kt + 1 < t.k_tiles) issue_range<N0, LA + LB - N0>(t, smem, kt + 1);
-                    if (kt + 2 < t.k_tiles) {
-                        asm volatile("s_barrier" ::: "memory");
-                        issue_range<0, N0>(t, smem, kt + 2);
                     }
                 }
             } else {
@@ -675,7 +576,7 @@ struct Gemm16 {
             using Q2 = std::integral_constant<int, 2>; using Q3 = std::integral_constant<int, 3>;
             using NoSync = std::integral_constant<int, -1>;
             static_assert(MI == 16 || TN + TM <= kPerQuarter, "the first quarter of a K step has a matrix instruction for every fragment read");
-            if constexpr (kEarlyRelease) {
+            if constexpr (AHEAD2) {
                 // The barrier that frees the stage sits kReleaseAt matrix instructions into the second K step, and
                 // all loads of the slice after the next go out behind it, half in each quarter.
                 constexpr int L = LA + LB;
@@ -699,51 +600,6 @@ struct Gemm16 {
                     const SliceLoads l2 = NEXT2 ? loads_of(kt + 2) : SliceLoads{};
                     quarter(st, Q2{}, l2, None{}, std::integral_constant<int, NEXT2 ? M2 : 0>{}, std::integral_constant<int, NEXT2 ? AT : -1>{});
                     quarter(st, Q3{}, l2, std::integral_constant<int, M2>{}, std::integral_constant<int, NEXT2 ? L - M2 : 0>{}, NoSync{});
-                };
-                const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;   // slices that request slice kt+2
-                for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::true_type{}, std::true_type{});
-                if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::true_type{}, std::false_type{});
-                slice(t.k_tiles - 1, std::false_type{}, std::false_type{});
-            } else if constexpr (AHEAD2) {
-                static_assert(LA + LB <= kPerQuarter, "the loads of a slice fit behind the matrix instructions of one quarter");
-                constexpr int N0 = spread_count(0), N1 = spread_count(1), N2 = spread_count(2), N3 = spread_count(3);
-                // Slice 0 was requested by begin(). Every wavefront has left the previous tile's epilogue,
-                // which staged its output in the stage slice 1 goes to: its first loads go out here, the
-                // others behind the first quarters of slice 0.
-                asm volatile("s_barrier" ::: "memory");
-                if (t.k_tiles > 1) issue_range<0, N0>(t, smem, 1);
-                // One slice: `next_tag` - slice kt+1 exists (its loads N0 .. are issued behind quarters 0 to 2),
-                // `next2_tag` - slice kt+2 exists (its first N0 loads go behind the last quarter, into the
-                // stage of slice kt, once every wavefront has read its last fragments of it).
-                auto slice = [&](uint32_t kt, auto next_tag, auto next2_tag) {
-                    constexpr bool NEXT = decltype(next_tag)::value, NEXT2 = decltype(next2_tag)::value;
-                    // this wavefront's loads of slice kt are complete once only the first N0 of slice kt+1
-                    // are outstanding (the stores of the previous tile's epilogue are older than both)
-                    if constexpr (NEXT) wait_vmcnt<N0>();
-                    else wait_vmcnt<0>();
-                    asm volatile("s_barrier" ::: "memory");   // every wavefront's share of slice kt is in LDS
-                    if (kt == 0) after_first_barrier();
-                    const char* st = smem + stage_of(t, kt) * kStage;
-                    read_fragments(st, 0);
-                    const SliceLoads l1 = NEXT ? loads_of(kt + 1) : SliceLoads{};
-                    quarter(st, Q0{}, l1, std::integral_constant<int, N0>{}, std::integral_constant<int, NEXT ? N1 : 0>{}, NoSync{});
-                    quarter(st, Q1{}, l1, std::integral_constant<int, N0 + N1>{}, std::integral_constant<int, NEXT ? N2 : 0>{}, NoSync{});
-                    if constexpr (kEarlyFirst) {
-                        const SliceLoads l2 = NEXT2 ? loads_of(kt + 2) : SliceLoads{};
-                        quarter(st, Q2{}, l2, std::integral_constant<int, 0>{}, std::integral_constant<int, NEXT2 ? N0 : 0>{},
-                                std::integral_constant<int, NEXT2 ? kReleaseAt : -1>{});
-                        quarter(st, Q3{}, l2, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, NoSync{});
-                        return;
-                    }
-                    quarter(st, Q2{}, l1, std::integral_constant<int, N0 + N1 + N2>{}, std::integral_constant<int, NEXT ? N3 : 0>{}, NoSync{});
-                    if constexpr (NEXT2) {
-                        // this wavefront's last reads of the stage have returned; once that holds for every
-                        // wavefront the stage takes slice kt+2
-                        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-                        asm volatile("s_barrier" ::: "memory");
-                    }
-                    const SliceLoads l2 = NEXT2 ? loads_of(kt + 2) : SliceLoads{};
-                    quarter(st, Q3{}, l2, std::integral_constant<int, 0>{}, std::integral_constant<int, NEXT2 ? N0 : 0>{}, NoSync{});
                 };
                 const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;   // slices that request slice kt+2
                 for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::true_type{}, std::true_type{});
@@ -860,6 +716,193 @@ struct Gemm16 {
         if (rows_absent(t, __builtin_amdgcn_readfirstlane(int(local_tid() >> 6)) / WAVES_N)) return;   // nothing of this wavefront's is stored
         const TileOut out{t.c_base, t.ldc, t.m_valid, t.n_valid, t.act};
         epilogue16<E, WM, WN, WAVES_N, STREAM_OUT>(out, acc, smem + last_stage(t) * kStage, smem + kBiasOffset + t.bias_slot * kBiasBytes);
+    }
+};
+
+// ------------------------------------------------------------------------------------------------
+// The 256 x 256 tile, 2 x 4 wavefronts of 128 x 64, in which the two wavefronts of a SIMD take turns: while one
+// multiplies, the other reads its next fragments from LDS and requests loads. A slice of 64 values of K is two
+// sections of 32 matrix instructions, the upper and the lower half of the wavefront's rows against all of its
+// columns, each behind the LDS reads it needs; wavefronts 4 to 7 run one half section behind wavefronts 0 to 3,
+// which sit on the same SIMDs, and a workgroup barrier ends every half section:
+//
+//     wavefronts 0-3   read 0 | multiply 0 | read 1     | multiply 1 | read 0 of the next slice ...
+//     wavefronts 4-7          | read 0     | multiply 0 | read 1     | multiply 1 ...
+//
+// (Both wavefronts of a SIMD in step, the reads between the matrix instructions, is the main loop of Gemm16 with AHEAD2:
+// its slices begin with reads that nothing covers and its matrix cores are busy 66 % of an 8-expert forward.)
+// Every accumulator takes the two K steps of a section one right behind the other: the second reads the sum where
+// the first leaves it, which takes 5 % less energy (register operands, whole device, both 32 instructions a run: 2 160 against
+// 2 055 TFLOP/s). K is added in the order of Gemm16, so that a row's bits do not depend on the tile that computes it.
+//
+// Two stages. The rows a section reads are free once both groups of wavefronts have read them, and take the slice
+// after the next: the weights and the upper halves' activations behind section 0, the lower halves' behind section 1.
+// Of the 8 loads of a wavefront and slice, 6 go out in section 1 and 2 in section 0 of the next slice, and a wait
+// always leaves the 8 youngest outstanding: every load has a whole slice to land.
+//
+// What bounds it: power, and where it is not reached the ends of a tile. In a loop over the tiles of 8 experts of 2 048 rows (random data) a slice takes 2 240 to
+// 2 400 clocks of which the matrix cores need 2 048, against 2 700 to 2 830 in step; they run at 1.65 GHz instead of 1.8, and
+// the projections of 4 096 x 14 336 take 1 289 + 1 264 us (1 490 + 1 520 TFLOP/s) instead of 1 437 + 1 392, of 2 048 x 2 048 98 instead of 112 each. Four sections
+// of 16 instructions a slice: 1 382 + 1 328, 107. Us per forward: 8 192 tokens, 8 experts top-2, 4 096 x 14 336:
+// 3 085 -> 2 806; 4 608 tokens, 16 experts, 2 048 x 4 096: 371 -> 344; 4 096, 2 048 x 2 048: 146.5 -> 139.5; 8 192, 64 experts,
+// skewed: 281 -> 276.5; 1 280, 8 experts top-1, 4 096 x 7 168: 262 -> 254.
+// ------------------------------------------------------------------------------------------------
+template <typename E, bool STREAM_B>
+struct GemmPingPong : Gemm16<E, 256, 256, 2, 4, 64, 2, STREAM_B, true> {
+    typedef Gemm16<E, 256, 256, 2, 4, 64, 2, STREAM_B, true> Base;
+    typedef typename Base::Tile Tile;
+    typedef typename Base::Acc Acc;
+    typedef typename Base::vec8 vec8;
+    using Base::kStage; using Base::kABytes; using Base::kRowBytes; using Base::kSteps; using Base::WM; using Base::WN; using Base::TM; using Base::TN;
+    static constexpr int kLive = TM / 2;                 // blocks of 16 rows in a section
+    static constexpr int kLoads = 4;                     // loads of a wavefront and slice: as many for the activations as for the weights
+    static_assert(Base::LA == kLoads && Base::LB == kLoads && kSteps == 2 && Base::kWaves == 8 && WM == 128);
+
+    // The first row of the tile that load j of wavefront w covers, 8 rows each: loads 0 and 1 bring the upper halves of the
+    // two wavefront rows, 2 and 3 the lower ones. (Weight rows: as in Gemm16.)
+    static __device__ __forceinline__ uint32_t x_row(uint32_t w, int j) { return uint32_t(j & 1) * WM + uint32_t(j >> 1) * (WM / 2) + 8 * w; }
+    static __device__ __forceinline__ uint32_t w_row(uint32_t w, int j) { return 64 * uint32_t(j) + 8 * w; }
+
+    struct SliceLoads { uint32_t lds, k0; };   // the LDS address of the wavefront's rows in the stage, the first value of K
+    static __device__ __forceinline__ SliceLoads loads_of(const Tile& t, char* smem, uint32_t kt) {
+        uint32_t slice = kt + t.k_first;
+        slice = slice >= t.k_tiles ? slice - t.k_tiles : slice;
+        return SliceLoads{lds_address(smem) + Base::stage_of(t, kt) * kStage + 1024 * wave_index(), slice * Base::kSliceK};
+    }
+    // The loads of a slice that replace what section 0 reads, and those that replace what only section 1 reads.
+    static __device__ __forceinline__ void load_x(const Tile& t, const SliceLoads& l, int j) { direct_load16<false>(t.pa[j] + l.k0, l.lds + x_row(0, j) * kRowBytes); }
+    static __device__ __forceinline__ void load_first(const Tile& t, const SliceLoads& l) {
+        load_x(t, l, 0); load_x(t, l, 1);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) direct_load16<STREAM_B>(t.pb[j] + l.k0, l.lds + kABytes + w_row(0, j) * kRowBytes);
+    }
+    static __device__ __forceinline__ void load_second(const Tile& t, const SliceLoads& l) { load_x(t, l, 2); load_x(t, l, 3); }
+    static constexpr int kFirst = 2 + kLoads, kSecond = 2;   // how many they are
+
+    static __device__ __forceinline__ void begin(Tile& t, const GemmTileArgs<elem16_t>& g, int stage0, int bias_slot, char* smem) {
+        const uint32_t lane = local_tid() & 63, wave = __builtin_amdgcn_readfirstlane(local_tid() >> 6);
+        const uint32_t ld_r = lane / Base::kChunks, ld_p = lane % Base::kChunks;
+        Base::load_bias(g, bias_slot, smem, wave, lane);
+        uint32_t row[kLoads];
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) row[j] = x_row(wave, j) + ld_r;
+        Base::source_rows(t.pa, g, row, ld_p);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) row[j] = w_row(wave, j) + ld_r;
+        Base::weight_rows(t.pb, g, row, ld_p);
+        Base::describe(t, g, stage0, bias_slot);
+        const SliceLoads l = loads_of(t, smem, 0);
+        load_first(t, l);
+        load_second(t, l);
+    }
+
+    // (`after_first_barrier`: as in Gemm16)
+    template <typename Hook>
+    static __device__ __forceinline__ void mainloop(const Tile& t, Acc& acc, char* smem, Hook&& after_first_barrier) {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+        const int wm = wave / Base::kWavesN, wn = wave % Base::kWavesN;
+        const bool behind = wave >= Base::kWaves / 2;   // (a scalar condition: the branches on it hold barriers)
+        auto barrier = [] { asm volatile("s_barrier" ::: "memory"); };
+
+        barrier();   // every wavefront has left the previous tile's epilogue, staged where slice 1 goes
+        if (t.k_tiles > 1) {
+            load_first(t, loads_of(t, smem, 1));
+            wait_vmcnt<kSecond + kFirst>();
+        } else {
+            wait_vmcnt<kSecond>();
+        }
+        barrier();   // what section 0 of slice 0 reads is in LDS
+        after_first_barrier();
+        if (behind) barrier();
+
+        const int fr_row = lane & 15, fr_part = lane >> 4;
+        const int rx = wm * WM + fr_row, rw = wn * WN + fr_row;
+        const int base_x = rx * kRowBytes + ((fr_part ^ Base::swizzle(rx)) << 4);
+        const int base_w = kABytes + rw * kRowBytes + ((fr_part ^ Base::swizzle(rw)) << 4);
+        // Blocks of 16 of the wavefront's rows that the tile has rows in. Only they are multiplied, and a section without any
+        // reads no fragments. A branch around the matrix instructions of a block costs a full tile 8 % of its loop, so that
+        // wavefronts with all their rows run a version without (the same in all lanes, and the same barriers in both).
+        const int rows_here = int(t.m_valid) - wm * WM;
+        const int blocks = rows_here <= 0 ? 0 : (rows_here + 15) / 16;
+        auto body = [&](auto full_tag) {
+            constexpr bool FULL = decltype(full_tag)::value;
+            auto used = [&](int block) { return FULL || block < blocks; };
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int mi = 0; mi < TM; ++mi) acc[ni][mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+            vec8 fx[kSteps][kLive], fw[kSteps][TN];
+            auto read_x = [&](const char* st, int section) {
+                if (!used(section * kLive)) return;
+#pragma unroll
+                for (int ks = 0; ks < kSteps; ++ks)
+#pragma unroll
+                    for (int i = 0; i < kLive; ++i)
+                        fx[ks][i] = __builtin_bit_cast(vec8, load16(st + (base_x ^ (ks << 6)) + (section * kLive + i) * 16 * kRowBytes));
+            };
+            auto read_w = [&](const char* st) {
+                if (!used(0)) return;
+#pragma unroll
+                for (int ks = 0; ks < kSteps; ++ks)
+#pragma unroll
+                    for (int i = 0; i < TN; ++i) fw[ks][i] = __builtin_bit_cast(vec8, load16(st + (base_w ^ (ks << 6)) + i * 16 * kRowBytes));
+            };
+            auto product = [&](int ni, int i, int section) {
+#pragma unroll
+                for (int ks = 0; ks < kSteps; ++ks) {
+                    acc[ni][section * kLive + i] = Elem16<E>::mfma16(fw[ks][ni], fx[ks][i], acc[ni][section * kLive + i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            // The half section that multiplies, and the barriers around it. The reads have returned in front of the first of
+            // them: behind it, loads may replace what they read.
+            auto multiply = [&](int section) {
+                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+                __builtin_amdgcn_sched_barrier(0);
+                barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_setprio(1);        // ahead of the reads and loads of the SIMD's other wavefront
+                if constexpr (FULL) {
+#pragma unroll
+                    for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                        for (int i = 0; i < kLive; ++i) product(ni, i, section);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < kLive; ++i)
+                        if (used(section * kLive + i)) {
+#pragma unroll
+                            for (int ni = 0; ni < TN; ++ni) product(ni, i, section);
+                        }
+                }
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_sched_barrier(0);
+                barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            // LATER: slices behind this one, 2 standing for any number from there on. Its wait leaves outstanding what the
+            // next section does not read.
+            auto slice = [&](uint32_t kt, auto later_tag) {
+                constexpr int LATER = decltype(later_tag)::value;
+                const char* st = smem + Base::stage_of(t, kt) * kStage;
+                read_w(st);
+                read_x(st, 0);
+                if constexpr (LATER >= 1) load_second(t, loads_of(t, smem, kt + 1));
+                wait_vmcnt<(LATER >= 1 ? kFirst + kSecond : 0)>();
+                multiply(0);
+                read_x(st, 1);
+                if constexpr (LATER >= 2) load_first(t, loads_of(t, smem, kt + 2));
+                if constexpr (LATER >= 1) wait_vmcnt<(LATER >= 2 ? kSecond + kFirst : kSecond)>();
+                multiply(1);
+            };
+            const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;
+            for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::integral_constant<int, 2>{});
+            if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::integral_constant<int, 1>{});
+            slice(t.k_tiles - 1, std::integral_constant<int, 0>{});
+        };
+        if (blocks >= TM) body(std::true_type{});
+        else body(std::false_type{});
+        if (!behind) barrier();
     }
 };
 

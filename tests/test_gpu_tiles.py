@@ -601,6 +601,20 @@ def test_every_pair_of_16_bit_tiles_at_the_edges_of_its_rows(mode, dt, want, S, 
     np.testing.assert_array_equal(v["expert_count"], np.array(rows))
 
 
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("H,I", [(64, 128), (128, 64), (192, 320), (256, 64)])
+def test_large_tiles_of_few_slices(mode, dt, H, I):
+    """256 x 256 tiles whose loads end while the first slices are multiplied: one to five slices of K, with experts that
+    end inside the upper and the lower half of a wavefront's rows and between them."""
+    rows = [17, 193, 241, 256, 433, 700, 1025, 2255]
+    keys = _keys(sum(rows), H, I, len(rows), 1, cf=4.0, act=0, dt=dt)
+    _assert_tiles(keys, (2, 0))
+    c = moe_ref.cfg_from_keys(keys)
+    _, v, _, _ = check_against_oracle(c, keys, _one_hot_layer(c, rows, seed=H + I), mode)
+    np.testing.assert_array_equal(v["expert_count"], np.array(rows))
+
+
 @pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("want,S,H,I", [((2, 0), 6272, 704, 704), ((2, 1), 4224, 1088, 1216), ((4, 0), 3072, 64, 704), ((4, 1), 1152, 64, 8192),
                                         ((4, 1), 2176, 192, 4160), ((5, 0), 640, 320, 192)],
