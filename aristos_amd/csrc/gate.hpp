@@ -609,21 +609,24 @@ __device__ __forceinline__ void gate_reduce_group(const LayerParams& p, uint32_t
     if (valid) {
         const uint32_t token = tile * kGateTileTokens + tl;
         const coherent_rows_t partial = coherent_rows(p.gate_partial);
-        // range by range, in ascending order; the loads of two ranges in flight together
-        for (uint32_t s0 = 0; s0 < p.gate_splits; s0 += 2) {
-            u32x4 v[2][NL];
+        // range by range, in ascending order; the loads of eight ranges in flight together (two at a time the sixteen ranges of 128 tokens of 7 168
+        // values, 256 experts, were eight trips to memory)
+        constexpr uint32_t kRanges = 8;
+        for (uint32_t s0 = 0; s0 < p.gate_splits; s0 += kRanges) {
+            u32x4 v[kRanges][NL];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+            for (uint32_t u = 0; u < kRanges; ++u) {
                 const uint32_t s = s0 + u < p.gate_splits ? s0 + u : s0;
                 const uint32_t row = ((s * p.S + token) * p.PX + 4 * sub) * 4u;
 #pragma unroll
-                for (int j = 0; j < NL; ++j) v[u][j] = uint32_t(64 * j) < p.PX ? load16_coherent(partial, row + 256u * j) : u32x4{0, 0, 0, 0};
+                for (int j = 0; j < NL; ++j) v[u][j] = uint32_t(64 * j) < p.PX && s0 + u < p.gate_splits ? load16_coherent(partial, row + 256u * j) : u32x4{0, 0, 0, 0};
             }
 #pragma unroll
-            for (int j = 0; j < NL; ++j) acc[j] += __builtin_bit_cast(f32x4, v[0][j]);
-            if (s0 + 1 < p.gate_splits) {
+            for (uint32_t u = 0; u < kRanges; ++u) {
+                if (s0 + u < p.gate_splits) {
 #pragma unroll
-                for (int j = 0; j < NL; ++j) acc[j] += __builtin_bit_cast(f32x4, v[1][j]);
+                    for (int j = 0; j < NL; ++j) acc[j] += __builtin_bit_cast(f32x4, v[u][j]);
+                }
             }
         }
     }
@@ -787,32 +790,41 @@ __device__ __forceinline__ void gate_reduce_tile_wide(const LayerParams& p, uint
     gate_wide_epilogue<T>(p, tile, smem, lane);
 }
 
-// Slot assignment for one 16-token tile per wavefront. Every thread of the workgroup must call it
-// (it contains workgroup barriers); a wave without work passes valid = false. `base` is LDS
-// scratch of E uint32 private to the calling wave. Must run after every gate tile has finished
+// Slot assignment for one 16-token tile, by a group of `gsize` threads (whole wavefronts). Every thread of the workgroup must call
+// it (it contains workgroup barriers); a group without work passes valid = false. `part` is LDS scratch of
+// slot_tile_words(E, gsize) words private to the group. Must run after every gate tile has finished
 // and released its results; what the gate tiles wrote is read with device-coherent loads.
 //   slot = (tokens routed to e in all earlier tiles) + (rank inside this tile); a token keeps its
 //   expert iff slot < EC (gate.cuh:710-716).
-__device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, bool valid,
-                                          uint32_t* base) {
-    const int lane = threadIdx.x & 63;
+// What bounds it: trips to memory that other XCDs wrote, well over a microsecond each. The rows of counts before a tile (31 of its
+// block and the coarse ones) are shared out over up to eight threads per expert (SHARED), so that they are one trip or two; by a single wavefront, 64
+// experts after the other, they were eight with 256 experts. Up to 64 experts a single wavefront's two trips are the shorter way (the
+// shares cost a sum per pair and more code, all of it executed once: 8 192 tokens, 64 experts: 8.3 us for the phase, 8.9 shared out).
+// The phase with its barrier, with 256 experts: 128 tokens top-8 29 -> 8 us, 4 096 38 -> 12. Us per forward: 2 048 tokens, 128 experts
+// top-3, 448 x 448: 72 -> 61; 1 280, 256 experts top-2, 2 304 x 576: 311 -> 284; 384, 128 experts top-2, 4 544 x 704: 331 -> 318.
+__host__ __device__ inline uint32_t slot_tile_words(uint32_t E, uint32_t gsize) { return E > gsize ? E : gsize; }
+template <bool SHARED>
+__device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, bool valid, uint32_t* part, uint32_t gtid, uint32_t gsize) {
     const uint32_t E = p.E;
     const uint32_t* super = p.super_count + size_t(p.epoch & 1u) * p.n_super * E;
-    // The tile's (token, expert) pairs are requested first: they do not depend on the counts, and
-    // every dependent round trip to memory written by other XCDs costs more than a microsecond.
+    // The tile's (token, expert) pairs are requested first: they do not depend on the counts.
     const uint32_t pairs = kGateTileTokens * p.k;
-    constexpr uint32_t kInline = 4;            // pairs per lane kept in registers (k <= 16)
+    constexpr uint32_t kInline = 4;            // pairs per thread kept in registers
     uint32_t pe[kInline];
     int32_t pr[kInline];
 #pragma unroll
     for (uint32_t u = 0; u < kInline; ++u) {
-        const uint32_t i = lane + u * kWave;
+        const uint32_t i = gtid + u * gsize;
         pe[u] = 0; pr[u] = 0;
         if (valid && i < pairs) {
             pe[u] = uint32_t(load_coherent(p.topk_expert + size_t(tile) * pairs + i));
             pr[u] = load_coherent(p.topk_slot + size_t(tile) * pairs + i);
         }
     }
+    // expert e's rows of counts: thread e of every run of 2^lg threads, run g taking the rows g, g + runs, ...
+    constexpr uint32_t kRuns = 8;
+    const uint32_t lg = SHARED && E > 1 ? 32u - uint32_t(__builtin_clz(E - 1)) : 0u;
+    const uint32_t most = SHARED ? gsize >> lg : 1u, runs = most > kRuns ? kRuns : (most ? most : 1u), g = runs > 1 ? gtid >> lg : 0u;
     if (valid) {
         const uint32_t sup = tile / kSuperTiles;
         const uint32_t first = sup * kSuperTiles;
@@ -823,19 +835,22 @@ __device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, b
         auto row_ptr = [&](uint32_t r) {
             return r < sup ? super + size_t(r) * E : p.tile_count + size_t(first + (r - sup)) * E;
         };
-        for (uint32_t e = lane; e < E; e += kWave) {
+        for (uint32_t e = runs > 1 ? gtid & ((1u << lg) - 1u) : gtid; e < E && g < runs; e += runs > 1 ? E : gsize) {
             uint32_t acc = 0;
             constexpr uint32_t kBatch = 16;
-            for (uint32_t r0 = 0; r0 < n; r0 += kBatch) {
+            for (uint32_t r0 = g; r0 < n; r0 += kBatch * runs) {
                 uint32_t v[kBatch];
 #pragma unroll
-                for (uint32_t u = 0; u < kBatch; ++u) v[u] = load_coherent(row_ptr(r0 + u < n ? r0 + u : n - 1) + e);
+                for (uint32_t u = 0; u < kBatch; ++u) {
+                    const uint32_t r = r0 + u * runs;
+                    v[u] = load_coherent(row_ptr(r < n ? r : n - 1) + e);
+                }
 #pragma unroll
-                for (uint32_t u = 0; u < kBatch; ++u) acc += r0 + u < n ? v[u] : 0u;
+                for (uint32_t u = 0; u < kBatch; ++u) acc += r0 + u * runs < n ? v[u] : 0u;
             }
-            base[e] = acc;
-            // training: the wavefront of a block's first tile also sums the block's probability rows
-            if (p.is_training && tile == first) {
+            part[g * E + e] = acc;
+            // training: the group of a block's first tile also sums the block's probability rows
+            if (p.is_training && tile == first && g == 0) {
                 const uint32_t rows = p.n_gate_tiles - first < uint32_t(kSuperTiles) ? p.n_gate_tiles - first
                                                                                       : uint32_t(kSuperTiles);
                 float total = 0.f;
@@ -849,9 +864,6 @@ __device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, b
                 }
                 store_through(p.super_prob + size_t(sup) * E + e, total);
             }
-            // total routed per expert, dropped tokens included (the reference's eC, gate.cuh:699)
-            if (tile + 1 == p.n_gate_tiles)
-                store_through(p.expert_count + e, acc + load_coherent(p.tile_count + size_t(tile) * E + e));
         }
     }
     __syncthreads();
@@ -860,15 +872,16 @@ __device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, b
             const size_t idx = size_t(tile) * pairs + i;
             const uint32_t token = tile * kGateTileTokens + i / p.k;
             if (e >= E) e = E - 1;   // cannot happen; keeps every address below inside its table
-            const uint32_t slot = base[e] + uint32_t(rank);
+            uint32_t slot = uint32_t(rank);
+            for (uint32_t r = 0; r < runs; ++r) slot += part[r * E + e];
             const bool keep = slot < p.EC && slot < p.cap_rows;
             store_through(p.topk_slot + idx, keep ? int32_t(slot) : -1);
             if (keep) store_through(p.slot_token + size_t(e) * p.cap_rows + slot, int32_t(token));
         };
 #pragma unroll
         for (uint32_t u = 0; u < kInline; ++u)
-            if (lane + u * kWave < pairs) assign(lane + u * kWave, pe[u], pr[u]);
-        for (uint32_t i = lane + kInline * kWave; i < pairs; i += kWave)
+            if (gtid + u * gsize < pairs) assign(gtid + u * gsize, pe[u], pr[u]);
+        for (uint32_t i = gtid + kInline * gsize; i < pairs; i += gsize)
             assign(i, uint32_t(load_coherent(p.topk_expert + size_t(tile) * pairs + i)),
                    load_coherent(p.topk_slot + size_t(tile) * pairs + i));
     }

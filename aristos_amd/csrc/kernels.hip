@@ -18,7 +18,9 @@ __global__ __launch_bounds__(kPhaseThreads) void slot_kernel(const LayerParams p
     extern __shared__ uint32_t slot_smem[];
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t tile = blockIdx.x * 4 + wave;
-    slot_tile(p, tile, tile < p.n_gate_tiles, slot_smem + wave * p.E);
+    slot_tile<false>(p, tile, tile < p.n_gate_tiles, slot_smem + wave * slot_tile_words(p.E, kWave), threadIdx.x % kWave, kWave);
+    if (blockIdx.x == 0)
+        for (uint32_t e = threadIdx.x; e < p.E; e += kPhaseThreads) p.expert_count[e] = routed_count(p, e);
     // the coarse counts of the other epoch are free now: clear them for the next launch
     uint32_t* other = p.super_count + size_t((p.epoch & 1u) ^ 1u) * p.n_super * p.E;
     for (uint32_t i = blockIdx.x * kPhaseThreads + threadIdx.x; i < p.n_super * p.E; i += gridDim.x * kPhaseThreads)
@@ -228,7 +230,7 @@ hipError_t launch_gate(const LayerParams& p, int dtype, int num_cus, hipStream_t
 
 hipError_t launch_slots(const LayerParams& p, hipStream_t s) {
     const uint32_t grid = ceil_div_u32(p.n_gate_tiles, 4);
-    hipLaunchKernelGGL(slot_kernel, dim3(grid), dim3(kPhaseThreads), 4 * p.E * sizeof(uint32_t), s, p);
+    hipLaunchKernelGGL(slot_kernel, dim3(grid), dim3(kPhaseThreads), 4 * slot_tile_words(p.E, kWave) * sizeof(uint32_t), s, p);
     return hipGetLastError();
 }
 

@@ -179,6 +179,28 @@ def test_gate_of_many_experts_in_32_bits(dt, S, H, E, k):
     np.testing.assert_allclose(g["mean_prob"], ref["mean_prob"], rtol=3e-5, atol=1e-8)
 
 
+@pytest.mark.parametrize("dt,S,E,k", [
+    (2, 8320, 65, 2),             # a workgroup's slot tiles by four groups of two wavefronts; queues of eight experts, one of nine
+    (2, 4224, 128, 3),            # by two groups of four; every queue full
+    (3, 128, 256, 8),             # by the whole workgroup, two threads per expert's counts
+    (2, 640, 257, 2),             # more experts than a group of the gate takes
+    (2, 1152, 512, 4),            # a thread per expert's counts, queues of 64 experts
+    (0, 4224, 96, 2),             # workgroups of four wavefronts, two queues each
+    (1, 1152, 300, 5),            # more experts than threads
+], ids=lambda v: str(v))
+def test_slots_and_queues_of_many_experts(dt, S, E, k):
+    """Above 64 experts the counts of a slot tile are shared out over a group's threads and the queues are made a wavefront
+    each: slots against the oracle, the same bits in every launch mode and under both schedules."""
+    keys = _keys(S, 64, 64, E, k, cf=1.25, dt=dt)
+    c = moe_ref.cfg_from_keys(keys)
+    iP = pack_inputs(c, *random_layer(c, seed=S + E, w_std=0.05, bias_std=0.1))
+    got = [check_against_oracle(c, keys, iP, mode, launches=2)[1:3] for mode in MODES]
+    for v, out in got[1:]:
+        for name in ("topk_slot", "expert_count"):
+            np.testing.assert_array_equal(v[name], got[0][0][name])
+        np.testing.assert_array_equal(out, got[0][1])
+
+
 @pytest.mark.parametrize("dt,S,H,I", [(2, 128, 64, 64), (2, 2048, 320, 448), (3, 1152, 192, 1216), (0, 640, 128, 320), (1, 2304, 1088, 1152)])
 def test_dense_forward_leaves_the_routing_out(dt, S, H, I):
     """One expert in the dense packing: rows are tokens, nothing is routed. The bits of a routed forward, also between
