@@ -7,7 +7,7 @@
 //     shuffle work; the reference bounces the accumulator through shared memory to get one
 //     thread per token (gate.cuh:560-572);
 //   * every expert count is handled inside one workgroup: up to 256 experts with the logits in
-//     registers, more in passes of 256 with the logits read back from memory (the reference chains
+//     registers, more in passes of 256 (the reference chains
 //     64-expert blocks through global-memory mailboxes, gate.cuh:93-468);
 //   * slots are assigned in token order from per-tile histograms and their prefix sums, which
 //     makes dropping deterministic; the reference takes a tile's base slot from atomicAdd arrival
@@ -50,9 +50,9 @@ constexpr int kGateParkStride = kWave + 1;
 template <int NG>
 constexpr int gate_smem_floats(int kw) {
     if (gate_unit_grouped<NG>(kw)) return 2 * kw * NG * 4 * kGateParkStride + (kw / 4) * int(kGateTileTokens * 64 + 64 + kGateTileTokens * 64);
-    return kw * (NG == 0 ? 16 * kWave : NG * kGateParkStride) * 4;
+    return kw * (NG == 0 ? 16 : NG) * kGateParkStride * 4;
 }
-constexpr uint32_t kWideGateMaxK = 32;   // the wide gate keeps a tile's 16 * k picks in LDS
+constexpr uint32_t kWideGateMaxK = 32, kWideGateMaxE = 512;   // of the gate of more than 256 experts
 
 // Sums of the K steps s0 .. s1-1 of TB token blocks against NG groups of 16 experts, from zero: logits^T, experts are
 // the matrix-core rows, tokens its columns (gate.cuh:526-534). `xrow`, `wrow`: the lane's own row at its chunk of a step.
@@ -358,23 +358,17 @@ __device__ __forceinline__ void gate_spread(const LayerParams& p, uint32_t ways,
     }
 }
 
-template <typename T>
-__device__ __forceinline__ void gate_wide_epilogue(const LayerParams& p, uint32_t tile, float* smem, int lane);
-
-// The gate for more than 256 experts: one 16-token block per unit, the experts in passes of 256.
-// Every pass is the K loop and the reduction of gate_unit with 16 groups; wavefront 0 stores the
-// pass's logits, and when all passes are done it reads them back for softmax and top-k (each lane
-// reads exactly the words it stored). Selection needs no record of what was picked: round r takes
-// the largest logit that comes after the previous pick in the order (logit descending, expert
-// ascending), which is the same k rounds of arg-max with ties to the lower index
-// (gate.cuh:654-670). The tile's picks go through LDS for the in-tile ranks and the histogram.
+// The gate of 32-bit Elements for more than 256 experts: one 16-token block per unit, the experts in passes of 256.
+// Every pass is the K loop of gate_unit with 16 groups; a group of four wavefronts adds the shares in ascending order, keeps them (each
+// lane four experts of every 64) and finishes the block when all passes are done. Before, one wavefront stored the logits and read them
+// back once and more for every pick, alone in its workgroup: 4 992 tokens of 256 values, 360 experts top-4, tf32: 221 us of 1 062.
 // Every thread of the workgroup must call the function; `smem` holds gate_smem_floats<0>(KW) floats.
 template <typename T, int KW>
 __device__ __forceinline__ void gate_unit_wide(const LayerParams& p, uint32_t unit, float* smem) {
-    constexpr int NG = 16;
+    constexpr int NG = 16, kPasses = int(kWideGateMaxE) / (16 * NG), NL = kPasses * NG / 4;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)) % KW, lane = threadIdx.x & 63;
     const int col = lane & 15, chunk = lane >> 4;
-    const uint32_t H = p.H, E = p.E;
+    const uint32_t H = p.H;
     constexpr int kStepK = GateK<T>::kStepK;
     constexpr int kPer = GateK<T>::kElemsPer16B;
     const uint32_t steps = H / kStepK;
@@ -384,9 +378,16 @@ __device__ __forceinline__ void gate_unit_wide(const LayerParams& p, uint32_t un
     const bool live = tile < p.n_gate_tiles;
     const uint32_t token = (live ? tile : p.n_gate_tiles - 1) * kGateTileTokens + col;
     const T* xrow = static_cast<const T*>(p.x) + size_t(token) * H + chunk * kPer;
-    float* my_logits = p.logits + size_t(token) * E;
+    const uint32_t group = uint32_t(wave) >> 2, gtid = threadIdx.x & 255u;
+    const int sub = lane & 15;                              // experts 64 j + 4 sub .. + 3
+    const int tl = 4 * (wave & 3) + (lane >> 4);            // token inside the block
+    const bool mine = live && group == 0;
+    constexpr int kShare = NG * 4 * kGateParkStride;
+    f32x4 sum[NL];
 
-    for (uint32_t e0 = 0; e0 < E; e0 += 16 * NG) {
+#pragma unroll
+    for (int pass = 0; pass < kPasses; ++pass) {
+        const uint32_t e0 = uint32_t(pass) * 16 * NG;
         f32x4 acc[NG];
 #pragma unroll
         for (int g = 0; g < NG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -395,171 +396,38 @@ __device__ __forceinline__ void gate_unit_wide(const LayerParams& p, uint32_t un
             const uint32_t r = e0 + 16 * g + col;
             return static_cast<const T*>(p.wg) + size_t(r < p.PX ? r : p.PX - 1) * H + chunk * kPer;
         };
-        // the loads of U steps are issued together before their matrix instructions
-        constexpr int U = 2;
-        uint32_t s = s0;
-        for (; s + U <= s1; s += U) {
-            u32x4 xb[U], wa[U][NG];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t off = (s + u) * kStepK;
-                xb[u] = load16(xrow + off);
-#pragma unroll
-                for (int g = 0; g < NG; ++g) wa[u][g] = load16(wrow(g) + off);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int g = 0; g < NG; ++g) acc[g] = mma16_step(wa[u][g], xb[u], acc[g], T{});
-        }
-        for (; s < s1; ++s) {
+        for (uint32_t s = s0; s < s1; ++s) {
             const uint32_t off = s * kStepK;
             const u32x4 xb = load16(xrow + off);
+            u32x4 wa[NG];
 #pragma unroll
-            for (int g = 0; g < NG; ++g) acc[g] = mma16_step(load16(wrow(g) + off), xb, acc[g], T{});
+            for (int g = 0; g < NG; ++g) wa[g] = load16(wrow(g) + off);
+#pragma unroll
+            for (int g = 0; g < NG; ++g) acc[g] = mma16_step(wa[g], xb, acc[g], T{});
         }
-        float* dst = smem + part * (NG * 4 * kWave);
+        float* dst = smem + part * kShare;
 #pragma unroll
         for (int g = 0; g < NG; ++g)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) dst[(g * 4 + v) * kWave + lane] = acc[g][v];
+            for (int v = 0; v < 4; ++v) dst[(g * 4 + v) * kGateParkStride + lane] = acc[g][v];
         __syncthreads();
-        if (wave == 0 && live) {
 #pragma unroll
-            for (int g = 0; g < NG; ++g)
+        for (int j = 0; j < NG / 4; ++j) {
+            f32x4 total{0.f, 0.f, 0.f, 0.f};
+            if (mine) {
+                const float* src = smem + (16 * j + (sub & 12)) * kGateParkStride + 16 * (sub & 3) + tl;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float sum = smem[(g * 4 + v) * kWave + lane];
+                for (int v = 0; v < 4; ++v) total[v] = src[v * kGateParkStride];
 #pragma unroll
-                    for (int w = 1; w < KW; ++w) sum += smem[w * (NG * 4 * kWave) + (g * 4 + v) * kWave + lane];
-                    const uint32_t e = e0 + 16 * g + 4 * chunk + v;
-                    if (e < E) my_logits[e] = sum;
-                }
+                for (int w = 1; w < KW; ++w)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) total[v] += src[w * kShare + v * kGateParkStride];
+            }
+            sum[pass * (NG / 4) + j] = total;
         }
         __syncthreads();
     }
-
-    if (wave == 0 && live) gate_wide_epilogue<T>(p, tile, smem, lane);
-    __syncthreads();
-}
-
-// Softmax, top-k, outputs and the tile histogram of one 16-token tile whose logits are in memory
-// (p.logits), run by one wavefront; `smem` holds E + 16 k words private to it. A lane reads the
-// logits it (or the wavefront that runs this) stored itself, or ones stored before a grid-wide
-// barrier: device-coherent loads either way.
-template <typename T>
-__device__ __forceinline__ void gate_wide_epilogue(const LayerParams& p, uint32_t tile, float* smem, int lane) {
-    const int col = lane & 15, chunk = lane >> 4;
-    const uint32_t E = p.E, k = p.k;
-    const uint32_t token = tile * kGateTileTokens + col;
-    float* my_logits = p.logits + size_t(token) * E;
-    {
-        // lane (col, chunk) owns experts 16 j + 4 chunk + v of token col, as in the register gate
-        const float kNegInf = -__builtin_inff();
-        const uint32_t groups = (E + 15) / 16;
-        auto logit = [&](uint32_t e) { return load_coherent(my_logits + e); };
-        float m = kNegInf;
-        for (uint32_t j = 0; j < groups; ++j)
-#pragma unroll
-            for (uint32_t v = 0; v < 4; ++v) {
-                const uint32_t e = 16 * j + 4 * chunk + v;
-                if (e < E) m = fmaxf(m, logit(e));
-            }
-        m = fmaxf(m, __shfl_xor(m, 16));
-        m = fmaxf(m, __shfl_xor(m, 32));
-        float d = 0.f;
-        for (uint32_t j = 0; j < groups; ++j)
-#pragma unroll
-            for (uint32_t v = 0; v < 4; ++v) {
-                const uint32_t e = 16 * j + 4 * chunk + v;
-                if (e < E) d += __expf(logit(e) - m);
-            }
-        d += __shfl_xor(d, 16);
-        d += __shfl_xor(d, 32);
-        const float inv_d = 1.0f / d;
-        auto prob = [&](float l) { return __expf(l - m) * inv_d; };
-        T* grow = static_cast<T*>(p.gate_out) + size_t(token) * p.PX;
-        for (uint32_t j = 0; 16 * j < p.PX; ++j)
-#pragma unroll
-            for (uint32_t v = 0; v < 4; ++v) {
-                const uint32_t e = 16 * j + 4 * chunk + v;
-                const float pe = e < E ? prob(logit(e)) : 0.f;
-                if (e < p.PX) grow[e] = float_to_elem<T>(pe);   // padded columns are zero (gate.cuh:590-605)
-                if (p.is_training) {
-                    // column sum over the tile's 16 tokens, a fixed xor tree (gate.cuh:608-635)
-                    float col_sum = pe;
-                    col_sum += __shfl_xor(col_sum, 1);
-                    col_sum += __shfl_xor(col_sum, 2);
-                    col_sum += __shfl_xor(col_sum, 4);
-                    col_sum += __shfl_xor(col_sum, 8);
-                    if (col == 0 && e < E) store_through(p.tile_prob + size_t(tile) * E + e, col_sum);
-                }
-            }
-
-        uint32_t* s_hist = reinterpret_cast<uint32_t*>(smem);   // [E] tokens of the tile routed to e
-        uint32_t* s_sel = s_hist + E;                           // [16][k] the tile's picks
-        for (uint32_t e = lane; e < E; e += kWave) s_hist[e] = 0u;
-        constexpr uint32_t kNone = 0x7fffffffu;
-        float den = 0.f, prev_l = 0.f;
-        uint32_t prev_e = 0;
-        for (uint32_t r = 0; r < k; ++r) {
-            float best = kNegInf;
-            uint32_t bi = kNone;
-            for (uint32_t j = 0; j < groups; ++j)
-#pragma unroll
-                for (uint32_t v = 0; v < 4; ++v) {
-                    const uint32_t e = 16 * j + 4 * chunk + v;
-                    if (e >= E) continue;
-                    const float l = logit(e);
-                    const bool open = r == 0 || l < prev_l || (l == prev_l && e > prev_e);
-                    if (open && (bi == kNone || l > best)) {
-                        best = l;
-                        bi = e;
-                    }
-                }
-#pragma unroll
-            for (int off = 16; off <= 32; off <<= 1) {
-                const float ob = __shfl_xor(best, off);
-                const uint32_t oi = __shfl_xor(bi, off);
-                if (oi != kNone && (bi == kNone || ob > best || (ob == best && oi < bi))) {
-                    best = ob;
-                    bi = oi;
-                }
-            }
-            // all four lanes of the token hold the pick now
-            const float pv = bi != kNone ? prob(best) : 0.f;
-            den += pv;   // mCw, accumulated in selection order (gate.cuh:669)
-            prev_l = best;
-            prev_e = bi;
-            if (chunk == 0) {
-                store_through(p.topk_expert + size_t(token) * k + r, int32_t(bi));
-                store_through(p.topk_prob + size_t(token) * k + r, pv);
-                s_sel[uint32_t(col) * k + r] = bi;
-            }
-        }
-        if (chunk == 0) store_through(p.combine_den + token, den);
-        // in-tile rank of every pick and the tile histogram (gate.cuh:678-696); the LDS operations of
-        // one wavefront complete in order, so the picks written above are visible here
-        uint32_t* super = p.super_count + size_t(p.epoch & 1u) * p.n_super * E + size_t(tile / kSuperTiles) * E;
-        const uint32_t pairs = kGateTileTokens * k;
-        for (uint32_t i = lane; i < pairs; i += kWave) {
-            const uint32_t t = i / k, e = s_sel[i];
-            uint32_t before = 0, total = 0;
-            for (uint32_t o = 0; o < pairs; ++o) {
-                const bool same = s_sel[o] == e;
-                total += same;
-                before += same && o / k < t;
-            }
-            store_through(p.topk_slot + ((size_t(tile) * kGateTileTokens + t) * k + (i % k)), int32_t(before));
-            if (before == 0 && e < E) s_hist[e] = total;   // one writer: the first token that picked e
-        }
-        for (uint32_t e = lane; e < E; e += kWave) {
-            const uint32_t cnt = s_hist[e];
-            store_through(p.tile_count + size_t(tile) * E + e, cnt);
-            if (cnt) atomic_add_agent(super + e, cnt);
-        }
-    }
+    gate_group_finish<T, NL>(p, tile, mine, sum, reinterpret_cast<uint32_t*>(smem) + group * gate_group_words(p.E, p.k, p.is_training != 0), gtid);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -567,24 +435,11 @@ __device__ __forceinline__ void gate_wide_epilogue(const LayerParams& p, uint32_
 // (128 tokens x 256 experts per workgroup, the hidden dimension split into p.gate_splits ranges
 // whose fp32 sums land in p.gate_partial[split][token][PX]), so the gate weights are read once per
 // 128 tokens instead of once per 16 or 32. After a grid-wide barrier the 16-token tiles are
-// reduced - by a group of four wavefronts each up to 256 experts, by one wavefront above: the
+// reduced by a group of four wavefronts each: the
 // ranges are added in ascending order (a fixed order: the logits do not depend on timing or on the
 // launch mode), then softmax, top-k and the tile's histogram as in the other gates.
 // ------------------------------------------------------------------------------------------------
-// The sum over the ranges of the 4 experts e0 .. e0+3 of `token` (e0 a multiple of 4; experts past
-// the padded count read as 0).
-__device__ __forceinline__ f32x4 gate_partial_sum(const LayerParams& p, coherent_rows_t partial, uint32_t token, uint32_t e0) {
-    f32x4 sum{0.f, 0.f, 0.f, 0.f};
-    if (e0 < p.PX) {
-        for (uint32_t s = 0; s < p.gate_splits; ++s) {
-            const uint32_t offset = ((s * p.S + token) * p.PX + e0) * 4u;
-            sum += __builtin_bit_cast(f32x4, load16_coherent(partial, offset));
-        }
-    }
-    return sum;
-}
-
-// Up to 256 experts, a tile worked on by a group of four wavefronts (256 threads): wavefront w of
+// A tile worked on by a group of four wavefronts (256 threads): wavefront w of
 // the group takes tokens 4 w .. 4 w + 3 of the tile, 16 lanes per token, each lane the experts
 // 64 j + 4 (lane % 16) + v (j < NL, NL * 64 >= PX, v < 4). Against one wavefront per tile every per-lane
 // loop over the experts is four times shorter, and the partial sums, logits and gate outputs move
@@ -611,7 +466,7 @@ __device__ __forceinline__ void gate_reduce_group(const LayerParams& p, uint32_t
         const coherent_rows_t partial = coherent_rows(p.gate_partial);
         // range by range, in ascending order; the loads of eight ranges in flight together (two at a time the sixteen ranges of 128 tokens of 7 168
         // values, 256 experts, were eight trips to memory)
-        constexpr uint32_t kRanges = 8;
+        constexpr uint32_t kRanges = NL > 4 ? 4 : 8;   // (at most 128 registers)
         for (uint32_t s0 = 0; s0 < p.gate_splits; s0 += kRanges) {
             u32x4 v[kRanges][NL];
 #pragma unroll
@@ -772,22 +627,6 @@ __device__ __forceinline__ void gate_group_finish(const LayerParams& p, uint32_t
         }
     }
     __syncthreads();   // the next tile clears the histogram
-}
-
-// More than 256 experts: the sums go to p.logits, which the epilogue for many experts reads back.
-// `smem` holds E + 16 k words private to the calling wavefront.
-template <typename T>
-__device__ __forceinline__ void gate_reduce_tile_wide(const LayerParams& p, uint32_t tile, float* smem, int lane) {
-    const int col = lane & 15, chunk = lane >> 4;
-    const uint32_t token = tile * kGateTileTokens + col;
-    const coherent_rows_t partial = coherent_rows(p.gate_partial);
-    for (uint32_t e0 = 4 * chunk; e0 < p.E; e0 += 16) {
-        const f32x4 sum = gate_partial_sum(p, partial, token, e0);
-#pragma unroll
-        for (uint32_t v = 0; v < 4; ++v)
-            if (e0 + v < p.E) p.logits[size_t(token) * p.E + e0 + v] = sum[v];
-    }
-    gate_wide_epilogue<T>(p, tile, smem, lane);
 }
 
 // Slot assignment for one 16-token tile, by a group of `gsize` threads (whole wavefronts). Every thread of the workgroup must call

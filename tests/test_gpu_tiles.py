@@ -179,6 +179,17 @@ def test_gate_of_many_experts_in_32_bits(dt, S, H, E, k):
     np.testing.assert_allclose(g["mean_prob"], ref["mean_prob"], rtol=3e-5, atol=1e-8)
 
 
+@pytest.mark.parametrize("dt,S,H,E,k", [
+    (0, 256, 64, 257, 32),        # a second pass that holds one expert; the most picks
+    (1, 4224, 128, 384, 3),       # several units to a workgroup
+    (0, 128, 1024, 512, 5),
+    (2, 384, 128, 300, 3),        # 16-bit: the sums of the product
+    (3, 128, 1152, 512, 32),
+], ids=lambda v: str(v))
+def test_gate_of_more_than_256_experts(dt, S, H, E, k):
+    test_gate_of_many_experts_in_32_bits(dt, S, H, E, k)
+
+
 @pytest.mark.parametrize("dt,S,E,k", [
     (2, 8320, 65, 2),             # a workgroup's slot tiles by four groups of two wavefronts; queues of eight experts, one of nine
     (2, 4224, 128, 3),            # by two groups of four; every queue full
