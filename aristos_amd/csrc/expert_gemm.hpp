@@ -907,6 +907,114 @@ struct GemmPingPong : Gemm16<E, 256, 256, 2, 4, 64, 2, STREAM_B, true> {
 };
 
 // ------------------------------------------------------------------------------------------------
+// The same turns for tiles of half the size, 128 x 256 or 256 x 128: wavefronts of 64 x 64, so that a slice is one section of 32
+// matrix instructions. Three stages: a slice's loads go out two slices ahead, in the half section that reads, where the stage of
+// the slice before is free of both groups' reads; the wait behind them is for the next slice.
+//
+// What bounds it: its loads, 48 KB a slice. In a loop over the tiles of one expert (2 048 rows, 4 096 x 4 096, random data) a slice takes
+// 1 290 clocks of which the matrix cores need 1 024, against 1 720 in step (Gemm16 with three stages); with the wait of the wavefronts in front
+// moved behind their matrix instructions (a scalar branch) 1 430. As the smaller tile of 256-row layers, us per forward: 2 944 tokens, 6 experts top-4,
+// 448 x 1 088: 89.7 -> 86.0; 2 560, 16 experts top-3, 1 472 x 11 200: 580 -> 571.5; 8 192, 8 experts top-2, 4 096 x 14 336: 2 851 -> 2 837.
+// Where weights stream from HBM and are read once the loads of Gemm16, half a slice earlier, are the better ones (variant 1: 1 280 tokens, 256
+// experts, 2 304 x 576: 280.5 -> 283).
+// ------------------------------------------------------------------------------------------------
+template <typename E, int BM, int BN, int WAVES_M, int WAVES_N>
+struct GemmTurns : Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> {
+    typedef Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> Base;
+    typedef typename Base::Tile Tile;
+    typedef typename Base::Acc Acc;
+    typedef typename Base::vec8 vec8;
+    using Base::kStage; using Base::kABytes; using Base::kRowBytes; using Base::kSteps; using Base::WM; using Base::WN; using Base::TM; using Base::TN;
+    static constexpr int L = Base::kLoadsPerSlice;
+    static_assert(WM == 64 && WN == 64 && Base::kWaves == 8 && kSteps == 2);
+
+    // (`after_first_barrier`, the blocks of rows, the barriers: as in GemmPingPong)
+    template <typename Hook>
+    static __device__ __forceinline__ void mainloop(const Tile& t, Acc& acc, char* smem, Hook&& after_first_barrier) {
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+        const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+        const bool behind = wave >= Base::kWaves / 2;
+        auto barrier = [] { asm volatile("s_barrier" ::: "memory"); };
+        if (t.k_tiles > 1) wait_vmcnt<L>();
+        else wait_vmcnt<0>();
+        barrier();   // slice 0 is in LDS, and every wavefront has left the previous tile's epilogue
+        after_first_barrier();
+        if (behind) barrier();
+
+        const int fr_row = lane & 15, fr_part = lane >> 4;
+        const int rx = wm * WM + fr_row, rw = wn * WN + fr_row;
+        const int base_x = rx * kRowBytes + ((fr_part ^ Base::swizzle(rx)) << 4);
+        const int base_w = kABytes + rw * kRowBytes + ((fr_part ^ Base::swizzle(rw)) << 4);
+        const int rows_here = int(t.m_valid) - wm * WM;
+        const int blocks = rows_here <= 0 ? 0 : (rows_here + 15) / 16;
+        auto body = [&](auto full_tag) {
+            constexpr bool FULL = decltype(full_tag)::value;
+            auto used = [&](int block) { return FULL || block < blocks; };
+#pragma unroll
+            for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                for (int mi = 0; mi < TM; ++mi) acc[ni][mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+            vec8 fx[kSteps][TM], fw[kSteps][TN];
+            auto product = [&](int ni, int i) {
+#pragma unroll
+                for (int ks = 0; ks < kSteps; ++ks) {
+                    acc[ni][i] = Elem16<E>::mfma16(fw[ks][ni], fx[ks][i], acc[ni][i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            auto slice = [&](uint32_t kt, auto later_tag) {
+                constexpr int LATER = decltype(later_tag)::value;
+                const char* st = smem + Base::stage_of(t, kt) * kStage;
+                if (used(0)) {
+#pragma unroll
+                    for (int ks = 0; ks < kSteps; ++ks) {
+#pragma unroll
+                        for (int i = 0; i < TN; ++i) fw[ks][i] = __builtin_bit_cast(vec8, load16(st + (base_w ^ (ks << 6)) + i * 16 * kRowBytes));
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) fx[ks][i] = __builtin_bit_cast(vec8, load16(st + (base_x ^ (ks << 6)) + i * 16 * kRowBytes));
+                    }
+                }
+                if constexpr (LATER >= 2) Base::issue_slice(t, smem, kt + 2);
+                if constexpr (LATER >= 1) wait_vmcnt<(LATER >= 2 ? L : 0)>();
+                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+                __builtin_amdgcn_sched_barrier(0);
+                barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_setprio(1);
+                if constexpr (FULL) {
+#pragma unroll
+                    for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) product(ni, i);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        if (used(i)) {
+#pragma unroll
+                            for (int ni = 0; ni < TN; ++ni) product(ni, i);
+                        }
+                }
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_sched_barrier(0);
+                barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;
+            for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::integral_constant<int, 2>{});
+            if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::integral_constant<int, 1>{});
+            slice(t.k_tiles - 1, std::integral_constant<int, 0>{});
+        };
+        if (blocks >= TM) body(std::true_type{});
+        else body(std::false_type{});
+        if (!behind) barrier();
+    }
+    static __device__ __forceinline__ void finish(const Tile& t, Acc& acc, char* smem) {
+        const TileOut out{t.c_base, t.ldc, t.m_valid, t.n_valid, t.act};
+        epilogue16<E, WM, WN, WAVES_N, false>(out, acc, smem + Base::last_stage(t) * kStage, smem + Base::kBiasOffset + t.bias_slot * Base::kBiasBytes);
+    }
+};
+
+// ------------------------------------------------------------------------------------------------
 // A tile small enough for four wavefronts, worked on by eight: two groups of four each run the main loop
 // of G over one half of K, on LDS of their own, and the halves are added at the end. For layers whose
 // tiles would otherwise leave CUs without one. Four wavefronts of 64 x 64 read half as much LDS per

@@ -125,6 +125,7 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     const uint32_t rows = mean_rows(p);
     p.tile_variant = 0u;
     p.down_small = 0u;
+    p.tall = 0u;
     if (dtype == 0 || dtype == 1) {
         const double split = projections_us(p, TileCost{256, 256, 128.0, 0.0}, rows, num_cus, true);
         const double plain = projections_us(p, TileCost{64, 64, 32.0, 0.0}, rows, num_cus, false);
@@ -140,10 +141,13 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     // (bm x bn tiles, the down-projection on dm x dn tiles)
     RowShare shares[4];
     const int n_shares = row_shares(p, shares);
-    auto projection = [&](uint32_t bm, uint32_t bn, uint32_t N, uint32_t K) {
+    auto row_blocks = [&](uint32_t bm) {   // of an expert, in the mean
         double blocks = 0.0;
         for (int i = 0; i < n_shares; ++i) blocks += shares[i].share * std::ceil(shares[i].rows / bm - 1e-9);
-        const double rounds = p.E * blocks * ceil_div_u32(N, bn) / num_cus;
+        return blocks;
+    };
+    auto projection = [&](uint32_t bm, uint32_t bn, uint32_t N, uint32_t K) {
+        const double rounds = p.E * row_blocks(bm) * ceil_div_u32(N, bn) / num_cus;
         const TileCost t = tile16_cost(bm, bn, rows);
         return double(uint64_t(rounds + 0.999999)) * (K * t.per_k + t.fixed);
     };
@@ -188,6 +192,18 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     consider(4, 0, estimate(128, 128, 128, 128, false));
     consider(4, 1, two_tiles(128, 128, 64, 128, false));
     if (!likely) low();
+    // Variant 4 on tiles of 256 x 128 where experts hold more than 128 rows and whole rounds of what a value of K takes on either
+    // tile (GemmTurns, 1 290 clocks per 64, against GemmKSplit, 1 010) come to less: half as many tiles in whatever runs on them.
+    // Of 39 layers of variant 4, timed on both, the rule takes the tall tile at 20: 7 % faster in the mean, most at 1 408 tokens, 16 experts top-2,
+    // 832 x 1 152 (65.2 -> 52.9 us) and 1 536 tokens, 8 experts top-2, 448 x 3 328 (79.9 -> 67.9); 2 048 tokens, one expert, 1 024 x 4 096,
+    // dense: 60.2 -> 52.6. One loses, 384 tokens, 2 experts top-2, 5 120 x 6 400 (224 -> 236); one that it leaves out would gain 20 %, the others at most 6.
+    if (p.tile_variant == 4u && rows > 128u) {
+        auto rounds_us = [&](uint32_t bm, double per_k) {
+            const double up = std::ceil(p.E * row_blocks(bm) * ceil_div_u32(p.I, 128) / num_cus - 1e-6) * (p.H * per_k + 5.0);
+            return p.down_small ? up : up + std::ceil(p.E * row_blocks(bm) * ceil_div_u32(p.H, 128) / num_cus - 1e-6) * (p.I * per_k + 5.0);
+        };
+        p.tall = rounds_us(256, 0.0115) < rounds_us(128, 0.0085);
+    }
 }
 
 uint32_t gate_splits_for(uint32_t S, uint32_t H, uint32_t E, uint32_t PX, int dtype, int num_cus) {

@@ -21,6 +21,7 @@ struct LayerParams {
     uint32_t n_super;         // ceil(n_gate_tiles / 32)
     uint32_t tile_variant;    // tile of the expert projections (choose_tiles)
     uint32_t down_small;      // 1: the down-projection on the smaller tile of the variant (NarrowCfg)
+    uint32_t tall;            // 1: variant 4 on tiles of 256 rows instead of 128
     uint32_t dense;           // one expert that keeps every token, no gate output: rows are tokens; a kDense value
     // ---- caller buffers, sliced as moe.cuh:92-98
     const void* x;            // [S, H]

@@ -636,6 +636,29 @@ def test_every_pair_of_16_bit_tiles_at_the_edges_of_its_rows(mode, dt, want, S, 
 
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("S,H,I,cf,down,edges", [
+    (5120, 192, 704, 2.0, (256, 128), _ROWS_256[:12]),
+    (5120, 192, 704, 2.0, (256, 128), _ROWS_256[-12:]),
+    (5632, 704, 64, 2.4, (256, 128), _ROWS_256[-12:]),      # half a column tile and one slice of K
+    (5632, 64, 1344, 2.0, (256, 128), _ROWS_256[-12:]),
+    (5120, 192, 4160, 2.0, (64, 128), _ROWS_256[-12:]),     # the down-projection in quarters of a row block
+], ids=lambda v: str(len(v)) + "e" if isinstance(v, list) else str(v))
+def test_tall_tiles_at_the_edges_of_their_rows(mode, dt, S, H, I, cf, down, edges):
+    """256 x 128 tiles, at the edges of the 16 rows of a matrix instruction, the 64 of a wavefront and the tile."""
+    E = 24
+    keys = _keys(S, H, I, E, 1, cf=cf, act=1, dt=dt)
+    t = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
+    assert (t["variant"], t["up"], t["down"]) == (4, (256, 128), down)
+    c = moe_ref.cfg_from_keys(keys)
+    share, rest = divmod(S - sum(edges), E - len(edges))
+    rows = edges + [share + 1] * rest + [share] * (E - len(edges) - rest)
+    assert max(rows) <= c.EC
+    _, v, _, _ = check_against_oracle(c, keys, _one_hot_layer(c, rows, seed=S + H), mode)
+    np.testing.assert_array_equal(v["expert_count"], np.array(rows))
+
+
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("H,I", [(64, 128), (128, 64), (192, 320), (256, 64)])
 def test_large_tiles_of_few_slices(mode, dt, H, I):
     """256 x 256 tiles whose loads end while the first slices are multiplied: one to five slices of K, with experts that

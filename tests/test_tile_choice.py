@@ -33,6 +33,19 @@ def test_measured_choices(layer, want):
     assert (t["variant"], t["down_small"]) == want
 
 
+@pytest.mark.parametrize("layer,up,down", [
+    # us per forward on 256 x 128 and on 128 x 128 tiles (with the down-projection on 64 x 128 ones, if it is, in both)
+    (dict(S=2048, H=1024, I=4096, E=1, k=1), (256, 128), (64, 128)),     # 52.6 : 60.3
+    (dict(S=1664, H=576, I=5120, E=1, k=1), (256, 128), (64, 128)),      # 75.5 : 85.4
+    (dict(S=1408, H=832, I=1152, E=16, k=2), (256, 128), (256, 128)),    # 52.9 : 65.2
+    (dict(S=1024, H=2624, I=6592, E=1, k=1, drop=0), (128, 128), (128, 128)),    # 139 : 120
+    (dict(S=128, H=512, I=9728, E=8, k=8), (128, 128), (64, 128)),       # 158 : 154, experts of one low row block
+], ids=str)
+def test_tall_tiles_where_they_save_rounds(layer, up, down):
+    t = tiles(**layer)
+    assert (t["variant"], t["up"], t["down"]) == (4, up, down)
+
+
 def test_every_layer_gets_tiles_its_type_has():
     rng = random.Random(1)
     for _ in range(2000):
