@@ -75,6 +75,10 @@ __device__ __forceinline__ void direct_load16(const void* src, uint32_t lds) {
     else
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
+// Brings the 128-byte line that every lane names into the L2. (4 bytes of each land in LDS, 256 bytes at `lds`, where nobody reads them.)
+__device__ __forceinline__ void touch_lines(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
+}
 #pragma clang diagnostic pop
 // The LDS address of a pointer into the workgroup's LDS, in a scalar register.
 __device__ __forceinline__ uint32_t lds_address(const char* p) {
@@ -918,7 +922,10 @@ struct GemmPingPong : Gemm16<E, 256, 256, 2, 4, 64, 2, STREAM_B, true> {
 // Where weights stream from HBM and are read once the loads of Gemm16, half a slice earlier, are the better ones (variant 1: 1 280 tokens, 256
 // experts, 2 304 x 576: 280.5 -> 283).
 // ------------------------------------------------------------------------------------------------
-template <typename E, int BM, int BN, int WAVES_M, int WAVES_N>
+// HALVES: the sums of the two halves of K are formed apart and added at the end, as GemmKSplit's are, in whose place such a tile runs (relative
+// error against 64 bits, 2 048 tokens, one expert, 1 024 x 4 096, GELU: K in one run 1.66323e-3 in bf16 and 2.0794e-4 in fp16, in halves 1.66308e-3 and
+// 2.0783e-4, as on 128 x 128 tiles; 50.8 -> 51.8 us per forward).
+template <typename E, int BM, int BN, int WAVES_M, int WAVES_N, bool HALVES>
 struct GemmTurns : Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> {
     typedef Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> Base;
     typedef typename Base::Tile Tile;
@@ -1000,9 +1007,28 @@ struct GemmTurns : Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> {
                 __builtin_amdgcn_sched_barrier(0);
             };
             const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;
-            for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::integral_constant<int, 2>{});
+            uint32_t kt = 0;
+            f32x4 saved[HALVES ? TN : 1][HALVES ? TM : 1];
+            if constexpr (HALVES) {
+                const uint32_t half = t.k_tiles >= 4 ? (t.k_tiles + 1) / 2 : 0u;   // (at most `ahead`; three slices and fewer are one run)
+                for (; kt < half; ++kt) slice(kt, std::integral_constant<int, 2>{});
+#pragma unroll
+                for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                    for (int mi = 0; mi < TM; ++mi) {
+                        saved[ni][mi] = acc[ni][mi];
+                        acc[ni][mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+            for (; kt < ahead; ++kt) slice(kt, std::integral_constant<int, 2>{});
             if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::integral_constant<int, 1>{});
             slice(t.k_tiles - 1, std::integral_constant<int, 0>{});
+            if constexpr (HALVES) {
+#pragma unroll
+                for (int ni = 0; ni < TN; ++ni)
+#pragma unroll
+                    for (int mi = 0; mi < TM; ++mi) acc[ni][mi] = saved[ni][mi] + acc[ni][mi];
+            }
         };
         if (blocks >= TM) body(std::true_type{});
         else body(std::false_type{});
@@ -1064,6 +1090,20 @@ struct GemmKSplit {
         if (g.k_first >= mine) g.k_first = mine ? g.k_first % mine : 0u;
         t.missing = barriers_of(first) - barriers_of(mine);
         G::begin(t.half, g, stage0, bias_slot, smem + group() * G::kSmemBytes);
+    }
+
+    // Brings the weight rows of a tile's first slices, two of either half of K, into the L2: called between the main loop of a tile and its
+    // finish(), for the next one. Its own loads go out behind that and behind the look-up of its rows, and the memory has nothing to do meanwhile
+    // where all CUs are between two tiles at the same time and a weight row is read by nobody else. `scratch`: kTouchBytes of LDS.
+    // Us per forward: 512 tokens, 16 experts top-2, 2 048 x 2 048: 84.4 -> 83.5; 128 tokens, 8 experts, 4 096 x 14 336: 332.4 -> 327.6. Tiles that
+    // share weights lose (256 x 256 ones 2 %, 128-row ones that stream their weights between +2.5 and -1 %), as do 64-row ones of several row blocks.
+    static constexpr int kTouchBytes = kGroups * G::kWaves * 256;
+    static __device__ __forceinline__ void touch(const GemmTileArgs<elem16_t>& args, char* scratch) {
+        static_assert(kThreads == 4 * BN);
+        const uint32_t tid = local_tid(), row = tid % BN, half = (tid / BN) & 1u, n = args.K / kSliceK, first = (n + 1) / 2;
+        const uint32_t mine = half ? n - first : first, slice = mine ? (args.k_first + tid / (2 * BN)) % mine + half * first : 0u;
+        const elem16_t* from = args.b_base + size_t(row < args.n_valid ? row : args.n_valid - 1) * args.ldb + size_t(slice) * kSliceK;
+        touch_lines(from, lds_address(scratch) + 256 * wave_index());
     }
 
     template <typename Hook>

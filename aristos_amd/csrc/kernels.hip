@@ -196,7 +196,7 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     // tile (GemmTurns, 1 290 clocks per 64, against GemmKSplit, 1 010) come to less: half as many tiles in whatever runs on them.
     // Of 39 layers of variant 4, timed on both, the rule takes the tall tile at 20: 7 % faster in the mean, most at 1 408 tokens, 16 experts top-2,
     // 832 x 1 152 (65.2 -> 52.9 us) and 1 536 tokens, 8 experts top-2, 448 x 3 328 (79.9 -> 67.9); 2 048 tokens, one expert, 1 024 x 4 096,
-    // dense: 60.2 -> 52.6. One loses, 384 tokens, 2 experts top-2, 5 120 x 6 400 (224 -> 236); one that it leaves out would gain 20 %, the others at most 6.
+    // dense: 60.3 -> 51.8. One loses, 384 tokens, 2 experts top-2, 5 120 x 6 400 (224 -> 236); one that it leaves out would gain 20 %, the others at most 6.
     if (p.tile_variant == 4u && rows > 128u) {
         auto rounds_us = [&](uint32_t bm, double per_k) {
             const double up = std::ceil(p.E * row_blocks(bm) * ceil_div_u32(p.I, 128) / num_cus - 1e-6) * (p.H * per_k + 5.0);
