@@ -144,15 +144,14 @@ __device__ __forceinline__ void gate_accumulate(const T* (&xrow)[TB], const T* w
     }
 }
 
-// One gate unit: gate_unit_blocks<NG>() consecutive 16-token tiles, computed by KW wavefronts of the
+// One gate unit: TB consecutive 16-token tiles (gate_unit_blocks<NG>(), or one where the tiles are fewer than workgroups), computed by KW wavefronts of the
 // workgroup (all of them, or one of several such groups, each with a unit and LDS of its own), which
 // split the hidden dimension. Wavefront b then reduces the partial sums of block
 // b in a fixed order and runs its epilogue. Every thread of the workgroup must call the function
 // (it contains workgroup barriers); `smem` holds gate_smem_floats<NG>(KW) floats and may be reused
 // after the call.
-template <typename T, int NG, int KW>
+template <typename T, int NG, int KW, int TB = gate_unit_blocks<NG>()>
 __device__ __forceinline__ void gate_unit(const LayerParams& p, uint32_t unit, float* smem) {
-    constexpr int TB = gate_unit_blocks<NG>();
     static_assert(TB <= KW);
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)) % KW, lane = threadIdx.x & 63;
     const int col = lane & 15;       // token inside a block / expert row inside a group
@@ -188,7 +187,7 @@ __device__ __forceinline__ void gate_unit(const LayerParams& p, uint32_t unit, f
         // belongs to group b of four wavefronts (one group: block after block), 16 lanes per token
         // and four experts per lane, which add the shares in ascending order (a fixed order: the
         // logits depend neither on timing nor on which wavefront worked on which share).
-        static_assert(TB == 2);
+        static_assert(TB <= 2);
         constexpr int kShare = NG * 4 * kGateParkStride;
 #pragma unroll
         for (int b = 0; b < TB; ++b) {

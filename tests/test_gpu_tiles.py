@@ -145,6 +145,17 @@ def test_gate_tiles_spread_over_workgroups_keep_their_bits(dt, S, H, I, E):
     np.testing.assert_array_equal(out0, out1)
 
 
+@pytest.mark.parametrize("dt,S,H,I,E", [
+    (2, 2176, 1024, 64, 16),      # 136 tiles, workgroups without one
+    (3, 4096, 64, 64, 33),        # a tile for every workgroup; shares of no step and of one
+    (2, 4096, 2112, 64, 64),
+    (2, 4224, 192, 64, 8),        # one tile more than workgroups have groups of wavefronts for: units of two
+], ids=lambda v: str(v))
+def test_gate_tiles_one_to_a_workgroup(dt, S, H, I, E):
+    """As many tiles as workgroups or a little fewer, against the units of two tiles of the phased mode, bit for bit."""
+    test_gate_tiles_spread_over_workgroups_keep_their_bits(dt, S, H, I, E)
+
+
 @pytest.mark.parametrize("dt,S,H,E,k", [
     (0, 512, 64, 65, 3),          # whole units in both modes; one expert past the first run of 64
     (1, 384, 64, 128, 128),       # every expert picked by every token
