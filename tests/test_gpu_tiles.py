@@ -606,6 +606,19 @@ def test_scheduler_statistics_count_tiles(dt, S, H, I, E, k, schedule):
     assert st["tiles"] == int((-(-kept // um)).sum()) * -(-I // un) + int((-(-kept // dm)).sum()) * -(-H // dn)
 
 
+@pytest.mark.parametrize("schedule", [ka.SCHEDULE_DYNAMIC, ka.SCHEDULE_STATIC], ids=["dynamic", "static"])
+@pytest.mark.parametrize("dt,S,H,I,E,k", [(2, 2304, 192, 4672, 16, 2), (3, 4608, 320, 2816, 16, 2), (2, 1664, 448, 1088, 40, 3), (0, 1152, 64, 576, 8, 2)], ids=lambda v: str(v))
+def test_every_row_block_is_handed_out_once(dt, S, H, I, E, k, schedule):
+    """Experts of two and more row blocks, which the static schedule takes in another order from round to round: as many tiles
+    as there are, and the outputs of the launch-by-launch mode."""
+    test_scheduler_statistics_count_tiles(dt, S, H, I, E, k, schedule)
+    keys = _keys(S, H, I, E, k, dt=dt)
+    c = moe_ref.cfg_from_keys(keys)
+    iP = pack_inputs(c, *random_layer(c, seed=S + I, w_std=0.05, bias_std=0.1))
+    outs = [check_against_oracle(c, keys, iP, mode)[2] for mode in ((ka.MODE_PHASED, ka.SCHEDULE_AUTO), (ka.MODE_FUSED, schedule))]
+    np.testing.assert_array_equal(outs[0], outs[1])
+
+
 def _assert_tiles(keys, want):
     t = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
     assert (t["variant"], t["down_small"]) == want, f"the layer runs on {t}: another layer is needed for these tiles"
