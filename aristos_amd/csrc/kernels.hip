@@ -112,6 +112,8 @@ TileCost tile16_cost(uint32_t bm, uint32_t bn, uint32_t rows) {
 // every expert at its mean). Where it moves a layer from the
 // 256- and 128-row tiles to the smaller ones: 640 tokens, 8 experts top-2, 704 x 512: 58 -> 37 us per forward; 2 176
 // tokens, 16 experts top-2, 2 048 x 512: 91 -> 75; 2 048 tokens, one expert, 1 024 x 4 096: 148 -> 108.
+// (The figures above are from before the wavefronts of a SIMD took turns in the 256-row tiles. With them, and the tall tiles below, the choice lies 4 % from the
+// best at 155 other layers drawn alike; all constants fitted anew brought 1.9 %, at layers that other rules here are pinned to, and were not taken.)
 // tf32: 256 x 256 tiles on the 16-bit matrix cores, 128 clocks per value of K, one on a CU, against 64 x 64 tiles on the fp32 ones,
 // 32 clocks, two on a CU in turn. The large tile takes what it is charged (607 us per forward at 8 192 tokens, 64 experts top-2, 2 048 x
 // 2 048, four rounds: 133 clocks; 272 at 2 048 tokens, 8 experts, one round each way: 123), bound by its loads; the 32 are the small one's
