@@ -1185,6 +1185,10 @@ struct GemmKSplit {
 // workgroup on a CU): 1 024 tokens, 8 experts top-2, 1 024 x 4 096, fp32: 567 -> 347 us per forward, the
 // matrix cores busy 65 % of the whole launch at 2.3 GHz; 8 192 tokens, 64 experts top-2, 2 048 x 2 048, tf32:
 // 4 177 -> 2 729 us; 128 tokens, 8 experts, 256 x 512: 57 -> 44 us.
+// With barrier and first reads of a slice inside the last group of the slice before, and its first loads there too, against all of them in
+// front of it: that fp32 layer 342.6 -> 333.4; 9 984 tokens, 16 experts top-1, 704 x 7 808, fp32: 2 195 -> 2 115; 1 920, 128 experts top-3, 1 472 x
+// 640, tf32: 478 -> 457; 16 layers between 0 and 10 % faster. (Loads a group later: 340, and 415 us where 256 tokens, one expert, 832 x 11 200, tf32
+// take 380: a CU that has one workgroup waits for its loads, 412 before.)
 // T: float, or tf32_t - then the operands lose their lower 13 mantissa bits on the way into the matrix
 // cores and the results are rounded to tf32 Elements.
 // ------------------------------------------------------------------------------------------------
@@ -1313,23 +1317,34 @@ struct Gemm32 {
         f32x4 fw[2][TN], fx[2][TM];
         auto read = [&](const char* st, int g) {
 #pragma unroll
-            for (int ni = 0; ni < TN; ++ni) fw[g & 1][ni] = operand(load16(st + (base_w ^ (g << 5)) + ni * 32 * kRowBytes));
+            for (int ni = 0; ni < TN; ++ni) fw[g & 1][ni] = __builtin_bit_cast(f32x4, load16(st + (base_w ^ (g << 5)) + ni * 32 * kRowBytes));
 #pragma unroll
-            for (int mi = 0; mi < TM; ++mi) fx[g & 1][mi] = operand(load16(st + (base_x ^ (g << 5)) + mi * 32 * kRowBytes));
+            for (int mi = 0; mi < TM; ++mi) fx[g & 1][mi] = __builtin_bit_cast(f32x4, load16(st + (base_x ^ (g << 5)) + mi * 32 * kRowBytes));
         };
-        // A slice: behind the first instruction of every group a share of the loads of slice kt+STAGES-1, behind
-        // them the reads of the next group's fragments, all pinned. (Left alone the compiler reads a group where
-        // it is used and waits for it there; and a slice's loads in one run hold up the instructions behind them.)
-        auto slice = [&](uint32_t kt, auto loads_tag) {
-            constexpr bool LOADS = decltype(loads_tag)::value;
-            wait_slice(t.k_tiles - 1 - kt);
-            if (kt == 0) after_first_barrier();
-            const char* st = smem + stage_of(t, kt) * kStage;
-            read(st, 0);
-            const uint32_t sa = lds_address(smem) + stage_of(t, kt + STAGES - 1) * kStage + 1024 * wave_index();
-            uint32_t src = kt + STAGES - 1 + t.k_first;
+        // share `part` of this wavefront's loads of slice kt
+        constexpr int kShare = (kLoadsPerSlice + kGroups - 1) / kGroups;
+        auto request = [&](uint32_t kt, int part) {
+            const uint32_t to = lds_address(smem) + stage_of(t, kt) * kStage + 1024 * wave_index();
+            uint32_t src = kt + t.k_first;
             src = src >= t.k_tiles ? src - t.k_tiles : src;
             const uint32_t k0 = src * kSliceK;
+#pragma unroll
+            for (int i = part * kShare; i < (part + 1) * kShare && i < kLoadsPerSlice; ++i) {
+                if (i < LA) direct_load16<false>(t.pa[i < LA ? i : 0] + k0, to + 1024 * kWaves * i);
+                else direct_load16<false>(t.pb[i < LA ? 0 : i - LA] + k0, to + kABytes + 1024 * kWaves * (i - LA));
+            }
+        };
+        // A slice: behind the first instruction of every group a share of the loads of a later slice, behind
+        // them the reads of the next group's fragments, all pinned. (Left alone the compiler reads a group where
+        // it is used and waits for it there; and a slice's loads in one run hold up the instructions behind them.)
+        // The last group does so for the next slice: its barrier lies behind that group's first instruction, which has waited for
+        // this slice's last reads, so that the stage is free from there on and takes the first share of slice kt+STAGES. (In front of a
+        // slice, barrier and first reads lay open.) LOADS: 2 this slice requests the rest of slice kt+STAGES-1 and the first share of the one behind it,
+        // 1 there is none behind it, 0 neither. NEXT: there is a slice kt+1.
+        auto slice = [&](uint32_t kt, auto loads_tag, auto next_tag) {
+            constexpr int LOADS = decltype(loads_tag)::value;
+            constexpr bool NEXT = decltype(next_tag)::value;
+            const char* st = smem + stage_of(t, kt) * kStage;
 #pragma unroll
             for (int g = 0; g < kGroups; ++g) {
 #pragma unroll
@@ -1338,28 +1353,43 @@ struct Gemm32 {
                     for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
                         for (int mi = 0; mi < TM; ++mi)
-                            acc[ni][mi] = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[g & 1][ni][j], fx[g & 1][mi][j], acc[ni][mi], 0, 0, 0);
+                            acc[ni][mi] = __builtin_amdgcn_mfma_f32_32x32x2f32(operand(fw[g & 1][ni][j]), operand(fx[g & 1][mi][j]), acc[ni][mi], 0, 0, 0);
                     if (j == 0) {
                         __builtin_amdgcn_sched_barrier(0);
-                        if (g + 1 < kGroups) read(st, g + 1);
-                        if constexpr (LOADS) {
-                            constexpr int kPerGroup = (kLoadsPerSlice + kGroups - 1) / kGroups;
-#pragma unroll
-                            for (int i = g * kPerGroup; i < (g + 1) * kPerGroup && i < kLoadsPerSlice; ++i) {
-                                if (i < LA) direct_load16<false>(t.pa[i < LA ? i : 0] + k0, sa + 1024 * kWaves * i);
-                                else direct_load16<false>(t.pb[i < LA ? 0 : i - LA] + k0, sa + kABytes + 1024 * kWaves * (i - LA));
-                            }
+                        if (g + 1 < kGroups) {
+                            read(st, g + 1);
+                            if constexpr (LOADS > 0) request(kt + STAGES - 1, g + 1);
+                        } else if constexpr (NEXT) {
+                            wait_slice(t.k_tiles - 2 - kt);
+                            read(smem + stage_of(t, kt + 1) * kStage, 0);
+                            if constexpr (LOADS > 1) request(kt + STAGES, 0);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
             }
         };
-        const uint32_t ahead = t.k_tiles >= uint32_t(STAGES - 1) ? t.k_tiles - (STAGES - 1) : 0u;   // slices that request a later one
-        for (uint32_t kt = 0; kt < ahead; ++kt) slice(kt, std::true_type{});
-        for (uint32_t kt = ahead; kt < t.k_tiles; ++kt) slice(kt, std::false_type{});
+        static_assert(kGroups % 2 == 0 && STAGES > 2);
+        using Zero = std::integral_constant<int, 0>;
+        wait_slice(t.k_tiles - 1);
+        after_first_barrier();
+        read(smem + stage_of(t, 0) * kStage, 0);
+        const uint32_t ahead = t.k_tiles >= uint32_t(STAGES) ? t.k_tiles - STAGES : 0u;   // slices with LOADS 2
+        uint32_t kt = 0;
+        if (t.k_tiles >= uint32_t(STAGES)) {
+            request(STAGES - 1, 0);
+            for (; kt < ahead; ++kt) slice(kt, std::integral_constant<int, 2>{}, std::true_type{});
+            slice(kt++, std::integral_constant<int, 1>{}, std::true_type{});
+        }
+        for (; kt + 1 < t.k_tiles; ++kt) slice(kt, Zero{}, std::true_type{});
+        slice(kt, Zero{}, std::false_type{});
     }
 
+    // (one value where an instruction takes it: a whole fragment where it is read would wait for the read there)
+    static __device__ __forceinline__ float operand(float v) {
+        if constexpr (kTf32) v = __uint_as_float(__float_as_uint(v) & 0xffffe000u);
+        return v;
+    }
     static __device__ __forceinline__ f32x4 operand(u32x4 v) {
         if constexpr (kTf32) v &= u32x4{0xffffe000u, 0xffffe000u, 0xffffe000u, 0xffffe000u};
         return __builtin_bit_cast(f32x4, v);
