@@ -444,9 +444,7 @@ __device__ __forceinline__ void gate_unit_wide(const LayerParams& p, uint32_t un
 // loop over the experts is four times shorter, and the partial sums, logits and gate outputs move
 // in runs of 256 and 128 bytes per token. The tile's picks meet in LDS: every pick counts the picks
 // of its expert by earlier tokens for its in-tile rank and adds itself to the tile's histogram,
-// which the group then writes out. Same sums over the
-// ranges, same selection rule and same order of the denominator as the gate of more than 256 experts; the softmax
-// denominator is summed in a different (fixed) order.
+// which the group then writes out.
 // `gsm`: gate_group_words(p) words of LDS private to the group. Every thread of the workgroup must
 // call the function the same number of times (it contains workgroup barriers); a group without a
 // tile passes valid = false.
@@ -544,12 +542,15 @@ __device__ __forceinline__ void gate_group_finish(const LayerParams& p, uint32_t
             if (uint32_t(64 * j) < p.PX) *reinterpret_cast<Quad*>(grow + 64 * j + 4 * sub) = raw;
         }
         // top-k: k rounds of arg-max, equal values go to the lower expert index (gate.cuh:654-670);
-        // a picked expert leaves the working copy
+        // a picked expert leaves the working copy. There -inf stands for what cannot be picked, an expert that was or none at all:
+        // a logit of -inf or NaN counts as the lowest finite value, so that a token that holds such logits picks k distinct experts too.
         f32x4 w[NL];
 #pragma unroll
-        for (int j = 0; j < NL; ++j) w[j] = acc[j];
+        for (int j = 0; j < NL; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) w[j][v] = uint32_t(64 * j + 4 * sub + v) < E ? fmaxf(acc[j][v], -__FLT_MAX__) : kNegInf;
         float den = 0.f;
-        constexpr uint32_t kNone = 0x7fffffffu;
+        constexpr uint32_t kNone = 0x7fffffffu;   // of a lane whose experts are taken
         for (uint32_t r = 0; r < k; ++r) {
             float best = kNegInf;
             uint32_t bi = kNone;
@@ -572,8 +573,8 @@ __device__ __forceinline__ void gate_group_finish(const LayerParams& p, uint32_t
             { const float ob = row16_peer<1>(best); const uint32_t oi = row16_peer<1>(bi); better(ob, oi); }
             { const float ob = row16_peer<2>(best); const uint32_t oi = row16_peer<2>(bi); better(ob, oi); }
             { const float ob = row16_peer<3>(best); const uint32_t oi = row16_peer<3>(bi); better(ob, oi); }
-            // every lane of the token knows the winner and its logit
-            const float pv = bi != kNone ? prob(best) : 0.f;
+            // every lane of the token knows the winner and its logit (some expert is left: k <= E)
+            const float pv = prob(best);
             den += pv;   // mCw, accumulated in selection order (gate.cuh:669)
 #pragma unroll
             for (int j = 0; j < NL; ++j)
@@ -709,10 +710,11 @@ __device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, b
         auto assign = [&](uint32_t i, uint32_t e, int32_t rank) {
             const size_t idx = size_t(tile) * pairs + i;
             const uint32_t token = tile * kGateTileTokens + i / p.k;
-            if (e >= E) e = E - 1;   // cannot happen; keeps every address below inside its table
+            const bool real = e < E;   // (always: the rounds of the gate pick experts; anything else would have no place)
+            e = real ? e : 0u;
             uint32_t slot = uint32_t(rank);
             for (uint32_t r = 0; r < runs; ++r) slot += part[r * E + e];
-            const bool keep = slot < p.EC && slot < p.cap_rows;
+            const bool keep = real && slot < p.EC && slot < p.cap_rows;
             store_through(p.topk_slot + idx, keep ? int32_t(slot) : -1);
             if (keep) store_through(p.slot_token + size_t(e) * p.cap_rows + slot, int32_t(token));
         };

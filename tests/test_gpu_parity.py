@@ -148,6 +148,48 @@ def test_tiny_fp32_config(mode):
     assert rel_fro(moe_out, g["moe_out"]) < 1e-5
 
 
+# ------------------------------------------------------------------ logits that are not finite
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("E", [8, 64, 256, 300])
+@pytest.mark.parametrize("dt", [0, 1, 2, 3], ids=["fp32", "tf32", "bf16", "fp16"])
+def test_tokens_beside_one_without_finite_logits(dt, E, k):
+    """One token of NaN, and one whose logits are -inf but for one expert (not in fp16, whose products cannot get there): both pick
+    k distinct experts, the lowest first among those that count alike, as the oracle does, and every other token is what it is
+    without them, bit for bit."""
+    S, H, I, nan_at, inf_at = 256, 64, 64, 5, 197
+    keys = _keys(S, H, I, E, k, drop=0, dt=dt)
+    c = moe_ref.cfg_from_keys(keys)
+    x, wg, *rest = random_layer(c, seed=3 + E + k, w_std=0.1, bias_std=0.1)
+    x[:, H - 1] = 0.0
+    wg[:, H - 1] = -16.0
+    wg[E // 2, H - 1] = 0.0
+    plain = pack_inputs(c, x, wg, *rest)
+    x[nan_at] = np.nan
+    x[inf_at, H - 1] = 0.0 if dt == 3 else 2.0 ** 126
+    iP = pack_inputs(c, x, wg, *rest)
+    others = np.ones(S, bool)
+    others[[nan_at, inf_at]] = False
+    for mode in MODES:
+        _, oP, v = run_gpu(keys, _to_device(c, iP), mode, launches=2)
+        _, oP0, v0 = run_gpu(keys, _to_device(c, plain), mode)
+        assert np.isnan(v["logits"][nan_at]).all()
+        if dt != 3:
+            assert np.flatnonzero(np.isfinite(v["logits"][inf_at])).tolist() == [E // 2]
+            assert (np.delete(v["logits"][inf_at], E // 2) == -np.inf).all()
+        ref = moe_ref.forward(c, iP, logits=v["logits"], token_mask=np.zeros(S, np.uint8))
+        for name in ("topk_expert", "topk_slot", "expert_count"):
+            np.testing.assert_array_equal(v[name], ref[name])
+        assert v["topk_expert"][nan_at].tolist() == list(range(k))
+        for e in range(E):
+            n = int(v["expert_count"][e])
+            np.testing.assert_array_equal(v["slot_token"][e, :n], ref["slot_token"][e, :n])
+        for name in ("topk_expert", "topk_prob", "combine_den"):
+            np.testing.assert_array_equal(v[name][others], v0[name][others])
+        out, out0 = (_out_to_np(c, o) for o in (oP, oP0))
+        np.testing.assert_array_equal(out[:S * c.PX].reshape(S, c.PX)[others], out0[:S * c.PX].reshape(S, c.PX)[others])
+        np.testing.assert_array_equal(out[S * c.PX:].reshape(S, H)[others], out0[S * c.PX:].reshape(S, H)[others])
+
+
 # ------------------------------------------------------------------ shapes and edge cases
 CASES = [
     # S, H, I, E, k, cf, drop, act, dt, bias_std
