@@ -542,13 +542,13 @@ __device__ __forceinline__ void gate_group_finish(const LayerParams& p, uint32_t
             if (uint32_t(64 * j) < p.PX) *reinterpret_cast<Quad*>(grow + 64 * j + 4 * sub) = raw;
         }
         // top-k: k rounds of arg-max, equal values go to the lower expert index (gate.cuh:654-670);
-        // a picked expert leaves the working copy. There -inf stands for what cannot be picked, an expert that was or none at all:
-        // a logit of -inf or NaN counts as the lowest finite value, so that a token that holds such logits picks k distinct experts too.
+        // a picked expert becomes -inf in the working copy. A logit of -inf or NaN counts as the lowest finite value there, so that a
+        // token that holds such logits picks k distinct experts too; so does what lies past the last expert, behind all of them by its index.
         f32x4 w[NL];
 #pragma unroll
         for (int j = 0; j < NL; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) w[j][v] = uint32_t(64 * j + 4 * sub + v) < E ? fmaxf(acc[j][v], -__FLT_MAX__) : kNegInf;
+            for (int v = 0; v < 4; ++v) w[j][v] = fmaxf(acc[j][v], -__FLT_MAX__);
         float den = 0.f;
         constexpr uint32_t kNone = 0x7fffffffu;   // of a lane whose experts are taken
         for (uint32_t r = 0; r < k; ++r) {
