@@ -1337,7 +1337,7 @@ struct Gemm32 {
         // A slice: behind the first instruction of every group a share of the loads of a later slice, behind
         // them the reads of the next group's fragments, all pinned. (Left alone the compiler reads a group where
         // it is used and waits for it there; and a slice's loads in one run hold up the instructions behind them.)
-        // The last group does so for the next slice: its barrier lies behind that group's first instruction, which has waited for
+        // The last group does so for the next slice: its barrier lies behind that group's first instruction and a wait for
         // this slice's last reads, so that the stage is free from there on and takes the first share of slice kt+STAGES. (In front of a
         // slice, barrier and first reads lay open.) LOADS: 2 this slice requests the rest of slice kt+STAGES-1 and the first share of the one behind it,
         // 1 there is none behind it, 0 neither. NEXT: there is a slice kt+1.
@@ -1360,6 +1360,7 @@ struct Gemm32 {
                             read(st, g + 1);
                             if constexpr (LOADS > 0) request(kt + STAGES - 1, g + 1);
                         } else if constexpr (NEXT) {
+                            __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the whole of this slice's last fragments, of which the instruction above took one value each
                             wait_slice(t.k_tiles - 2 - kt);
                             read(smem + stage_of(t, kt + 1) * kStage, 0);
                             if constexpr (LOADS > 1) request(kt + STAGES, 0);
