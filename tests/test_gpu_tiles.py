@@ -619,6 +619,21 @@ def test_every_row_block_is_handed_out_once(dt, S, H, I, E, k, schedule):
     np.testing.assert_array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("E,counters", [(62, 496), (63, 504)])
+def test_readiness_counters_on_either_side_of_their_lines(mode, E, counters):
+    """Eight row blocks to an expert, as many counters as the scheduler's spare words hold and a few more: every tile is
+    worked on once, launch after launch."""
+    keys = _keys(4096, 64, 192, E, 1, cf=7.5, dt=0)
+    c = moe_ref.cfg_from_keys(keys)
+    assert ka.moe.debug_tiles(keys)["up"] == (64, 64) and E * -(-min(c.EC, c.cap_rows) // 64) == counters
+    edges = [c.EC, 1, 0, 64, 65, 449, 448]
+    share, rest = divmod(4096 - sum(edges), E - len(edges))
+    rows = [share + 1] * rest + [share] * (E - len(edges) - rest) + edges
+    _, v, _, _ = check_against_oracle(c, keys, _one_hot_layer(c, rows, seed=E), mode, launches=3)
+    np.testing.assert_array_equal(v["expert_count"], np.array(rows))
+
+
 def _assert_tiles(keys, want):
     t = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
     assert (t["variant"], t["down_small"]) == want, f"the layer runs on {t}: another layer is needed for these tiles"
