@@ -1009,9 +1009,7 @@ struct GemmTurns : Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> {
             const uint32_t ahead = t.k_tiles >= 2 ? t.k_tiles - 2 : 0u;
             uint32_t kt = 0;
             f32x4 saved[HALVES ? TN : 1][HALVES ? TM : 1];
-            if constexpr (HALVES) {
-                const uint32_t half = t.k_tiles >= 4 ? (t.k_tiles + 1) / 2 : 0u;   // (at most `ahead`; three slices and fewer are one run)
-                for (; kt < half; ++kt) slice(kt, std::integral_constant<int, 2>{});
+            auto halfway = [&] {
 #pragma unroll
                 for (int ni = 0; ni < TN; ++ni)
 #pragma unroll
@@ -1019,9 +1017,17 @@ struct GemmTurns : Gemm16<E, BM, BN, WAVES_M, WAVES_N, 64, 3, false, false> {
                         saved[ni][mi] = acc[ni][mi];
                         acc[ni][mi] = f32x4{0.f, 0.f, 0.f, 0.f};
                     }
+            };
+            if constexpr (HALVES) {
+                const uint32_t half = t.k_tiles >= 4 ? (t.k_tiles + 1) / 2 : 0u;   // (at most `ahead`)
+                for (; kt < half; ++kt) slice(kt, std::integral_constant<int, 2>{});
+                halfway();
             }
             for (; kt < ahead; ++kt) slice(kt, std::integral_constant<int, 2>{});
             if (t.k_tiles >= 2) slice(t.k_tiles - 2, std::integral_constant<int, 1>{});
+            if constexpr (HALVES) {
+                if (t.k_tiles == 2 || t.k_tiles == 3) halfway();   // (what it saved above was zero)
+            }
             slice(t.k_tiles - 1, std::integral_constant<int, 0>{});
             if constexpr (HALVES) {
 #pragma unroll

@@ -10,7 +10,7 @@ import aristos_amd as ka
 from aristos_amd import synth
 from helpers import pack_inputs, random_layer
 from oracle import moe_ref
-from test_gpu_parity import MODE_IDS, MODES, _apply, _keys, _one_hot_layer, _out_to_np, _to_device, check_against_oracle
+from test_gpu_parity import MODE_IDS, MODES, _apply, _keys, _one_hot_layer, _out_to_np, _to_device, check_against_oracle, run_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -694,6 +694,33 @@ def test_tall_tiles_at_the_edges_of_their_rows(mode, dt, S, H, I, cf, down, edge
     assert max(rows) <= c.EC
     _, v, _, _ = check_against_oracle(c, keys, _one_hot_layer(c, rows, seed=S + H), mode)
     np.testing.assert_array_equal(v["expert_count"], np.array(rows))
+
+
+@pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
+@pytest.mark.parametrize("dt", [2, 3], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("projection", ["up", "down"])
+@pytest.mark.parametrize("K", [128, 192, 256])
+def test_tall_tiles_sum_short_k_in_halves(mode, dt, projection, K):
+    """Tall tiles form the sums of the two halves of K apart, as the 128-row tiles in whose place they run, also where K is two
+    or three slices: 2^15 in the first slice, and 2^-9 in both matrix instructions of the last. In one run of fp32 sums each of
+    the small products is lost, half of the last place of 2^15 that they are; in halves their sum arrives. All values are exact."""
+    S, N = 6144, 1216
+    H, I = (K, N) if projection == "up" else (N, K)
+    keys = _keys(S, H, I, 1, 1, act=0, dt=dt)
+    t = ka.moe.debug_tiles(keys, torch.cuda.get_device_properties(0).multi_processor_count)
+    assert (t["variant"], t["up"], t["down"]) == (4, (256, 128), (256, 128))
+    c = moe_ref.cfg_from_keys(keys)
+    factors, w = np.zeros(K, np.float32), np.zeros((N, K), np.float32)
+    factors[0], factors[[K - 64, K - 32]] = 256.0, 2.0 ** -5
+    w[:, 0], w[:, [K - 64, K - 32]] = 128.0, 2.0 ** -4
+    x, w_up, w_down, b_up, b_down = (np.zeros(n, np.float32) for n in ((S, H), (I, H), (H, I), I, H))
+    if projection == "up":
+        x[:], w_up, b_up[:], w_down[:, 5] = factors, w, -2.0 ** 15, 1.0
+    else:
+        b_up, w_down, b_down[:] = factors, w, -2.0 ** 15
+    _, oP, _ = run_gpu(keys, _to_device(c, pack_inputs(c, x, np.zeros((1, H), np.float32), w_up, w_down, b_up, b_down)), mode)
+    out = moe_ref.elems_to_f32(_out_to_np(c, oP), c)[S * c.PX:]
+    np.testing.assert_array_equal(out, np.full(S * H, 2.0 ** -8, np.float32))
 
 
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
