@@ -619,6 +619,38 @@ def test_every_row_block_is_handed_out_once(dt, S, H, I, E, k, schedule):
     np.testing.assert_array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("H,I,blocks,want", [
+    (2368, 1536, [4] * 7 + [5], ka.SCHEDULE_DYNAMIC),   # 2 H + 3 I strided, 2 H + 2 I spread over the grid
+    (1152, 2368, [4] * 7 + [5], ka.SCHEDULE_DYNAMIC),   # 3 H + 2 I : 2 H + 2 I, with an up-projection that sums less than half as long
+    (2368, 256, [4] * 7 + [5], ka.SCHEDULE_STATIC),     # H + 3 I : H + 2 I, a round more that hardly counts
+    (2368, 1536, [4] * 8, ka.SCHEDULE_STATIC),
+], ids=lambda v: str(v))
+def test_schedule_of_lists_that_end_unevenly(H, I, blocks, want):
+    """Layers each of whose projections alone takes no queue longer than the grid (64 x 64 tiles, 64 workgroups to an XCD): what is
+    strided and what is handed out goes by both together, in the values of K that a workgroup sums; outputs are those of the other mode."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    last = 298 if blocks[-1] == 5 else 256
+    rows = [(2048 - last) // 7] * 7 + [last]
+    assert sum(rows) == 2048 and [-(-r // 64) for r in rows] == blocks
+    keys = _keys(2048, H, I, 8, 1, cf=1.25, dt=0)
+    assert ka.moe.debug_tiles(keys)["up"] == ka.moe.debug_tiles(keys)["down"] == (64, 64)
+    c = moe_ref.cfg_from_keys(keys)
+    iP = _to_device(c, _one_hot_layer(c, rows, seed=H))
+    outs = []
+    d = ka.initialize(keys)
+    try:
+        for mode in (ka.MODE_PHASED, ka.MODE_FUSED):
+            ka.moe.set_mode(mode)
+            oP = synth.alloc_outputs(d)
+            ka.moe.forward_host(iP, oP)
+            ka.moe.stream_synchronize()
+            outs.append(_out_to_np(c, oP))
+        assert ka.moe.schedule_taken() == want
+    finally:
+        ka.finalize()
+    np.testing.assert_array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("mode", MODES, ids=MODE_IDS)
 @pytest.mark.parametrize("E,counters", [(62, 496), (63, 504)])
 def test_readiness_counters_on_either_side_of_their_lines(mode, E, counters):
