@@ -195,14 +195,23 @@ void choose_tiles(LayerParams& p, int dtype, int num_cus) {
     consider(4, 1, two_tiles(128, 128, 64, 128, false));
     if (!likely) low();
     // Variant 4 on tiles of 256 x 128 where experts hold more than 128 rows and whole rounds of what a value of K takes on either
-    // tile (GemmTurns, 1 290 clocks per 64, against GemmKSplit, 1 010) come to less: half as many tiles in whatever runs on them.
-    // Of 39 layers of variant 4, timed on both, the rule takes the tall tile at 20: 7 % faster in the mean, most at 1 408 tokens, 16 experts top-2,
-    // 832 x 1 152 (65.2 -> 52.9 us) and 1 536 tokens, 8 experts top-2, 448 x 3 328 (79.9 -> 67.9); 2 048 tokens, one expert, 1 024 x 4 096,
-    // dense: 60.3 -> 51.8. One loses, 384 tokens, 2 experts top-2, 5 120 x 6 400 (224 -> 236); one that it leaves out would gain 20 %, the others at most 6.
+    // tile (GemmTurns, 1 290 clocks per 64, against GemmKSplit, 1 010) come to less: half as many tiles in whatever runs on them. Row blocks of another
+    // height also lie differently on the XCDs, and a layer whose fullest queue takes longer than the grid would is handed out (set_up in the persistent
+    // kernel), which costs some 10 us at these sizes. Us per forward on tall and on 128-row tiles: 2 304 tokens, 4 experts top-4, 384 x 384, strided on tall ones
+    // only 48.3 / 68.5; 3 072 tokens, one expert, 2 240 x 832, strided on 128-row ones only 93.3 / 73.3; 2 048 tokens, one expert, 1 024 x 4 096 70.3 / 76.2.
+    // Of 540 layers of variant 4, timed on both (weights from HBM), the choice lies 1.2 % from the better tile in the mean; without the 10 us 2.4, without tall tiles 5.1,
+    // with nothing but tall ones 2.8. It loses more than 5 % to 128-row tiles at 20 (29 without the 10 us, 27 % at most).
     if (p.tile_variant == 4u && rows > 128u) {
         auto rounds_us = [&](uint32_t bm, double per_k) {
-            const double up = std::ceil(p.E * row_blocks(bm) * ceil_div_u32(p.I, 128) / num_cus - 1e-6) * (p.H * per_k + 5.0);
-            return p.down_small ? up : up + std::ceil(p.E * row_blocks(bm) * ceil_div_u32(p.H, 128) / num_cus - 1e-6) * (p.I * per_k + 5.0);
+            const double blocks = row_blocks(bm), queue = p.E == 1 ? std::ceil(blocks / kXcds - 1e-6) : double(ceil_div_u32(p.E, kXcds)) * blocks;
+            const double small = row_blocks(64), small_queue = p.E == 1 ? queue * (bm / 64) : double(ceil_div_u32(p.E, kXcds)) * small;
+            auto rounds = [&](double tiles) { return std::ceil(tiles / num_cus - 1e-6); };
+            auto fits = [&](double of_queue, double of_all, uint32_t columns) { return rounds(of_queue * kXcds * columns) <= rounds(of_all * columns); };
+            const uint32_t up = ceil_div_u32(p.I, 128), down = ceil_div_u32(p.H, 128);
+            double us = rounds(p.E * blocks * up) * (p.H * per_k + 5.0);
+            if (!p.down_small) us += rounds(p.E * blocks * down) * (p.I * per_k + 5.0);
+            const bool strided = fits(queue, p.E * blocks, up) && (p.down_small ? fits(small_queue, p.E * small, down) : fits(queue, p.E * blocks, down));
+            return strided ? us : us + 10.0;
         };
         p.tall = rounds_us(256, 0.0115) < rounds_us(128, 0.0085);
     }

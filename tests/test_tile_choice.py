@@ -34,11 +34,16 @@ def test_measured_choices(layer, want):
 
 
 @pytest.mark.parametrize("layer,up,down", [
-    # us per forward on 256 x 128 and on 128 x 128 tiles (with the down-projection on 64 x 128 ones, if it is, in both)
-    (dict(S=2048, H=1024, I=4096, E=1, k=1), (256, 128), (64, 128)),     # 52.6 : 60.3
-    (dict(S=1664, H=576, I=5120, E=1, k=1), (256, 128), (64, 128)),      # 75.5 : 85.4
-    (dict(S=1408, H=832, I=1152, E=16, k=2), (256, 128), (256, 128)),    # 52.9 : 65.2
-    (dict(S=1024, H=2624, I=6592, E=1, k=1, drop=0), (128, 128), (128, 128)),    # 139 : 120
+    # us per forward on 256 x 128 and on 128 x 128 tiles (with the down-projection on 64 x 128 ones, if it is, in both), weights from HBM
+    (dict(S=2048, H=1024, I=4096, E=1, k=1), (256, 128), (64, 128)),     # 70.3 : 76.2
+    (dict(S=1664, H=576, I=5120, E=1, k=1), (256, 128), (64, 128)),      # 70.5 : 73.6
+    (dict(S=1408, H=832, I=1152, E=16, k=2), (256, 128), (256, 128)),    # 55.6 : 59.0
+    (dict(S=1024, H=2624, I=6592, E=1, k=1, drop=0), (128, 128), (128, 128)),    # 162 : 147
+    # strided through on one of the two only, handed out on the other
+    (dict(S=2304, H=384, I=384, E=4, k=4), (256, 128), (256, 128)),      # 48.3 : 68.5
+    (dict(S=1152, H=640, I=2752, E=1, k=1, cf=1.25), (256, 128), (64, 128)),     # 49.7 : 64.3
+    (dict(S=3072, H=2240, I=832, E=1, k=1, cf=1.25), (128, 128), (128, 128)),    # 93.3 : 73.3
+    (dict(S=1024, H=576, I=7552, E=1, k=1, cf=2.0), (128, 128), (64, 128)),      # 91.6 : 76.5
     (dict(S=128, H=512, I=9728, E=8, k=8), (128, 128), (64, 128)),       # 158 : 154, experts of one low row block
 ], ids=str)
 def test_tall_tiles_where_they_save_rounds(layer, up, down):
