@@ -636,7 +636,7 @@ __device__ __forceinline__ void gate_group_finish(const LayerParams& p, uint32_t
 //   slot = (tokens routed to e in all earlier tiles) + (rank inside this tile); a token keeps its
 //   expert iff slot < EC (gate.cuh:710-716).
 // What bounds it: trips to memory that other XCDs wrote, well over a microsecond each. The rows of counts before a tile (31 of its
-// block and the coarse ones) are shared out over up to eight threads per expert (SHARED), so that they are one trip or two; by a single wavefront, 64
+// block and the coarse ones) are shared out over the threads that a workgroup of 512 has per expert (SHARED: four up to 128 experts, two up to 256), so that they are one trip or two; by a single wavefront, 64
 // experts after the other, they were eight with 256 experts. Up to 64 experts a single wavefront's two trips are the shorter way (the
 // shares cost a sum per pair and more code, all of it executed once: 8 192 tokens, 64 experts: 8.3 us for the phase, 8.9 shared out).
 // The phase with its barrier, with 256 experts: 128 tokens top-8 29 -> 8 us, 4 096 38 -> 12. Us per forward: 2 048 tokens, 128 experts
@@ -661,9 +661,8 @@ __device__ __forceinline__ void slot_tile(const LayerParams& p, uint32_t tile, b
         }
     }
     // expert e's rows of counts: thread e of every run of 2^lg threads, run g taking the rows g, g + runs, ...
-    constexpr uint32_t kRuns = 8;
     const uint32_t lg = SHARED && E > 1 ? 32u - uint32_t(__builtin_clz(E - 1)) : 0u;
-    const uint32_t most = SHARED ? gsize >> lg : 1u, runs = most > kRuns ? kRuns : (most ? most : 1u), g = runs > 1 ? gtid >> lg : 0u;
+    const uint32_t most = SHARED ? gsize >> lg : 1u, runs = most ? most : 1u, g = runs > 1 ? gtid >> lg : 0u;
     if (valid) {
         const uint32_t sup = tile / kSuperTiles;
         const uint32_t first = sup * kSuperTiles;

@@ -7,7 +7,7 @@ namespace kleos_amd {
 
 constexpr int kGateTileTokens = 16;   // tokens per gate tile (one MFMA column block)
 constexpr int kSuperTiles = 32;       // gate tiles per coarse count row (512 tokens)
-constexpr int kMaxGateGroups = 16;    // 16 experts per group: up to 256 experts keep their logits in registers
+constexpr int kMaxGateGroups = 16;    // 16 experts per group: up to 256 experts in one pass over the tokens
 
 // LayerParams::dense: routed as any layer | rows are tokens, results through y and the combine | results stored by the
 // down-projection (persistent kernel only)
