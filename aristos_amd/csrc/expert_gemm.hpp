@@ -1188,8 +1188,8 @@ struct GemmKSplit {
 // path and leaves the path half idle, so the tile is kept small for the sake of the tile counts: two
 // workgroups of four wavefronts on a CU, each in its own phase, cover each other's barriers.
 // Measured against the tile before it (slices of 16 values through registers, one at a time, one
-// workgroup on a CU): 1 024 tokens, 8 experts top-2, 1 024 x 4 096, fp32: 567 -> 347 us per forward, the
-// matrix cores busy 65 % of the whole launch at 2.3 GHz; 8 192 tokens, 64 experts top-2, 2 048 x 2 048, tf32:
+// workgroup on a CU): 1 024 tokens, 8 experts top-2, 1 024 x 4 096, fp32: 567 -> 347 us per forward (316 with all
+// that has changed since, the matrix cores busy 70 % of the whole launch at 2.26 GHz); 8 192 tokens, 64 experts top-2, 2 048 x 2 048, tf32:
 // 4 177 -> 2 729 us; 128 tokens, 8 experts, 256 x 512: 57 -> 44 us.
 // With barrier and first reads of a slice inside the last group of the slice before, and its first loads there too, against all of them in
 // front of it: that fp32 layer 342.6 -> 333.4; 9 984 tokens, 16 experts top-1, 704 x 7 808, fp32: 2 195 -> 2 115; 1 920, 128 experts top-3, 1 472 x
